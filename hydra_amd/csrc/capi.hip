@@ -93,8 +93,8 @@ static void free_ctx(Ctx *c) {
                   c->qdiss_map, c->qdiss_exp, c->qs, c->qd, c->qc, c->qq, c->pp, c->uu, c->vv,
                   c->qr, c->emq, c->epq, c->qsi, c->qsf, c->sqs, c->qdi, c->qdf, c->sqd, c->wa,
                   c->wb, c->wc, c->wd, c->cnt, c->fq, c->mq, c->qjx_cnt, c->qbot,
-                  c->flags, c->replay, c->replay_val, c->rp_tkey,
-                  c->rp_tid, c->rp_list, c->xq, c->yq, c->xqi, c->yqi, c->xqf, c->yqf, c->uq,
+                  c->flags, c->replay, c->replay_val, c->rp_cell,
+                  c->rp_list, c->xq, c->yq, c->xqi, c->yqi, c->xqf, c->yqf, c->uq,
                   c->vq, c->nextq, c->nxt_tmp, c->dsc, c->dsum, c->seq_work, c->uu32,
                   c->vv32, c->fa32, c->fb32, c->fc32, c->tmp32, c->fq32, c->mq32, c->xtrig32,
                   c->ytrig32, c->qb32, c->qdiss_u_dev, c->part, c->c2g_q, c->c2g_w, c->c2g_q32,
@@ -212,14 +212,11 @@ static int create(const hyd_params *p, hyd_ctx **out) {
   TRY(dalloc(&c->flags, 16));
   c->replay_cap = 1 << 22;
   c->rp_bcap = 1 << 20;
-  c->rp_tsize = 1 << 21;
   TRY(dalloc(&c->replay, c->replay_cap));
   TRY(dalloc(&c->replay_val, c->rp_bcap));
   TRY(dalloc(&c->rp_list, 4 * c->rp_bcap));
-  TRY(dalloc(&c->rp_tid, c->rp_tsize));
-  TRY(dalloc(&c->rp_tkey, c->rp_tsize));
-  if (hipMemset(c->rp_tkey, 0xff, sizeof(int32_t) * c->rp_tsize) != hipSuccess ||
-      hipMemset(c->flags, 0, sizeof(int32_t) * 16) != hipSuccess) {
+  TRY(dalloc(&c->rp_cell, c->rp_bcap));
+  if (hipMemset(c->flags, 0, sizeof(int32_t) * 16) != hipSuccess) {
     set_error("hipMemset failed");
     free_ctx(c);
     return HYD_EHIP;

@@ -31,19 +31,23 @@
 namespace hyd {
 
 // Order-dependent cells ("flagged": both signs, at least three of one) are
-// re-summed in node order from per-cell buckets: an open-addressing table
-// maps the cell key to a bucket; a claim pass gives every flagged cell a
-// bucket of exactly p+q slots, a fill pass drops each crossing's (node, sign)
-// into its cell's bucket, and one thread per bucket orders its few entries by
-// node and adds them as the reference does.  Nothing is sorted globally and
-// the table is left empty again at the end of the sweep.
+// re-summed in node order from per-cell buckets.  The node pass appends a
+// cell to a list when its counts first become order-dependent (its list
+// position is its bucket); a claim pass over the list gives every bucket
+// exactly p+q entries and replaces the cell's counter by the bucket number
+// (mark_bucket), so that whoever meets the cell later needs no search; a
+// fill pass over the nodes drops each crossing's (node, sign) into its
+// cell's bucket, and one thread per bucket, over the whole GPU, orders the
+// entries by node and adds them as the reference does.
+// A developed flow has 10^4 to 10^5 such cells.  300 steps into an ng=256
+// flow (4e5 nodes) the sweep's claim takes 5 us (205 us when it revisited
+// the nodes, with a hash table and two same-address atomics per cell) and
+// the sums 65 us (1754 us in one workgroup).
 struct Buckets {
-  int32_t *tkey;    // table keys, -1 = empty
-  int32_t *tid;     // bucket of each table slot
-  int32_t *list;    // per bucket: table slot, first entry, size, fill count
+  int32_t *cell;    // list: the counter's index, or nfine + column (bottom row)
+  int32_t *list;    // per bucket: first entry, size, fill count, unused
   int32_t *slots;   // entries: node << 1 | (sign > 0)
   double *vals;     // node-order sum of each bucket
-  uint32_t tmask;   // table size - 1 (power of two)
   int32_t bcap;     // buckets
   int64_t scap;     // entries
 };
@@ -58,8 +62,8 @@ struct C2GArgs {
   const double *xgf;
   int32_t *cnt;      // nyf*nxf packed counters
   int32_t *qjx;      // nxf packed counters (bottom row)
-  // [0] flagged cells, [1] flagged qjx, [2] bucket entries used, [4] buckets
-  // used, [5] dropped edge crossings; [8] sticky error (kept across sweeps)
+  // [0] flagged cells, [2] bucket entries used, [5] dropped edge crossings;
+  // [8] sticky error (kept across sweeps)
   int32_t *flags;
   Buckets bk;
 };
@@ -74,26 +78,34 @@ __device__ __forceinline__ bool is_flagged(int32_t w) {
   return p > 0 && q > 0 && (p >= 3 || q >= 3);
 }
 
-__device__ __forceinline__ void add_count(int32_t *slot, int sign, int32_t *flag) {
-  const int32_t d = sign > 0 ? 1 : (1 << 16);
-  const int32_t old = atomicAdd(slot, d);
-  if (!is_flagged(old) && is_flagged(old + d)) atomicAdd(flag, 1);
+// The counter of a claimed cell holds its bucket: 15 bits in each half, the
+// top bit of both set, which makes it a flagged word; every flagged cell is
+// claimed before the marks are read, so no count is mistaken for one.
+static constexpr int32_t kNoBucket = 0x3fffffff;  // the bucket list was full
+__device__ __forceinline__ int32_t mark_bucket(int32_t b) {
+  return (int32_t)(0x80008000u | ((uint32_t)(b >> 15) << 16) | (uint32_t)(b & 0x7fff));
+}
+__device__ __forceinline__ int32_t bucket_of(int32_t w) {
+  return (((w >> 16) & 0x7fff) << 15) | (w & 0x7fff);
 }
 
-__device__ __forceinline__ uint32_t bk_hash(int32_t key, uint32_t mask) {
-  return ((uint32_t)key * 2654435761u) & mask;
+// Cells that became flagged in this workgroup, listed with one global
+// atomic per workgroup (one per cell beyond the list's length).
+static constexpr int kNewFlags = 512;
+struct FlagList {
+  int32_t n, base;
+  int32_t cell[kNewFlags];
+};
+__device__ __forceinline__ void put_bucket_cell(const Buckets &bk, int32_t *flags, int32_t b,
+                                                int32_t cell) {
+  if (b < bk.bcap) bk.cell[b] = cell;
+  else atomicOr(&flags[8], 1);
 }
-
-// table slot holding key, or -1
-__device__ __forceinline__ int64_t bk_find(const Buckets &b, int32_t key) {
-  uint32_t h = bk_hash(key, b.tmask);
-  for (uint32_t probe = 0; probe <= b.tmask; probe++) {
-    const int32_t k = b.tkey[h];
-    if (k == key) return h;
-    if (k == -1) return -1;
-    h = (h + 1) & b.tmask;
-  }
-  return -1;
+__device__ __forceinline__ void new_flag(FlagList &fl, const Buckets &bk, int32_t *flags,
+                                         int32_t cell) {
+  const int32_t k = atomicAdd(&fl.n, 1);
+  if (k < kNewFlags) fl.cell[k] = cell;
+  else put_bucket_cell(bk, flags, atomicAdd(&flags[0], 1), cell);
 }
 
 // The segment from node i to its successor: fine cell of the node,
@@ -125,9 +137,8 @@ __device__ __forceinline__ SegGeom seg_geom(const C2GArgs &a, int i) {
 
 // Node phase: contours.f90:206-231 and the crossing loop 249-269.
 static constexpr int kCrossBatch = 4;
-__global__ void c2g_nodes(C2GArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
+template <bool LIST>
+__device__ __forceinline__ void node_crossings(const C2GArgs &a, int i, FlagList *fl) {
   const SegGeom sg = seg_geom(a, i);
   const double xi = sg.xi, yi = sg.yi, dx = sg.dx, dy = sg.dy, yy = sg.yy;
   const int ixci = sg.ixci, nxc = sg.nxc;
@@ -137,8 +148,14 @@ __global__ void c2g_nodes(C2GArgs a) {
     const int ix = 1 + (int)(a.glxfi * (fmod(a.ellx + a.hlx + xi + p * dx, a.ellx)));
     // ix = nxf+1 can only come from rounding at the domain edge; the
     // reference would index past qjx there, so it is dropped and flagged
-    if (ix >= 1 && ix <= a.nxf) add_count(&a.qjx[ix - 1], cc > 0.0 ? -1 : 1, &a.flags[1]);
-    else atomicAdd(&a.flags[5], 1);
+    if (ix >= 1 && ix <= a.nxf) {
+      const int32_t d = cc > 0.0 ? (1 << 16) : 1;
+      const int32_t old = atomicAdd(&a.qjx[ix - 1], d);
+      if (LIST && !is_flagged(old) && is_flagged(old + d))
+        new_flag(*fl, a.bk, a.flags, (int32_t)((int64_t)a.nxf * a.nyf + ix - 1));
+    } else {
+      atomicAdd(&a.flags[5], 1);
+    }
   }
   if (nxc != 0) {
     const int jump = nxc >= 0 ? 1 : -1;
@@ -179,163 +196,33 @@ __global__ void c2g_nodes(C2GArgs a) {
       for (int b = 0; b < kCrossBatch; b++) old[b] = cell[b] >= 0 ? atomicAdd(&a.cnt[cell[b]], d) : 0;
 #pragma unroll
       for (int b = 0; b < kCrossBatch; b++)
-        if (cell[b] >= 0 && !is_flagged(old[b]) && is_flagged(old[b] + d)) atomicAdd(&a.flags[0], 1);
+        if (LIST && cell[b] >= 0 && !is_flagged(old[b]) && is_flagged(old[b] + d))
+          new_flag(*fl, a.bk, a.flags, (int32_t)cell[b]);
     }
   }
 }
 
-// Claim (PASS 0) and fill (PASS 1) of the buckets of flagged cells; both
-// revisit the crossings of node i exactly as c2g_nodes found them.
-template <int PASS>
-__device__ __forceinline__ void bk_visit(const C2GArgs &a, int32_t key, int32_t w, int node,
-                                         int sgn) {
-  const Buckets &b = a.bk;
-  if (PASS == 0) {
-    uint32_t h = bk_hash(key, b.tmask);
-    for (uint32_t probe = 0;; probe++) {
-      if (probe > b.tmask) {
-        atomicOr(&a.flags[8], 1);
-        return;
-      }
-      const int32_t prev = atomicCAS(&b.tkey[h], -1, key);
-      if (prev == key) return;
-      if (prev == -1) {
-        const int sz = (w & 0xffff) + ((w >> 16) & 0xffff);
-        const int nb = atomicAdd(&a.flags[4], 1);
-        const int base = atomicAdd(&a.flags[2], sz);
-        if (nb >= b.bcap || (int64_t)base + sz > b.scap) {
-          b.tid[h] = -1;
-          atomicOr(&a.flags[8], 1);
-          return;
-        }
-        b.tid[h] = nb;
-        b.list[4 * nb] = (int32_t)h;
-        b.list[4 * nb + 1] = base;
-        b.list[4 * nb + 2] = sz;
-        b.list[4 * nb + 3] = 0;
-        return;
-      }
-      h = (h + 1) & b.tmask;
-    }
-  } else {
-    const int64_t h = bk_find(b, key);
-    const int nb = h >= 0 ? b.tid[h] : -1;
-    if (nb < 0) {
-      atomicOr(&a.flags[8], 1);
-      return;
-    }
-    const int pos = atomicAdd(&b.list[4 * nb + 3], 1);
-    if (pos >= b.list[4 * nb + 2]) {
-      atomicOr(&a.flags[8], 2);
-      return;
-    }
-    b.slots[b.list[4 * nb + 1] + pos] = (node << 1) | (sgn > 0 ? 1 : 0);
+// LIST: list the cells that become order-dependent (the integer sweep of
+// the mixed step has none).
+template <bool LIST>
+__global__ void c2g_nodes(C2GArgs a) {
+  __shared__ FlagList fl;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (LIST) {
+    if (threadIdx.x == 0) fl.n = 0;
+    __syncthreads();
   }
+  if (i < a.n) node_crossings<LIST>(a, i, &fl);
+  if (!LIST) return;
+  __syncthreads();
+  const int n = min(fl.n, kNewFlags);
+  if (n == 0) return;
+  if (threadIdx.x == 0) fl.base = atomicAdd(&a.flags[0], n);
+  __syncthreads();
+  for (int k = threadIdx.x; k < n; k += blockDim.x)
+    put_bucket_cell(a.bk, a.flags, fl.base + k, fl.cell[k]);
 }
 
-template <int PASS>
-__device__ __forceinline__ void bk_node(const C2GArgs &a, int i) {
-  const SegGeom sg = seg_geom(a, i);
-  const double xi = sg.xi, yi = sg.yi, dx = sg.dx, dy = sg.dy, yy = sg.yy;
-  const int nxc = sg.nxc, ixci = sg.ixci;
-  const int64_t nkey = (int64_t)a.nxf * a.nyf;
-  if (a.flags[1] != 0 && fabs(yy) > a.hly) {
-    const double cc = copysign(1.0, dy);
-    const double p = -(yi - a.hly * cc) / (dy + a.small);
-    const int ix = 1 + (int)(a.glxfi * (fmod(a.ellx + a.hlx + xi + p * dx, a.ellx)));
-    if (ix >= 1 && ix <= a.nxf) {
-      const int32_t w = a.qjx[ix - 1];
-      if (is_flagged(w)) bk_visit<PASS>(a, (int32_t)(nkey + ix - 1), w, i, cc > 0.0 ? -1 : 1);
-    }
-  }
-  if (a.flags[0] != 0 && nxc != 0) {
-    const int jump = nxc >= 0 ? 1 : -1;
-    const int ixbeg = a.ultra ? ixci + (1 + jump) / 2 + a.nxf : ixci + (jump - 1) / 2 + a.nxf;
-    const int sgn = a.ultra ? jump : (copysign(1.0, dx) > 0.0 ? 1 : -1);
-    for (int ncr = 0; ncr != nxc; ncr += jump) {
-      const int ix = 1 + (ixbeg + ncr) % a.nxf;
-      const double x2 = a.xgf[ix - 1] - xi;
-      const double px0 = (x2 - a.ellx * (double)(int)(x2 * a.hlxi)) / dx;
-      const double y2 = yi + px0 * dy;
-      const int iy = 2 + (int)(a.glyfi * (y2 - a.elly * (double)(int)(y2 * a.hlyi) - a.ymin));
-      if (iy < 2 || iy > a.nyf) continue;
-      const int64_t cell = (int64_t)(ix - 1) * a.nyf + (iy - 1);
-      const int32_t w = a.cnt[cnt_at(ix - 1, iy - 1, a.nyf)];
-      if (is_flagged(w)) bk_visit<PASS>(a, (int32_t)cell, w, i, sgn);
-    }
-  }
-}
-
-// Grid-stride over the nodes: the launch is small, since it usually finds
-// no flagged cell and returns at once.
-template <int PASS>
-__global__ void c2g_buckets(C2GArgs a) {
-  if (a.flags[0] == 0 && a.flags[1] == 0) return;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x)
-    bk_node<PASS>(a, i);
-}
-
-// Bucket nb: order the entries by node and add them in that order (the
-// reference's node loop).
-__device__ void bucket_sum(const Buckets &b, int nb, double qjump) {
-  const int base = b.list[4 * nb + 1], sz = b.list[4 * nb + 2];
-  int32_t *e = b.slots + base;
-  for (int t = 1; t < sz; t++) {
-    const int32_t v = e[t];
-    int u = t - 1;
-    while (u >= 0 && (e[u] >> 1) > (v >> 1)) {
-      e[u + 1] = e[u];
-      u--;
-    }
-    e[u + 1] = v;
-  }
-  double s = 0.0;
-  for (int t = 0; t < sz; t++) s = s + ((e[t] & 1) ? qjump : -qjump);
-  b.vals[nb] = s;
-}
-
-// Empty the table again (after the sweep has read the bucket sums; the
-// bucket count is the copy c2g_qbot kept in flags[6]) and zero the n4 int4
-// of counters for the next sweep, in whole lines.
-__global__ void c2g_bucket_clear(Buckets b, int32_t *flags, int4 *cnt, int64_t n4) {
-  const int nb_used = min(flags[6], b.bcap);
-  const int stride = gridDim.x * blockDim.x;
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int nb = tid; nb < nb_used; nb += stride) {
-    b.tkey[b.list[4 * nb]] = -1;
-    if (b.list[4 * nb + 3] != b.list[4 * nb + 2]) atomicOr(&flags[8], 2);
-  }
-  for (int64_t k = tid; k < n4; k += stride) cnt[k] = make_int4(0, 0, 0, 0);
-}
-
-// Value of a cell's node-order sum from its counts.
-__device__ __forceinline__ double cell_value(int32_t w, int64_t key, double qjump,
-                                             const Buckets &b) {
-  const int p = w & 0xffff, q = (w >> 16) & 0xffff;
-  if (q == 0) {
-    double s = 0.0;
-    for (int t = 0; t < p; t++) s = s + qjump;
-    return s;
-  }
-  if (p == 0) {
-    double s = 0.0;
-    for (int t = 0; t < q; t++) s = s + (-qjump);
-    return s;
-  }
-  if (p <= 2 && q <= 2) return (double)(p - q) * qjump;
-  const int64_t h = bk_find(b, (int32_t)key);
-  const int nb = h >= 0 ? b.tid[h] : -1;
-  return nb >= 0 ? b.vals[nb] : 0.0 / 0.0;
-}
-
-// cell_value for the common cells first: a single crossing of either sign
-// (0 + qjump and 0 - qjump are exact).
-__device__ __forceinline__ double cell_value_fast(int32_t w, int64_t key, double qjump,
-                                                  const Buckets &b) {
-  if (w == 1) return qjump;
-  if (w == (1 << 16)) return -qjump;
-  return cell_value(w, key, qjump, b);
-}
 
 // Inclusive wavefront scan of ints (row shifts, then row broadcasts).
 template <int CTRL>
@@ -354,6 +241,218 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
   return v;
 }
 
+// Claim: bucket b of the listed cells gets its p+q entries (a workgroup
+// scan and one atomic per 256 buckets) and the cell its mark.
+__global__ void __launch_bounds__(256) c2g_claim(C2GArgs a) {
+  const int total = a.flags[0], nb = min(total, a.bk.bcap);
+  if (nb == 0) return;
+  __shared__ int32_t wsum[4], base;
+  const int64_t nfine = (int64_t)a.nxf * a.nyf;
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int b0 = blockIdx.x * 256; b0 < nb; b0 += gridDim.x * 256) {
+    const int b = b0 + threadIdx.x;
+    int32_t *slot = nullptr;
+    int32_t sz = 0;
+    if (b < nb) {
+      const int32_t cell = a.bk.cell[b];
+      slot = cell >= nfine ? &a.qjx[cell - nfine] : &a.cnt[cell];
+      const int32_t w = *slot;
+      sz = (w & 0xffff) + ((w >> 16) & 0xffff);
+    }
+    const int32_t incl = wave_scan_i32(sz);
+    if (l == 63) wsum[wv] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0) base = atomicAdd(&a.flags[2], wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+    __syncthreads();
+    int64_t first = (int64_t)base + incl - sz;
+    for (int k = 0; k < wv; k++) first += wsum[k];
+    if (slot) {
+      const bool fits = first >= 0 && first + sz <= a.bk.scap;
+      if (!fits) atomicOr(&a.flags[8], 1);
+      a.bk.list[4 * b] = fits ? (int32_t)first : 0;
+      a.bk.list[4 * b + 1] = fits ? sz : 0;
+      a.bk.list[4 * b + 2] = 0;
+      *slot = mark_bucket(fits ? b : kNoBucket);
+    }
+    __syncthreads();
+  }
+}
+
+// Fill: the crossings of node i revisited as c2g_nodes found them.
+__device__ __forceinline__ void bk_put(const C2GArgs &a, int32_t w, int node, int sgn) {
+  const Buckets &b = a.bk;
+  const int32_t nb = bucket_of(w);
+  if (nb >= b.bcap) return;  // no bucket: reported by the claim
+  const int pos = atomicAdd(&b.list[4 * nb + 2], 1);
+  if (pos < b.list[4 * nb + 1]) b.slots[b.list[4 * nb] + pos] = (node << 1) | (sgn > 0 ? 1 : 0);
+}
+
+__device__ __forceinline__ void bk_node(const C2GArgs &a, int i) {
+  const SegGeom sg = seg_geom(a, i);
+  const double xi = sg.xi, yi = sg.yi, dx = sg.dx, dy = sg.dy, yy = sg.yy;
+  const int nxc = sg.nxc, ixci = sg.ixci;
+  if (fabs(yy) > a.hly) {
+    const double cc = copysign(1.0, dy);
+    const double p = -(yi - a.hly * cc) / (dy + a.small);
+    const int ix = 1 + (int)(a.glxfi * (fmod(a.ellx + a.hlx + xi + p * dx, a.ellx)));
+    if (ix >= 1 && ix <= a.nxf) {
+      const int32_t w = a.qjx[ix - 1];
+      if (is_flagged(w)) bk_put(a, w, i, cc > 0.0 ? -1 : 1);
+    }
+  }
+  if (nxc != 0) {
+    const int jump = nxc >= 0 ? 1 : -1;
+    const int ixbeg = a.ultra ? ixci + (1 + jump) / 2 + a.nxf : ixci + (jump - 1) / 2 + a.nxf;
+    const int sgn = a.ultra ? jump : (copysign(1.0, dx) > 0.0 ? 1 : -1);
+    for (int ncr = 0; ncr != nxc; ncr += jump) {
+      const int ix = 1 + (ixbeg + ncr) % a.nxf;
+      const double x2 = a.xgf[ix - 1] - xi;
+      const double px0 = (x2 - a.ellx * (double)(int)(x2 * a.hlxi)) / dx;
+      const double y2 = yi + px0 * dy;
+      const int iy = 2 + (int)(a.glyfi * (y2 - a.elly * (double)(int)(y2 * a.hlyi) - a.ymin));
+      if (iy < 2 || iy > a.nyf) continue;
+      const int32_t w = a.cnt[cnt_at(ix - 1, iy - 1, a.nyf)];
+      if (is_flagged(w)) bk_put(a, w, i, sgn);
+    }
+  }
+}
+
+// Grid-stride over the nodes: the launch is small, since on fresh contours
+// it usually finds no flagged cell and returns at once.
+__global__ void c2g_fill(C2GArgs a) {
+  if (a.flags[0] == 0) return;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x)
+    bk_node(a, i);
+}
+
+// The entries of a bucket of at most M, in registers: a bitonic network
+// orders them by node (the unused ones last), then the reference's sum.
+template <int M>
+__device__ __forceinline__ double bucket_sum_small(const int32_t *e, int sz, double qjump) {
+  int32_t v[M];
+#pragma unroll
+  for (int t = 0; t < M; t++) v[t] = t < sz ? e[t] : INT32_MAX;
+#pragma unroll
+  for (int k = 2; k <= M; k <<= 1)
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1)
+#pragma unroll
+      for (int t = 0; t < M; t++) {
+        const int u = t ^ j;
+        if (u > t) {
+          const int32_t lo = min(v[t], v[u]), hi = max(v[t], v[u]);
+          v[t] = (t & k) ? hi : lo;
+          v[u] = (t & k) ? lo : hi;
+        }
+      }
+  double s = 0.0;
+#pragma unroll
+  for (int t = 0; t < M; t++)
+    if (t < sz) s = s + ((v[t] & 1) ? qjump : -qjump);
+  return s;
+}
+
+// Orders the calling wavefront's LDS and memory accesses.
+__device__ __forceinline__ void c2g_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The sums of up to 64 buckets, one per lane (nb < 0: none): the entries
+// ordered by node and added in that order (the reference's node loop).  A
+// node crosses a cell's column at most once, so the entries' nodes differ.
+// A lane orders up to 32 entries in registers; more are ordered by the
+// whole wavefront, each entry written to its rank (a count of the smaller
+// ones, from LDS), beyond kWaveSort in place by the lane.  All lanes of the
+// wavefront call it.
+// Bound by the reads of the entries and, in crowded cells, by the chain of
+// dependent adds.  An ng=64 flow 200 steps in, with buckets of up to some
+// hundred entries: c2g_qbot 2440 us with a lane of one workgroup sorting
+// each bucket in memory, 431 us with those lanes spread over the GPU, 34 us
+// so; ng=256, 300 steps in: 1754, 346 and 65 us.
+static constexpr int kWaveSort = 512;
+__device__ double bucket_sums(const Buckets &b, int nb, double qjump, int32_t *lds) {
+  const int l = threadIdx.x & 63;
+  const int sz = nb >= 0 ? b.list[4 * nb + 1] : 0;
+  const int first = nb >= 0 ? b.list[4 * nb] : 0;
+  int32_t *e = b.slots + first;
+  uint64_t big = __ballot(sz > 32 && sz <= kWaveSort);
+  while (big) {
+    const int q = __ffsll((unsigned long long)big) - 1;
+    big &= big - 1;
+    const int n = __builtin_amdgcn_readlane(sz, q);
+    int32_t *eq = b.slots + __builtin_amdgcn_readlane(first, q);
+    for (int i = l; i < ((n + 3) & ~3); i += 64) lds[i] = i < n ? eq[i] : INT32_MAX;
+    c2g_wave_sync();
+    for (int i = l; i < n; i += 64) {
+      const int32_t v = lds[i];
+      int rank = 0;
+      for (int j = 0; j < n; j += 4) {
+        const int4 o = *(const int4 *)&lds[j];
+        rank += (o.x < v) + (o.y < v) + (o.z < v) + (o.w < v);
+      }
+      eq[rank] = v;
+    }
+    c2g_wave_sync();
+  }
+  if (sz <= 8) return bucket_sum_small<8>(e, sz, qjump);
+  if (sz <= 32) return bucket_sum_small<32>(e, sz, qjump);
+  if (sz > kWaveSort)
+    for (int t = 1; t < sz; t++) {
+      const int32_t v = e[t];
+      int u = t - 1;
+      while (u >= 0 && e[u] > v) {
+        e[u + 1] = e[u];
+        u--;
+      }
+      e[u + 1] = v;
+    }
+  double s = 0.0;
+  int t = 0;
+  for (; t + 8 <= sz; t += 8) {
+    int32_t v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = e[t + k];
+#pragma unroll
+    for (int k = 0; k < 8; k++) s = s + ((v[k] & 1) ? qjump : -qjump);
+  }
+  for (; t < sz; t++) s = s + ((e[t] & 1) ? qjump : -qjump);
+  return s;
+}
+
+// Zero the n4 int4 of counters for the next sweep, in whole lines.
+__global__ void c2g_clear(int4 *cnt, int64_t n4) {
+  const int stride = gridDim.x * blockDim.x;
+  for (int64_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n4; k += stride)
+    cnt[k] = make_int4(0, 0, 0, 0);
+}
+
+// Value of a cell's node-order sum from its counts.
+__device__ __forceinline__ double cell_value(int32_t w, double qjump, const Buckets &b) {
+  const int p = w & 0xffff, q = (w >> 16) & 0xffff;
+  if (q == 0) {
+    double s = 0.0;
+    for (int t = 0; t < p; t++) s = s + qjump;
+    return s;
+  }
+  if (p == 0) {
+    double s = 0.0;
+    for (int t = 0; t < q; t++) s = s + (-qjump);
+    return s;
+  }
+  if (p <= 2 && q <= 2) return (double)(p - q) * qjump;
+  const int32_t nb = bucket_of(w);  // flagged, hence marked
+  return nb < b.bcap ? b.vals[nb] : 0.0 / 0.0;
+}
+
+// cell_value for the common cells first: a single crossing of either sign
+// (0 + qjump and 0 - qjump are exact).
+__device__ __forceinline__ double cell_value_fast(int32_t w, double qjump, const Buckets &b) {
+  if (w == 1) return qjump;
+  if (w == (1 << 16)) return -qjump;
+  return cell_value(w, qjump, b);
+}
+
 // qbot (contours.f90:234-238): qbot(1) = 0, qbot(ix+1) = qbot(ix) + qjx(ix)
 // over the non-empty bottom-row counters, in order.  Per pass of kQbotPart
 // counters the block evaluates the counters' values and compacts the
@@ -362,22 +461,35 @@ __device__ __forceinline__ int wave_scan_i32(int v) {
 // each group of eight dependent adds, overwriting each value with the chain
 // after it; every counter then reads the value after the last non-empty one
 // at or before it.  The additions are the reference's, in its order.
-// Any nxf (passes of kQbotPart).  The bucket sums of the order-dependent cells (usually
-// none) are made first, one thread per bucket.  Being the last reader of
-// the counters and of flags[0..5], it leaves them zero for the next sweep
-// (the bucket count moves to flags[6] for c2g_bucket_clear).
+// Any nxf (passes of kQbotPart).  Block 0 runs the chain; the others make
+// the bucket sums of the order-dependent cells meanwhile, one thread per
+// bucket (block 0 those of its own counters).  Being the last reader of the
+// bottom-row counters, block 0 leaves them zero for the next sweep.
 static constexpr int kQbotPart = 4096;  // counters per pass, four per thread
 static constexpr int kQbotPer = kQbotPart / 1024;
 __global__ void __launch_bounds__(1024) c2g_qbot(int32_t *qjx, double *qbot, int nxf,
                                                  int64_t nkey, double qjump, Buckets bk,
                                                  int32_t *flags) {
-  __shared__ double comp[kQbotPart + 8];  // non-empty values, then the chain after each
+  __shared__ __align__(16) double comp[kQbotPart + 8];  // non-empty values, then the chain after each
   __shared__ int wsum[16];
   __shared__ double vin;  // the chain's value entering the pass
   const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
-  const int nb_used = min(flags[4], bk.bcap);
-  for (int nb = tid; nb < nb_used; nb += blockDim.x) bucket_sum(bk, nb, qjump);
-  __syncthreads();
+  int32_t *lds = (int32_t *)comp + wv * kWaveSort;
+  static_assert(16 * kWaveSort * sizeof(int32_t) <= sizeof(comp), "sorting space of 16 waves");
+  if (blockIdx.x > 0) {
+    // 64 buckets to a wavefront, neighbouring ones to different workgroups
+    const int nb_used = min(flags[0], bk.bcap), stride = (gridDim.x - 1) * 1024;
+    for (int b0 = (wv * (gridDim.x - 1) + blockIdx.x - 1) * 64; b0 < nb_used; b0 += stride) {
+      const int nb = b0 + l;
+      const bool mine = nb < nb_used && bk.cell[nb] < nkey;
+      const double s = bucket_sums(bk, mine ? nb : -1, qjump, lds);
+      if (mine) {
+        bk.vals[nb] = s;
+        if (bk.list[4 * nb + 2] != bk.list[4 * nb + 1]) atomicOr(&flags[8], 2);
+      }
+    }
+    return;
+  }
   double v = 0.0;  // qbot(1); thread 0 carries the chain across passes
   if (tid == 0) qbot[0] = 0.0;
   for (int part = 0; part < nxf - 1; part += kQbotPart) {
@@ -391,7 +503,13 @@ __global__ void __launch_bounds__(1024) c2g_qbot(int32_t *qjx, double *qbot, int
 #pragma unroll
     for (int u = 0; u < kQbotPer; u++) {
       if (w[u]) qjx[part + t0 + u] = 0;
-      cv[u] = w[u] ? cell_value(w[u], nkey + part + t0 + u, qjump, bk) : 0.0;
+      const bool fl = is_flagged(w[u]);
+      const int32_t nb = fl ? bucket_of(w[u]) : -1;
+      cv[u] = w[u] && !fl ? cell_value(w[u], qjump, bk) : 0.0;
+      if (__ballot(fl)) {
+        const double s = bucket_sums(bk, nb < bk.bcap ? nb : -1, qjump, lds);
+        if (fl) cv[u] = nb < bk.bcap ? s : 0.0 / 0.0;
+      }
       cnt += w[u] != 0;
     }
     const int incl = wave_scan_i32(cnt);
@@ -443,18 +561,18 @@ __global__ void __launch_bounds__(1024) c2g_qbot(int32_t *qjx, double *qbot, int
     }
     __syncthreads();
   }
-  if (tid == 0) {
-    qjx[nxf - 1] = 0;  // the last counter is never part of the chain
-    flags[6] = flags[4];
-#pragma unroll
-    for (int k = 0; k < 6; k++) flags[k] = 0;
-    flags[7] = 0;
-  }
+  if (tid == 0) qjx[nxf - 1] = 0;  // the last counter is never part of the chain
 }
 
 // y sweep (contours.f90:272-277): one wavefront per fine column.
+// It and c2g_colscan_avg9, running after the last readers of the sweep's
+// flags, leave them zero for the next sweep.
+__device__ __forceinline__ void reset_flags(int32_t *flags) {
+  if (blockIdx.x == 0 && threadIdx.x < 8) flags[threadIdx.x] = 0;
+}
 __global__ void c2g_colscan(const int32_t *cnt, const double *qbot, double *fq, int nxf, int nyf,
-                            double qjump, Buckets bk) {
+                            double qjump, Buckets bk, int32_t *flags) {
+  reset_flags(flags);
   const int wpb = blockDim.x / 64;
   const int col = blockIdx.x * wpb + threadIdx.x / 64;
   const int l = threadIdx.x & 63;
@@ -473,7 +591,7 @@ __global__ void c2g_colscan(const int32_t *cnt, const double *qbot, double *fq, 
     for (int u = 0; u < U; u++) {
       const int r = base + 64 * u + l;  // iy-1
       const double cv =
-          w[u] ? cell_value(w[u], (int64_t)col * nyf + r, qjump, bk) : 0.0;
+          w[u] ? cell_value(w[u], qjump, bk) : 0.0;
       uint64_t mask = __ballot(w[u] != 0);
       double mine = v;
       while (mask) {
@@ -518,8 +636,10 @@ static constexpr int kAvgW = 2 * kAvgK + 1;
 
 __global__ void __launch_bounds__(64 * kAvgW)
     c2g_colscan_avg9(const int32_t *__restrict__ cnt, const double *__restrict__ qbot,
-                     double *__restrict__ out, int n2, double qjump, Buckets bk) {
+                     double *__restrict__ out, int n2, double qjump, Buckets bk,
+                     int32_t *__restrict__ flags) {
   constexpr int TPS = 4;  // tiles of 64 rows per stage (one barrier each)
+  reset_flags(flags);
   __shared__ double tile[2][kAvgW][64 * TPS + 1];  // [buffer][column][1 + row], 0: carry
   __shared__ double edge[kAvgW][3];                // rows 0, 1 and n2 - 1 of each column
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -549,7 +669,7 @@ __global__ void __launch_bounds__(64 * kAvgW)
     for (int u = 0; u < TPS; u++) {
       if (t0 + u < ntiles) {
         const int r = 64 * (t0 + u) + l;
-        const double cv = wv[u] ? cell_value_fast(wv[u], (int64_t)col * n2 + r, qjump, bk) : 0.0;
+        const double cv = wv[u] ? cell_value_fast(wv[u], qjump, bk) : 0.0;
         uint64_t mask = __ballot(wv[u] != 0);
         double mine = v;
         while (mask) {
@@ -657,30 +777,27 @@ int fine_sweep(Ctx &c, const double *xq, const double *yq, const int32_t *nextq,
   a.cnt = cnt;
   a.qjx = qjx;
   a.flags = c.flags;
-  a.bk.tkey = c.rp_tkey;
-  a.bk.tid = c.rp_tid;
+  a.bk.cell = c.rp_cell;
   a.bk.list = c.rp_list;
   a.bk.slots = c.replay;
   a.bk.vals = c.replay_val;
-  a.bk.tmask = (uint32_t)(c.rp_tsize - 1);
   a.bk.bcap = (int32_t)c.rp_bcap;
   a.bk.scap = c.replay_cap;
   const int nb = (n + 255) / 256;
   if (n > 0) {
-    hipLaunchKernelGGL(c2g_nodes, dim3(nb), dim3(256), 0, c.s, a);
+    hipLaunchKernelGGL(c2g_nodes<true>, dim3(nb), dim3(256), 0, c.s, a);
     HYD_HIP(hipGetLastError());
-    const int nbk = std::min(nb, 1024);
-    hipLaunchKernelGGL(c2g_buckets<0>, dim3(nbk), dim3(256), 0, c.s, a);
-    hipLaunchKernelGGL(c2g_buckets<1>, dim3(nbk), dim3(256), 0, c.s, a);
+    hipLaunchKernelGGL(c2g_claim, dim3(256), dim3(256), 0, c.s, a);
+    hipLaunchKernelGGL(c2g_fill, dim3(std::min(nb, 1024)), dim3(256), 0, c.s, a);
   }
-  hipLaunchKernelGGL(c2g_qbot, dim3(1), dim3(1024), 0, c.s, qjx, qbot, nxf, nfine, a.qjump, a.bk,
+  hipLaunchKernelGGL(c2g_qbot, dim3(256), dim3(1024), 0, c.s, qjx, qbot, nxf, nfine, a.qjump, a.bk,
                      c.flags);
   if (avg)
     hipLaunchKernelGGL(c2g_colscan_avg9, dim3(nxf / 2 / kAvgK), dim3(64 * kAvgW), 0, c.s, cnt,
-                       qbot, avg, nxf, a.qjump, a.bk);
+                       qbot, avg, nxf, a.qjump, a.bk, c.flags);
   else
     hipLaunchKernelGGL(c2g_colscan, dim3((nxf + 3) / 4), dim3(256), 0, c.s, cnt, qbot, fq, nxf,
-                       nyf, a.qjump, a.bk);
+                       nyf, a.qjump, a.bk, c.flags);
   c.clr_cnt = cnt;
   c.clr_n4 = nfine / 4;
   c.clear_pending = true;
@@ -690,26 +807,12 @@ int fine_sweep(Ctx &c, const double *xq, const double *yq, const int32_t *nextq,
   return HYD_OK;
 }
 
-static Buckets ctx_buckets(const Ctx &c) {
-  Buckets b;
-  b.tkey = c.rp_tkey;
-  b.tid = c.rp_tid;
-  b.list = c.rp_list;
-  b.slots = c.replay;
-  b.vals = c.replay_val;
-  b.tmask = (uint32_t)(c.rp_tsize - 1);
-  b.bcap = (int32_t)c.rp_bcap;
-  b.scap = c.replay_cap;
-  return b;
-}
-
 // The pending clearing of the last sweep, on the current stream c.s (on
 // the second stream it leaves an event for the next sweep to wait on).
 int sweep_clear(Ctx &c) {
   if (!c.clear_pending) return HYD_OK;
   c.clear_pending = false;
-  hipLaunchKernelGGL(c2g_bucket_clear, dim3(1024), dim3(256), 0, c.s, ctx_buckets(c), c.flags,
-                     (int4 *)c.clr_cnt, c.clr_n4);
+  hipLaunchKernelGGL(c2g_clear, dim3(1024), dim3(256), 0, c.s, (int4 *)c.clr_cnt, c.clr_n4);
   HYD_HIP(hipGetLastError());
   if (c.s == c.s2) {
     HYD_HIP(hipEventRecord(c.ev_cleared, c.s));
@@ -729,17 +832,15 @@ int sweep_clear_join(Ctx &c) {
 }
 
 // Reports (and clears) an overflow of the order-dependent-cell buckets of any
-// sweep since the last check; the bucket table is emptied so that the next
-// sweep starts clean.
+// sweep since the last check.
 int c2g_status(Ctx &c) {
   int32_t e = 0;
   HYD_HIP(hipMemcpyAsync(&e, c.flags + 8, sizeof(int32_t), hipMemcpyDeviceToHost, c.s));
   HYD_HIP(hipStreamSynchronize(c.s));
   if (e == 0) return HYD_OK;
-  HYD_HIP(hipMemsetAsync(c.rp_tkey, 0xff, sizeof(int32_t) * c.rp_tsize, c.s));
   HYD_HIP(hipMemsetAsync(c.flags + 8, 0, sizeof(int32_t), c.s));
   HYD_HIP(hipStreamSynchronize(c.s));
-  set_error("con2grid: too many order-dependent cells for the bucket table");
+  set_error("con2grid: too many order-dependent cells for the buckets");
   return HYD_ECAPACITY;
 }
 
@@ -1011,7 +1112,7 @@ int con2grid_mixed(Ctx &c, float *qc, bool defer_mean) {
     a.cnt = c.cnt;
     a.qjx = c.qjx_cnt;
     a.flags = c.flags;
-    hipLaunchKernelGGL(c2g_nodes, dim3((n + 255) / 256), dim3(256), 0, c.s, a);
+    hipLaunchKernelGGL(c2g_nodes<false>, dim3((n + 255) / 256), dim3(256), 0, c.s, a);
   }
   const double qjump = c.hsc->qjump;  // fixed between recontourings
   hipLaunchKernelGGL(c2g_qbot_int, dim3(1), dim3(1024), 0, c.s, c.qjx_cnt, c.qb32, nxf);

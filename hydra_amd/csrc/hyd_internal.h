@@ -143,9 +143,9 @@ struct Ctx {
   // cnt, qjx_cnt and flags[0..7] are all zero: every FP64 sweep clears what
   // it used on its way out, so the next one skips the clearing fills
   bool sweep_clean = false;
-  // order-dependent cells: key -> bucket table, bucket list, entries, sums
-  int32_t *rp_tkey = nullptr, *rp_tid = nullptr, *rp_list = nullptr;
-  int64_t rp_tsize = 0, rp_bcap = 0;
+  // order-dependent cells: their list, buckets, entries, sums
+  int32_t *rp_cell = nullptr, *rp_list = nullptr;
+  int64_t rp_bcap = 0;
   int32_t *replay = nullptr;   // bucket entries (node << 1 | sign)
   double *replay_val = nullptr;
   int64_t replay_cap = 0;
@@ -226,8 +226,7 @@ struct Ctx {
   double *diag_out = nullptr;    // 8 scratch results
   hipStream_t s2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // The clearing that ends a sweep (counters zeroed, order-dependent cell
-  // table emptied) may be left to the caller (defer_clear), who runs it
+  // The clearing that ends a sweep (counters zeroed) may be left to the caller (defer_clear), who runs it
   // later on either stream (sweep_clear); the next sweep first waits for it
   // (sweep_clear_join), or runs it itself if nobody has.
   bool defer_clear = false, clear_pending = false, clear_event = false;

@@ -369,3 +369,53 @@ def test_con2grid_order_dependent_cells_bitwise(ng, hyd_cache):
         assert np.array_equal(cnt_h.ravel(), cnt_o.ravel())
         assert bits_equal(qc_h, qc_o)
         assert bits_equal(h.con2grid(c["x"], c["y"], c["nextq"], c["qjump"]), o.con2grid())
+
+
+def _crowded(ng, kind):
+    """Contours that fill cells' buckets: "chords", long random segments, so
+    that most fine cells become order-dependent, more of them per block of
+    nodes than its list holds; "ringsN", rings about one fine cell wide
+    inside N x N cells, so that buckets hold from a few entries to a thousand."""
+    rng = np.random.default_rng(len(kind))
+    h = 2 * np.pi / (4 * ng)
+    npq, xs, ys = [], [], []
+    if kind == "chords":
+        npq = [60] * 50
+        xs.append(rng.uniform(-np.pi, np.pi, 3000))
+        ys.append(rng.uniform(-np.pi, np.pi, 3000))
+    else:
+        side = int(kind[5:]) * h
+        for _ in range(2500 if kind == "rings1" else 400):
+            m = int(rng.integers(5, 60))
+            t = np.sort(rng.uniform(0, 2 * np.pi, m))[::int(rng.choice([-1, 1]))]
+            cx, cy = rng.uniform(0, side, 2) + 0.1
+            xs.append(cx + 0.9 * h * np.cos(t))
+            ys.append(cy + 0.9 * h * np.sin(t))
+            npq.append(m)
+    npq = np.array(npq, np.int32)
+    i2 = np.cumsum(npq).astype(np.int32)
+    nxt = np.arange(2, i2[-1] + 2, dtype=np.int32)
+    nxt[i2 - 1] = i2 - npq + 1
+    return dict(x=np.concatenate(xs), y=np.concatenate(ys), nextq=nxt, i1q=i2 - npq + 1, i2q=i2,
+                npq=npq, indq=np.ones(len(npq), np.int32), qjump=0.1234567891234)
+
+
+@pytest.mark.parametrize("kind,least", [("chords", 10000), ("rings1", 6), ("rings3", 10),
+                                        ("rings10", 60)])
+def test_con2grid_crowded_cells_bitwise(kind, least, hyd_cache):
+    """Buckets of every size, and more order-dependent cells in a block of
+    nodes than its list holds, against the oracle's grid."""
+    from oracle.hyo import Oracle
+    ng = 32
+    c = _crowded(ng, kind)
+    o = Oracle(ng)
+    o.set_contours(c)
+    qc_o, cnt_o = o.con2grid(with_counts=True)
+    cells, _ = _order_dependent(c, ng)
+    assert cells >= least  # the case is exercised
+    h = hyd_cache(ng)
+    for rep in range(2):
+        qc_h, cnt_h = h.con2grid(c["x"], c["y"], c["nextq"], c["qjump"], with_counts=True)
+        assert np.array_equal(cnt_h, cnt_o)
+        assert bits_equal(qc_h, qc_o)
+        assert bits_equal(h.con2grid(c["x"], c["y"], c["nextq"], c["qjump"]), qc_o)
