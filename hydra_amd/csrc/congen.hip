@@ -336,7 +336,7 @@ __global__ void cg_successor(const int64_t *kib, const int32_t *lev_of_gid, int6
 // exits (a saddle, whose exit depends on the order of visits: icrtab is
 // last-in-first-out and noctab counts down, not decremented when the walk
 // closes, congen.f90:283).  Pointer jumping finds every chain, its length and
-// each crossing's position; a thread per level then walks the chains in the
+// each crossing's position; a wavefront per level then walks the chains in the
 // reference's order -- start at the lowest unused crossing, which is the
 // lowest crossing of the first unused chain -- taking only the saddle
 // decisions sequentially; a last pass writes every crossing to its place in
@@ -420,7 +420,7 @@ __global__ void cw_rank_jump(const int32_t *R, const int32_t *Q, int64_t n, int3
 struct ChainTab {
   int32_t *key, *pos;       // per crossing
   int32_t *hd, *len, *cmin;  // per key: head distance, length, lowest crossing
-  int8_t *loop, *used;       // per key
+  int8_t *loop;              // per key
   int64_t *aoff, *boff;      // per key: output offsets of the (up to two) pieces
   int32_t *afrom;            // per key: first position of piece a
 };
@@ -464,67 +464,216 @@ __global__ void cw_fill_tab(ChainTab t, int64_t n) {
   t.len[c] = 0;
   t.cmin[c] = 0x7fffffff;
   t.loop[c] = 0;
-  t.used[c] = 0;
+  t.afrom[c] = 0;
 }
-// starts (chain minima) in crossing order; soff[lv] = first start of level lv
-__global__ void cw_walk(const int32_t *starts, const int64_t *soff, const int32_t *scnt,
-                        const int64_t *succ, const int64_t *sad2, int32_t *sadcnt,
-                        const int64_t *lev_base, const int64_t *lev_n, int nlev, ChainTab t,
-                        int64_t *cyc_start, int32_t *cyc_len, int32_t *cyc_count, int32_t *err) {
-  const int lv = blockIdx.x * blockDim.x + threadIdx.x;
-  if (lv >= nlev) return;
+// The chains that end at a saddle, as a graph: chain j (in the order of the
+// crossings that end them; rank = an exclusive scan of the saddle flags) has
+// len[j] crossings and, at its saddle, two exits: the chains a[j] (taken
+// first) and b[j], numbered within their level.  A saddle is known by its
+// first exit's chain.  kBadChain: not an exit of this level.
+static constexpr int32_t kBadChain = -1;
+struct WalkGraph {
+  int32_t *rank;      // per crossing
+  int32_t *end;       // per chain: its key (end crossing)
+  int32_t *a, *b, *len;
+  int32_t *off;       // per chain: where the walk put it (work space)
+  int8_t *state;      // per chain (work space): visits left of its saddle, used
+};
+
+__global__ void cw_saddle_flag(const int64_t *sad2, int64_t n, int32_t *flag) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < n) flag[c] = sad2[c] >= 0 ? 1 : 0;
+}
+__global__ void cw_graph(const int64_t *succ, const int64_t *sad2, const int32_t *lev_of_gid,
+                         const int64_t *lev_base, const int64_t *lev_n, int64_t n, ChainTab t,
+                         WalkGraph g) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= n || sad2[c] < 0) return;
+  const int lv = lev_of_gid[c];
+  const int64_t lb = lev_base[lv], le = lb + lev_n[lv];
+  const int32_t r0 = g.rank[lb], j = g.rank[c];
+  g.end[j] = (int32_t)c;
+  g.len[j] = t.len[c];
+  const int64_t ex[2] = {sad2[c], succ[c]};
+  int32_t id[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const bool in = ex[k] >= lb && ex[k] < le;
+    const int32_t kk = in ? t.key[ex[k]] : 0;
+    id[k] = in && t.pos[ex[k]] == 0 && !t.loop[kk] ? g.rank[kk] - r0 : kBadChain;
+  }
+  g.a[j] = id[0];
+  g.b[j] = id[1];
+}
+
+// The walk of a level's chains, a wavefront per level; starts (chain
+// minima, one per chain) in crossing order, soff[lv] = first start of level
+// lv.  64 starts are looked at together: loops only take their place in the
+// output (a scan of their lengths); a start on an unused saddle chain
+// begins a walk over the graph.  That walk is serial -- each exit depends on
+// the visits before -- and bound by the latency of its dependent reads, so
+// the level's graph and visit counts are kept in LDS (13 bytes a chain;
+// levels of more than kWalkChains chains walk them in global memory).  A
+// developed ng=64 flow (2e5 crossings): 38.0 ms with a thread per level
+// chasing the crossings' tables in global memory.
+static constexpr int kWalkChains = 12000;
+struct WalkLds {
+  int32_t len[kWalkChains], off[kWalkChains];
+  uint16_t a[kWalkChains], b[kWalkChains];  // 0xffff: kBadChain
+  int8_t state[kWalkChains];
+};
+
+// Visit counts and used marks, read and written by every lane alike.
+template <class T>
+struct WalkState {
+  volatile T *p;
+  __device__ int operator()(int32_t j) const { return p[j]; }
+  __device__ void operator()(int32_t j, int v) const { p[j] = (T)v; }
+};
+
+// Walks from chain h (position ps) at output offset w; returns the offset
+// after it.  Lane-uniform.
+template <class IDX, class LEN, class OFF, class ST>
+__device__ __forceinline__ int64_t walk_from(int32_t h, int32_t ps, int64_t w, int64_t nn,
+                                             IDX exits, LEN len, OFF off, ST state,
+                                             int64_t &tail, int32_t *err) {
+  // state: bits 0-1 visits left of the saddle whose first exit this is,
+  // bit 2 used
+  state(h, state(h) | 4);
+  off(h, w);
+  w += len(h) - ps;
+  tail = -1;
+  int32_t cur = h;
+  for (int64_t guard = 0;; guard++) {
+    int32_t ea, eb;
+    exits(cur, ea, eb);
+    if (ea == kBadChain || guard > nn) {
+      atomicAdd(err, 1);
+      break;
+    }
+    const int sa = state(ea);
+    const int32_t nxt = (sa & 3) == 2 ? ea : eb;
+    if (nxt == h && ps == 0) break;  // back at the start: not counted down
+    state(ea, (sa & 4) | (((sa & 3) - 1) & 3));
+    if (nxt == kBadChain) {
+      atomicAdd(err, 1);
+      break;
+    }
+    if (nxt == h) {  // the piece of the first chain before the start
+      tail = w;
+      w += ps;
+      break;
+    }
+    const int sn = state(nxt);
+    if (sn & 4) {
+      atomicAdd(err, 1);
+      break;
+    }
+    state(nxt, sn | 4);
+    off(nxt, w);
+    w += len(nxt);
+    cur = nxt;
+  }
+  return w;
+}
+
+__global__ void __launch_bounds__(64) cw_walk(const int32_t *starts, const int64_t *soff,
+                                              const int32_t *scnt, const int64_t *lev_base,
+                                              const int64_t *lev_n, ChainTab t, WalkGraph g,
+                                              int64_t ntot, int32_t nchain, int64_t *cyc_start,
+                                              int32_t *cyc_len, int32_t *cyc_count,
+                                              int32_t *err) {
+  extern __shared__ __align__(16) unsigned char walk_raw[];
+  WalkLds &L = *(WalkLds *)walk_raw;
+  const int lv = blockIdx.x, l = threadIdx.x;
   const int64_t b = lev_base[lv], nn = lev_n[lv];
+  const int32_t r0 = b < ntot ? g.rank[b] : nchain;
+  const int32_t m = (b + nn < ntot ? g.rank[b + nn] : nchain) - r0;
+  const bool in_lds = m <= kWalkChains;
+  for (int32_t j = l; j < m; j += 64) {
+    if (in_lds) {
+      L.a[j] = (uint16_t)g.a[r0 + j];
+      L.b[j] = (uint16_t)g.b[r0 + j];
+      L.len[j] = g.len[r0 + j];
+      L.state[j] = 2;
+    } else {
+      g.state[r0 + j] = 2;
+    }
+  }
+  __syncthreads();
   int64_t w = b;
   int32_t nc = 0;
-  for (int32_t i = 0; i < scnt[lv]; i++) {
-    const int32_t s = starts[soff[lv] + i];
-    const int32_t h = t.key[s];
-    if (t.used[h]) continue;
-    t.used[h] = 1;
-    const int64_t start = w;
-    if (t.loop[h]) {
-      t.afrom[h] = 0;
-      t.aoff[h] = w;
-      w += t.len[h];
-    } else {
-      const int32_t ps = t.pos[s];
-      t.afrom[h] = ps;
-      t.aoff[h] = w;
-      w += t.len[h] - ps;
-      int32_t cur = h;
-      for (int64_t guard = 0;; guard++) {
-        const int64_t e2 = sad2[cur];
-        const int32_t noc = sadcnt[e2];
-        const int64_t nxt = noc == 2 ? e2 : succ[cur];
-        if (nxt == s) break;
-        sadcnt[e2] = noc - 1;
-        if (nxt < b || nxt >= b + nn || guard > nn || t.pos[nxt] != 0) {
-          atomicAdd(err, 1);
-          break;
-        }
-        const int32_t kn = t.key[nxt];
-        if (kn == h) {
-          t.boff[h] = w;
-          w += ps;
-          break;
-        }
-        if (t.used[kn] || t.loop[kn]) {
-          atomicAdd(err, 1);
-          break;
-        }
-        t.used[kn] = 1;
-        t.afrom[kn] = 0;
-        t.aoff[kn] = w;
-        w += t.len[kn];
-        cur = kn;
-      }
+  for (int32_t i0 = 0; i0 < scnt[lv]; i0 += 64) {
+    const bool valid = i0 + l < scnt[lv];
+    const int32_t s = valid ? starts[soff[lv] + i0 + l] : 0;
+    const int32_t h = valid ? t.key[s] : 0;
+    const bool loop = valid && t.loop[h];
+    const int32_t llen = loop ? t.len[h] : 0;
+    const int32_t ps = valid && !loop ? t.pos[s] : 0;
+    const int32_t hj = valid && !loop ? g.rank[h] - r0 : 0;
+    int64_t at = llen;  // exclusive scan of the loops' lengths
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t u = __shfl_up(at, o);
+      if (l >= o) at += u;
     }
-    cyc_start[b + nc] = start;
-    cyc_len[b + nc] = (int32_t)(w - start);
-    nc++;
+    const int64_t loops = __shfl(at, 63);
+    at += w - llen;
+    uint64_t sad = __ballot(valid && !loop), emit = __ballot(loop);
+    int64_t walked = 0, mylen = llen;
+    while (sad) {
+      const int q = __ffsll((unsigned long long)sad) - 1;
+      sad &= sad - 1;
+      const int32_t hq = __builtin_amdgcn_readlane(hj, q), pq = __builtin_amdgcn_readlane(ps, q);
+      if ((in_lds ? L.state[hq] : g.state[r0 + hq]) & 4) continue;
+      const int64_t w0 = __shfl(at, q);
+      int64_t tail, w1;
+      if (in_lds) {
+        w1 = walk_from(
+            hq, pq, w0, nn,
+            [&](int32_t j, int32_t &ea, int32_t &eb) {
+              ea = L.a[j] == 0xffff ? kBadChain : L.a[j];
+              eb = L.b[j] == 0xffff ? kBadChain : L.b[j];
+            },
+            [&](int32_t j) { return L.len[j]; },
+            [&](int32_t j, int64_t v) { L.off[j] = (int32_t)v; },
+            WalkState<int8_t>{L.state}, tail, err);
+      } else {
+        w1 = walk_from(
+            hq, pq, w0, nn,
+            [&](int32_t j, int32_t &ea, int32_t &eb) {
+              ea = g.a[r0 + j];
+              eb = g.b[r0 + j];
+            },
+            [&](int32_t j) { return g.len[r0 + j]; },
+            [&](int32_t j, int64_t v) { g.off[r0 + j] = (int32_t)v; },
+            WalkState<int8_t>{g.state + r0}, tail, err);
+      }
+      if (l == q) {
+        t.afrom[h] = ps;  // the other chains' pieces start at 0 (cw_fill_tab)
+        if (tail >= 0) t.boff[h] = tail;
+        mylen = w1 - w0;
+      }
+      emit |= 1ull << q;
+      walked += w1 - w0;
+      if (l > q) at += w1 - w0;
+    }
+    w += loops + walked;
+    if (emit >> l & 1) {
+      if (loop) t.aoff[h] = at;
+      const int32_t k = nc + __popcll(emit & ((1ull << l) - 1));
+      cyc_start[b + k] = at;
+      cyc_len[b + k] = (int32_t)mylen;
+    }
+    nc += __popcll(emit);
   }
-  if (w != b + nn) atomicAdd(err, 1);
-  cyc_count[lv] = nc;
+  __syncthreads();
+  for (int32_t j = l; j < m; j += 64)
+    t.aoff[g.end[r0 + j]] = in_lds ? L.off[j] : g.off[r0 + j];
+  if (l == 0) {
+    if (w != b + nn) atomicAdd(err, 1);
+    cyc_count[lv] = nc;
+  }
 }
 __global__ void cw_expand(ChainTab t, int64_t n, const int32_t *err, int64_t *order) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -543,21 +692,25 @@ __global__ void cg_gather(const int64_t *order, const double *xcr, const double 
   yd[t] = ycr[g];
 }
 
-__global__ void cg_fill_i32(int32_t *a, int64_t n, int32_t v) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) a[k] = v;
-}
 __global__ void cg_fill_i64(int64_t *a, int64_t n, int64_t v) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) a[k] = v;
 }
-__global__ void cg_nextq(int32_t *nextq, const int64_t *off, const int32_t *np, int ncont) {
+// The new contour store: contour c's nodes from src[c] to off[c], and their
+// links; a workgroup per contour.  (A pair of copies per contour, 24000 of
+// them for a developed ng=64 flow, took 36 ms on the GPU and 60 ms in all.)
+__global__ void cg_store(const double *bx, const double *by, const int64_t *src, double *xq,
+                         double *yq, int32_t *nextq, const int64_t *off, const int32_t *np,
+                         int ncont) {
   const int c = blockIdx.x;
   if (c >= ncont) return;
-  const int64_t o = off[c];
+  const int64_t o = off[c], f = src[c];
   const int n = np[c];
-  for (int i = threadIdx.x; i < n; i += blockDim.x)
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    xq[o + i] = bx[f + i];
+    yq[o + i] = by[f + i];
     nextq[o + i] = (int32_t)(i + 1 < n ? o + i + 2 : o + 1);
+  }
 }
 
 template <class T>
@@ -835,21 +988,19 @@ int recontour(Ctx &c, const double *qq) {
   hipLaunchKernelGGL(cg_fill_i64, dim3((hcap + 255) / 256), dim3(256), 0, c.s, h.v1, hcap, -1);
   hipLaunchKernelGGL(cg_fill_i64, dim3((hcap + 255) / 256), dim3(256), 0, c.s, h.v2, hcap, -1);
   int64_t *succ, *sad2;
-  int32_t *sadcnt, *errs;
+  int32_t *errs;
   HYD_CHECK(dbuf(c, "succ", nalloc, &succ));
   HYD_CHECK(dbuf(c, "sad2", nalloc, &sad2));
-  HYD_CHECK(dbuf(c, "sadcnt", nalloc, &sadcnt));
   HYD_CHECK(dbuf(c, "errs", 4, &errs));
   HYD_HIP(hipMemsetAsync(errs, 0, 16, c.s));
   if (ntot > 0) {
-    hipLaunchKernelGGL(cg_fill_i32, gb, dim3(256), 0, c.s, sadcnt, ntot, 2);
     hipLaunchKernelGGL(cg_hash_insert, gb, dim3(256), 0, c.s, kob, lev_of_gid, ntot, h, errs);
     hipLaunchKernelGGL(cg_successor, gb, dim3(256), 0, c.s, kib, lev_of_gid, ntot, h, succ, sad2,
                        errs + 1);
   }
   HYD_HIP(hipGetLastError());
   // ---- 5. walk: chains between saddles by pointer jumping, then the
-  // saddle decisions in the reference's order (one thread per level)
+  // saddle decisions in the reference's order (one wavefront per level)
   int64_t *order, *cyc_start, *d_cyc_base;
   int32_t *cyc_len, *cyc_count;
   HYD_CHECK(dbuf(c, "order", nalloc, &order));
@@ -879,10 +1030,18 @@ int recontour(Ctx &c, const double *qq) {
     HYD_CHECK(dbuf(c, "cw_len", nalloc, &tb.len));
     HYD_CHECK(dbuf(c, "cw_cmin", nalloc, &tb.cmin));
     HYD_CHECK(dbuf(c, "cw_loop", nalloc, &tb.loop));
-    HYD_CHECK(dbuf(c, "cw_used", nalloc, &tb.used));
     HYD_CHECK(dbuf(c, "cw_aoff", nalloc, &tb.aoff));
     HYD_CHECK(dbuf(c, "cw_boff", nalloc, &tb.boff));
     HYD_CHECK(dbuf(c, "cw_afrom", nalloc, &tb.afrom));
+    WalkGraph wg;
+    HYD_CHECK(dbuf(c, "cw_rank", nalloc, &wg.rank));
+    HYD_CHECK(dbuf(c, "cw_end", nalloc, &wg.end));
+    HYD_CHECK(dbuf(c, "cw_ea", nalloc, &wg.a));
+    HYD_CHECK(dbuf(c, "cw_eb", nalloc, &wg.b));
+    HYD_CHECK(dbuf(c, "cw_clen", nalloc, &wg.len));
+    HYD_CHECK(dbuf(c, "cw_off", nalloc, &wg.off));
+    HYD_CHECK(dbuf(c, "cw_state", nalloc, &wg.state));
+    int32_t nchain = 0;
     int8_t *sflag;
     int32_t *levcnt, *starts, *nsel;
     int64_t *d_soff;
@@ -930,6 +1089,19 @@ int recontour(Ctx &c, const double *qq) {
       HYD_CHECK(dbuf(c, "cw_seltmp", (int64_t)tbytes, &tmp));
       HYD_HIP(hipcub::DeviceSelect::Flagged(tmp, tbytes, ids, sflag, starts, nsel, (int)ntot,
                                             c.s));
+      // the saddle chains' graph (end: the flags until the graph fills it)
+      hipLaunchKernelGGL(cw_saddle_flag, gb, dim3(256), 0, c.s, sad2, ntot, wg.end);
+      HYD_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tbytes, wg.end, wg.rank, (int)ntot, c.s));
+      HYD_CHECK(dbuf(c, "cw_seltmp", (int64_t)tbytes, &tmp));
+      HYD_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tbytes, wg.end, wg.rank, (int)ntot, c.s));
+      int32_t last[2] = {0, 0};
+      HYD_HIP(hipMemcpyAsync(&last[0], wg.rank + ntot - 1, 4, hipMemcpyDeviceToHost, c.s));
+      HYD_HIP(hipMemcpyAsync(&last[1], wg.end + ntot - 1, 4, hipMemcpyDeviceToHost, c.s));
+      HYD_HIP(hipStreamSynchronize(c.s));
+      nchain = last[0] + last[1];
+      hipLaunchKernelGGL(cw_graph, gb, dim3(256), 0, c.s, succ, sad2, lev_of_gid, d_lev_base,
+                         d_lev_n, ntot, tb, wg);
+      HYD_HIP(hipGetLastError());
     }
     std::vector<int32_t> hlc(nlev);
     HYD_HIP(hipMemcpyAsync(hlc.data(), levcnt, 4 * nlev, hipMemcpyDeviceToHost, c.s));
@@ -941,9 +1113,11 @@ int recontour(Ctx &c, const double *qq) {
       so += hlc[lv];
     }
     HYD_HIP(hipMemcpyAsync(d_soff, hso.data(), 8 * nlev, hipMemcpyHostToDevice, c.s));
-    hipLaunchKernelGGL(cw_walk, dim3((nlev + 63) / 64), dim3(64), 0, c.s, starts, d_soff, levcnt,
-                       succ, sad2, sadcnt, d_lev_base, d_lev_n, nlev, tb, cyc_start, cyc_len,
-                       cyc_count, errs + 2);
+    HYD_HIP(hipFuncSetAttribute((const void *)cw_walk,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    hipLaunchKernelGGL(cw_walk, dim3(nlev), dim3(64), sizeof(WalkLds), c.s, starts, d_soff, levcnt,
+                       d_lev_base, d_lev_n, tb, wg, ntot, nchain, cyc_start, cyc_len, cyc_count,
+                       errs + 2);
     if (ntot > 0) hipLaunchKernelGGL(cw_expand, gb, dim3(256), 0, c.s, tb, ntot, errs + 2, order);
     HYD_HIP(hipGetLastError());
   }
@@ -1046,7 +1220,6 @@ int recontour(Ctx &c, const double *qq) {
   // ---- 7. new contour store (congen.f90:312-322, 112-125)
   const int nq = (int)alive.size();
   std::vector<int64_t> src_off(nq);
-  std::vector<int32_t> src_np(nq);
   int64_t npt = 0;
   c.i1q.resize(nq);
   c.i2q.resize(nq);
@@ -1055,7 +1228,6 @@ int recontour(Ctx &c, const double *qq) {
   for (int j = 0; j < nq; j++) {
     const int a = alive[j];
     src_off[j] = off[a];
-    src_np[j] = np[a];
     c.i1q[j] = (int32_t)(npt + 1);
     npt += np[a];
     c.i2q[j] = (int32_t)npt;
@@ -1067,21 +1239,20 @@ int recontour(Ctx &c, const double *qq) {
     set_error("recontour: node count exceeds the context capacity");
     return HYD_ECAPACITY;
   }
-  for (int j = 0; j < nq; j++) {
-    const int64_t dst = c.i1q[j] - 1;
-    HYD_HIP(hipMemcpyAsync(c.xq + dst, bx[cur] + src_off[j], 8 * src_np[j], hipMemcpyDeviceToDevice, c.s));
-    HYD_HIP(hipMemcpyAsync(c.yq + dst, by[cur] + src_off[j], 8 * src_np[j], hipMemcpyDeviceToDevice, c.s));
-  }
   {
     std::vector<int64_t> o1(nq);
     for (int j = 0; j < nq; j++) o1[j] = c.i1q[j] - 1;
-    int64_t *d_o;
+    int64_t *d_o, *d_f;
     int32_t *d_n;
+    HYD_CHECK(dbuf(c, "nq_src", std::max(nq, 1), &d_f));
     HYD_CHECK(dbuf(c, "nq_off", std::max(nq, 1), &d_o));
     HYD_CHECK(dbuf(c, "nq_np", std::max(nq, 1), &d_n));
     HYD_HIP(hipMemcpyAsync(d_o, o1.data(), 8 * nq, hipMemcpyHostToDevice, c.s));
     HYD_HIP(hipMemcpyAsync(d_n, c.npq.data(), 4 * nq, hipMemcpyHostToDevice, c.s));
-    if (nq > 0) hipLaunchKernelGGL(cg_nextq, dim3(nq), dim3(256), 0, c.s, c.nextq, d_o, d_n, nq);
+    HYD_HIP(hipMemcpyAsync(d_f, src_off.data(), 8 * nq, hipMemcpyHostToDevice, c.s));
+    if (nq > 0)
+      hipLaunchKernelGGL(cg_store, dim3(nq), dim3(256), 0, c.s, bx[cur], by[cur], d_f, c.xq, c.yq,
+                         c.nextq, d_o, d_n, nq);
     HYD_HIP(hipGetLastError());
     HYD_HIP(hipStreamSynchronize(c.s));
   }

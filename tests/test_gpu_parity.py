@@ -419,3 +419,24 @@ def test_con2grid_crowded_cells_bitwise(kind, least, hyd_cache):
         assert np.array_equal(cnt_h, cnt_o)
         assert bits_equal(qc_h, qc_o)
         assert bits_equal(h.con2grid(c["x"], c["y"], c["nextq"], c["qjump"]), qc_o)
+
+
+@pytest.mark.parametrize("ng", [64, 256])
+def test_recontour_of_noise_bitwise(ng):
+    """White noise has a saddle in every few grid boxes: the ordered walk
+    through them, with a level's chains in LDS (ng=64) and, beyond its
+    capacity of 12000 chains a level, in global memory (ng=256)."""
+    from hydra_amd import Hydra
+    from oracle.hyo import Oracle
+    q = np.random.default_rng(ng).standard_normal((ng, ng))
+    o = Oracle(ng, ncontq=3)
+    o.init_from_field(q)
+    o.recontour(o.d("qr").copy())
+    h = Hydra(ng, ncontq=3)
+    h.set_field(q)
+    h.recontour()
+    c, g = o.contours(), h.contours()
+    for k in ("nextq", "i1q", "i2q", "npq", "indq"):
+        assert np.array_equal(g[k], c[k]), k
+    assert bits_equal(g["x"], c["x"]) and bits_equal(g["y"], c["y"])
+    h.close()
