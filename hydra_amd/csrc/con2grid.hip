@@ -607,8 +607,11 @@ __global__ void c2g_colscan(const int32_t *cnt, const double *qbot, double *fq, 
 
 // Nine-point average of an (nh2 x nh2) column-major field f to (nh x nh),
 // contours.f90:298-326; out layout column-major with leading dim nh.
+// tot (or null; nh % 64 == 0): the sum of each 64 consecutive values, in any
+// order, for the sequential mean's guesses.
 template <class T>
-__global__ void c2g_avg9(const T *__restrict__ f, T *__restrict__ out, int nh) {
+__global__ void c2g_avg9(const T *__restrict__ f, T *__restrict__ out, int nh,
+                         double *__restrict__ tot) {
   const int iy = blockIdx.x * blockDim.x + threadIdx.x + 1;
   const int ix = blockIdx.y + 1;
   if (iy > nh) return;
@@ -619,9 +622,16 @@ __global__ void c2g_avg9(const T *__restrict__ f, T *__restrict__ out, int nh) {
   const T qev1_a = F(r1, c1 - 1), qev1_b = F(r0, c1 - 1);
   const T qod0 = F(r1 - 1, c1), qod2 = F(r1 - 1, c0), qod1 = F(r1 - 1, c1 - 1);
 #undef F
-  out[(int64_t)(ix - 1) * nh + (iy - 1)] =
-      (T)0.0625 * (qev0_a + qev0_b + qev2_a + qev2_b) +
-      (T)0.125 * (qev1_a + qev1_b + qod0 + qod2) + (T)0.25 * qod1;
+  const int64_t k = (int64_t)(ix - 1) * nh + (iy - 1);
+  const T r = (T)0.0625 * (qev0_a + qev0_b + qev2_a + qev2_b) +
+              (T)0.125 * (qev1_a + qev1_b + qod0 + qod2) + (T)0.25 * qod1;
+  out[k] = r;
+  if (tot) {
+    double s = (double)r;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) tot[k >> 6] = s;
+  }
 }
 
 // y sweep fused with the first nine-point average (contours.f90:272-277
@@ -873,9 +883,11 @@ int con2grid(Ctx &c, const double *xq, const double *yq, const int32_t *nextq, i
                        c.qjx_cnt, c.qbot, c.fq, fused ? c.mq : nullptr));
   if (!fused)
     hipLaunchKernelGGL(c2g_avg9<double>, dim3((nh1 + 255) / 256, nh1), dim3(256), 0, c.s, c.fq,
-                       c.mq, nh1);
+                       c.mq, nh1, nullptr);
+  // whole wavefronts of one column (nh2 a power of two): chunk totals too
+  double *tot = nh2 % 64 == 0 ? c.seq_tot : nullptr;
   hipLaunchKernelGGL(c2g_avg9<double>, dim3((nh2 + 255) / 256, nh2), dim3(256), 0, c.s, c.mq,
-                     c.c2g_w, nh2);
+                     c.c2g_w, nh2, tot);
   HYD_HIP(hipGetLastError());
   if (c.after_sweep) {
     auto fn = std::move(c.after_sweep);
@@ -883,7 +895,7 @@ int con2grid(Ctx &c, const double *xq, const double *yq, const int32_t *nextq, i
     HYD_CHECK(fn());
   }
   // sequential mean, contours.f90:330-336
-  HYD_CHECK(seqsum(c, c.c2g_w, N, c.dsum));
+  HYD_CHECK(seqsum(c, c.c2g_w, N, c.dsum, tot));
   if (defer_mean) return HYD_OK;
   hipLaunchKernelGGL(c2g_subtract, dim3((N + 255) / 256), dim3(256), 0, c.s, c.c2g_w, qc, N, c.dsum,
                      (double)N);
@@ -1124,10 +1136,10 @@ int con2grid_mixed(Ctx &c, float *qc, bool defer_mean) {
     hipLaunchKernelGGL(c2g_colscan_int, dim3((nxf + 3) / 4), dim3(256), 0, c.s, c.cnt, c.qb32,
                        c.fq32, nxf, nyf, qjump);
     hipLaunchKernelGGL(c2g_avg9<float>, dim3((nh1 + 255) / 256, nh1), dim3(256), 0, c.s, c.fq32,
-                       c.mq32, nh1);
+                       c.mq32, nh1, nullptr);
   }
   hipLaunchKernelGGL(c2g_avg9<float>, dim3((nh2 + 255) / 256, nh2), dim3(256), 0, c.s, c.mq32,
-                     c.fc32, nh2);
+                     c.fc32, nh2, nullptr);
   hipLaunchKernelGGL(c2g_sum_partial, dim3(1024), dim3(256), 0, c.s, c.fc32, N, c.part);
   hipLaunchKernelGGL(c2g_mean, dim3(1), dim3(1024), 0, c.s, c.part, (double)N);
   if (defer_mean) {

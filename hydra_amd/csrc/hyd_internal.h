@@ -238,6 +238,7 @@ struct Ctx {
   // the GPU and the second stream's work overlaps the single-workgroup
   // sequential mean instead); con2grid runs and clears it
   std::function<int()> after_sweep;
+  double *seq_tot = nullptr;  // chunk totals that a sum's producer makes for it
   void *seq_work = nullptr; // chunk table of seqsum
   int64_t seq_cap = 0;      // chunks it holds
   // work buffers of recontour / renode, allocated on first use
@@ -288,7 +289,9 @@ int gradient_dev(Ctx &c, const double *ff, double *fx, double *fy, double *tmp);
 int launch_xderiv(Ctx &c, const double *var, double *der);
 int launch_yderiv(Ctx &c, const double *var, double *der);
 
-int seqsum(Ctx &c, const double *a, int64_t n, double *dout);
+// totals: the sums (in any order) of each 64 values of a, if its producer has
+// made them
+int seqsum(Ctx &c, const double *a, int64_t n, double *dout, const double *totals = nullptr);
 // diagnostics (diag.hip)
 int diag_energy(Ctx &c, double *ekin, double *epot);
 void monitor_record(Ctx &c, const Scalars &s);

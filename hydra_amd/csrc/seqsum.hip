@@ -14,23 +14,39 @@
 //     any start on the grid whose run stays inside, provided the starts
 //     agree mod 2u (exact ties round to even).  Simulating the run from g
 //     and from g+u gives both translations D0, D1.
-//   * Level 1: chunks of kChunk values are simulated in parallel from a
-//     guessed start (double-double prefix of the chunk totals).  The guessed
-//     run is cut into segments wherever its binade changes; a segment starts
-//     with that "head" addition, which the chain performs exactly.  Windows
-//     of kWin chunks whose runs are single segments fold into composites
-//     (translations and admissible start intervals per start parity).
-//   * Level 2: one wavefront walks the windows 64 at a time.  Lanes take
-//     their start parities from a GF(2) scan, their candidate starts from a
-//     scan of the chosen translations, and accept while the candidate lies
-//     on the guessed run's grid inside the window's admissible interval.
-//     While all earlier lanes are accepted every scan partial is a
-//     difference of two values of one binade, hence exact, so the first
-//     rejected lane's candidate is the true sequential value.  That window,
-//     and every window that did not fold, is walked record by record the
-//     same way (heads added in order, rejected segments summed in order).
+//   * Classes.  A run that crosses binades is a translation per residue
+//     class of its start: for a start S = G_c + Delta, G_c = g + c u (u the
+//     grid of g's binade, c < M) and Delta a multiple of M u = 2 u_max (u_max
+//     the coarsest grid the run visits), every rounding of the run from S
+//     happens on the grid it happens on from G_c, displaced by Delta, as
+//     long as every partial sum stays in its binade: it ends exactly at
+//     E_c + Delta.  A table holds E_c and the admissible Delta interval of
+//     each class.
+//   * Chunks of 64 values are simulated in parallel from a guessed start
+//     (prefix of the chunk totals); windows of 16 chunks that
+//     stay in one binade fold into a composite by row scans; the other
+//     windows get a table, 64 classes walked at once, one to a lane: over
+//     each chunk by its translation where it has one, value by value where
+//     it changes binade.  The four windows of a workgroup then make the
+//     segment's table the same way, and above kTop segments sixteen tables
+//     at a time make the next level's.
+//   * The chain takes the top level's tables in order: the class from the
+//     low mantissa bits of S - g, a range check, S = E_c + Delta.  A start
+//     that its table does not cover descends to the entry's parts, at last
+//     to windows summed in order.
 // Every accepted translation is exact by construction and every rejected
 // piece is summed in order, so the result is the sequential sum bit for bit.
+//
+// What bounds it: latency -- a workgroup is one wavefront with a serial walk
+// of 64 values (about 2 us), and the chain's lookups (about 0.1 us each) are
+// serial; a dependent FP64 add takes 2.3 ns from registers, 4.3 ns from LDS
+// on gfx950.  A sum whose producer has made the chunk totals takes (before:
+// windows of 1024 values with 8 classes in four launches)
+//   2^20 values  31 us segments + 12 fold + 8 chain   (118)
+//   2^18         25 + 13                               (61)
+//   2^16         22 + 9                                (53)
+//   2^10         11 in one launch                      (38)
+#include <atomic>
 #include <mutex>
 
 #include "hyd_internal.h"
@@ -38,16 +54,35 @@
 namespace hyd {
 
 static constexpr int kChunk = 64;    // values per chunk
+static constexpr int kWin = 16;      // chunks per window
+static constexpr int kWins = 4;      // windows per segment (one workgroup)
+static constexpr int kSegVals = kChunk * kWin * kWins;
+static constexpr int kClasses = 64;  // classes of a table, one to a lane
+static constexpr int kFold = 16;     // entries folded into one of the next level
+static constexpr int kTop = 64;      // most entries of the level that the chain takes
+static constexpr int kChainWaves = 16;
+static constexpr int kGroup = kTop / kChainWaves;  // entries of one of its wavefronts
+static constexpr int kMaxLevels = 6;
+static constexpr int64_t kSeqOwnTotals = 512 * (int64_t)kSegVals;
 
-// A segment of a chunk's guessed run: an optional head addition, then
-// values whose guessed partial sums all share the binade of g.
-struct SegRec {
-  double g;       // guessed value after the head (or the chunk's guess)
-  double d0, d1;  // translations from g and from g + u
-  double lo, hi;  // extremes of the pre-rounding sums of both runs, rel. to g
-  double xh;      // the head value
-  int32_t chunk;
-  int32_t meta;   // b | e << 9 | head << 18 | replay << 19 (b, e: offsets in chunk)
+// A table: M classes (0: none; -1: the entry's sum starts at the very
+// beginning, c[0].e is its exact end), emax the coarsest binade its runs visit.
+// Class c: its start G_c, the end E_c from there, the displacements.
+struct __align__(16) SeqClass {
+  double s, e, lo, hi;
+};
+struct __align__(16) SeqTab {
+  double g;
+  int32_t M, emax;
+  SeqClass c[kClasses];
+};
+
+// A window of chunks that stays in one binade, folded: a start S in g's
+// binade, p grid steps (mod 2) from g and inside [lo_p, hi_p], ends at
+// S + d_p.
+struct SeqComp {
+  double g, d0, d1, lo0, hi0, lo1, hi1;
+  int32_t ok, eb;
 };
 
 __device__ __forceinline__ int binade(double x) {
@@ -56,20 +91,6 @@ __device__ __forceinline__ int binade(double x) {
 
 __device__ __forceinline__ double pow2_field(int eb) {  // 2^(eb-1023)
   return __longlong_as_double((int64_t)eb << 52);
-}
-
-__device__ __forceinline__ void two_sum(double a, double b, double &s, double &e) {
-  s = a + b;
-  const double bb = s - a;
-  e = (a - (s - bb)) + (b - bb);
-}
-
-__device__ __forceinline__ void dd_add(double ah, double al, double bh, double bl, double &sh,
-                                       double &sl) {
-  double s, e;
-  two_sum(ah, bh, s, e);
-  e = e + (al + bl);
-  two_sum(s, e, sh, sl);
 }
 
 // Is a run from start x (binade eb, same sign as g) strictly inside the
@@ -93,19 +114,53 @@ __device__ __forceinline__ double dpp_d(double x) {
   const int hi = dpp_i<CTRL>(__double2hiint(x));
   return __hiloint2double(hi, lo);
 }
-__device__ __forceinline__ double readlane_d(double x, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(x), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(x), l);
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t x, int l) {
-  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)x, l);
-  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), l);
-  return ((uint64_t)hi << 32) | lo;
-}
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
-// Inclusive wavefront scan of doubles (row shifts, then row broadcasts).
+// Inclusive scans inside each DPP row of 16 lanes.
+__device__ __forceinline__ double row_incl_add(double v) {
+  const int rl = lane_id() & 15;
+  double t;
+  t = dpp_d<0x111>(v); if (rl >= 1) v = t + v;
+  t = dpp_d<0x112>(v); if (rl >= 2) v = t + v;
+  t = dpp_d<0x114>(v); if (rl >= 4) v = t + v;
+  t = dpp_d<0x118>(v); if (rl >= 8) v = t + v;
+  return v;
+}
+
+// GF(2) affine maps p -> k ? p ^ c : c packed as (k << 1) | c; "then" applies
+// the earlier map t first.
+__device__ __forceinline__ int map_then(int t, int v) {
+  const int kv = v >> 1, cv = v & 1, kt = t >> 1, ct = t & 1;
+  return ((kv & kt) << 1) | (kv ? (ct ^ cv) : cv);
+}
+__device__ __forceinline__ int row_incl_map(int v) {
+  const int rl = lane_id() & 15;
+  int t;
+  t = dpp_i<0x111>(v); if (rl >= 1) v = map_then(t, v);
+  t = dpp_i<0x112>(v); if (rl >= 2) v = map_then(t, v);
+  t = dpp_i<0x114>(v); if (rl >= 4) v = map_then(t, v);
+  t = dpp_i<0x118>(v); if (rl >= 8) v = map_then(t, v);
+  return v;
+}
+
+__device__ __forceinline__ int segkey(double x) {
+  return (int)((uint64_t)__double_as_longlong(x) >> 52);  // sign and exponent
+}
+// Binades whose grid and its inverse are ordinary numbers; sums below or
+// above are left to the in-order path.
+__device__ __forceinline__ bool binade_ok(int eb) { return eb >= 64 && eb <= 2045; }
+
+__device__ __forceinline__ int parity_of(double num, double uinv) {
+  // num is an exact multiple of u = 1/uinv (a power of two), |num/u| < 2^53
+  return (int)((long long)(num * uinv) & 1);
+}
+
+// Wavefront sum in every lane and inclusive scan (any order: for guesses).
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
+  return v;
+}
 __device__ __forceinline__ double wave_incl_add(double v) {
   const int l = lane_id(), rl = l & 15;
   double t;
@@ -117,361 +172,388 @@ __device__ __forceinline__ double wave_incl_add(double v) {
   t = dpp_d<0x143>(v); if (l >= 32) v = t + v;
   return v;
 }
-// Inclusive scans inside each DPP row of 16 lanes.
-__device__ __forceinline__ double row_incl_add(double v) {
-  const int rl = lane_id() & 15;
-  double t;
-  t = dpp_d<0x111>(v); if (rl >= 1) v = t + v;
-  t = dpp_d<0x112>(v); if (rl >= 2) v = t + v;
-  t = dpp_d<0x114>(v); if (rl >= 4) v = t + v;
-  t = dpp_d<0x118>(v); if (rl >= 8) v = t + v;
-  return v;
-}
-// value of lane l-1 (0 for lane 0)
-__device__ __forceinline__ double wave_prev_d(double v) {
-  const double t = dpp_d<0x138>(v);
-  return lane_id() == 0 ? 0.0 : t;
-}
 
-// GF(2) affine maps p -> k ? p ^ c : c packed as (k << 1) | c; "then" applies
-// the earlier map t first.
-__device__ __forceinline__ int map_then(int t, int v) {
-  const int kv = v >> 1, cv = v & 1, kt = t >> 1, ct = t & 1;
-  return ((kv & kt) << 1) | (kv ? (ct ^ cv) : cv);
-}
-__device__ __forceinline__ int wave_incl_map(int v) {
-  const int l = lane_id(), rl = l & 15;
-  int t;
-  t = dpp_i<0x111>(v); if (rl >= 1) v = map_then(t, v);
-  t = dpp_i<0x112>(v); if (rl >= 2) v = map_then(t, v);
-  t = dpp_i<0x114>(v); if (rl >= 4) v = map_then(t, v);
-  t = dpp_i<0x118>(v); if (rl >= 8) v = map_then(t, v);
-  t = dpp_i<0x142>(v); if ((l & 31) >= 16) v = map_then(t, v);
-  t = dpp_i<0x143>(v); if (l >= 32) v = map_then(t, v);
-  return v;
-}
-
-__device__ __forceinline__ int row_incl_map(int v) {
-  const int rl = lane_id() & 15;
-  int t;
-  t = dpp_i<0x111>(v); if (rl >= 1) v = map_then(t, v);
-  t = dpp_i<0x112>(v); if (rl >= 2) v = map_then(t, v);
-  t = dpp_i<0x114>(v); if (rl >= 4) v = map_then(t, v);
-  t = dpp_i<0x118>(v); if (rl >= 8) v = map_then(t, v);
-  return v;
-}
-
-// ---- segments of a guessed run ---------------------------------------------
-__device__ __forceinline__ int segkey(double x) {
-  return (int)((uint64_t)__double_as_longlong(x) >> 52);  // sign and exponent
-}
-
-struct SegState {
-  double g, s0, s1, lo, hi, xh, u;
-  int b, head, bad, key;
+// ---- classes ----------------------------------------------------------------
+// A lane's walk from one class start: the value, and the interval of
+// displacements that leave every partial sum so far in its binade.
+struct Walk {
+  double S, dlo, dhi;
+  int emax;
+  bool ok;
 };
 
-__device__ __forceinline__ void seg_open(SegState &z, int b, int head, double xh, double g) {
-  const int eb = binade(g);
-  z.g = g;
-  z.s0 = g;
-  z.key = segkey(g);
-  // tiny binades are left to the in-order path (the chain uses 1/u = 2^(52-E))
-  z.bad = (eb < 64 || eb > 2045) ? 1 : 0;
-  z.u = z.bad ? 0.0 : pow2_field(eb) * 0x1p-52;
-  z.s1 = g + z.u;
-  if (segkey(z.s1) != z.key) z.bad = 1;
-  z.lo = 0.0;
-  z.hi = 0.0;
-  z.xh = xh;
-  z.b = b;
-  z.head = head;
-}
-
-__device__ __forceinline__ void seg_close(const SegState &z, int e, int64_t c, SegRec *out,
-                                          int &cnt, int cap) {
-  if (!(z.head || e > z.b)) return;  // empty leading segment
-  if (cnt < cap) {
-    SegRec r;
-    r.g = z.g;
-    r.d0 = z.s0 - z.g;
-    r.d1 = z.s1 - (z.g + z.u);
-    r.lo = z.lo;
-    r.hi = z.hi;
-    r.xh = z.xh;
-    r.chunk = (int32_t)c;
-    r.meta = z.b | (e << 9) | (z.head << 18) | (z.bad << 19);
-    out[cnt] = r;
-  }
-  cnt++;
-}
-
-__device__ __forceinline__ int parity_of(double num, double uinv) {
-  // num is an exact multiple of u = 1/uinv (a power of two), |num/u| < 2^53
-  return (int)((long long)(num * uinv) & 1);
-}
-
-// ---- composites -----------------------------------------------------------
-// A window of kWin consecutive chunks whose guessed runs each form a single
-// segment (no binade change, no replay) folds into one composite.  For a
-// start S_1 = g_1 + delta u on the grid of that binade the members are pure
-// translations: with p = parity(delta), member i starts at S_1 + off_i(p)
-// (off_i the sum of the earlier members' chosen translations, parities
-// following the GF(2) maps) and the window adds D(p) = off_(K+1)(p).  The
-// member chain would accept member i iff its start lies on the grid, inside
-// the binade with the 4-ulp margins around its run; those conditions are
-// intervals in delta, intersected per parity (level 1) with one extra ulp for
-// the rounding of the margin tests.  A start inside its interval is
-// therefore accepted by every member and gives the member chain's value;
-// any other window is summed by the member chain.
-static constexpr int kWin = 16;
-
-struct CompRec {
-  double g;                   // first member's guess
-  double d0, d1;              // window translations for start parity 0 / 1
-  double lo0, hi0, lo1, hi1;  // admissible delta (units of u, magnitude) per parity
-  int32_t win;                // window index
-  int32_t meta;               // nm | ok << 5 | (map k << 1 | map c) << 6
-  uint64_t cnts;              // record count of member chunk i in bits 4i..4i+3
-};
-
-// ---- level 1 --------------------------------------------------------------
-// One wavefront owns 64 consecutive chunks (a thread per chunk); the block's
-// 64 x 64 values are staged through LDS in one coalesced pass and each
-// thread walks its chunk's row, reading eight values ahead of its adds.
-// MODE 0: chunk totals from +0 (tot) and the block's double-double total
-//         (blk).
-// MODE 1: guesses (double-double prefix of the chunk totals: earlier blocks,
-//         then the block's own scan), segments of the guessed runs, and the
-//         composites of the block's kWin-chunk windows.
-__device__ __forceinline__ void dd_shfl_xor(double &h, double &l, int m) {
-  const double oh = __shfl_xor(h, m), ol = __shfl_xor(l, m);
-  dd_add(h, l, oh, ol, h, l);
-}
-
-template <int MODE>
-__global__ void __launch_bounds__(64) seq_chunks(const double *__restrict__ a, int64_t n,
-                                                 int64_t nch, double *tot, double2 *blk,
-                                                 SegRec *segs, int32_t *segcnt, CompRec *cps,
-                                                 int cap) {
-  __shared__ double tile[64][kChunk + 1];
-  __shared__ SegRec first[64];
-  __shared__ int32_t fcnt[64];
-  __shared__ double gnx;
-  const int t = threadIdx.x;
-  const int64_t c0 = (int64_t)blockIdx.x * 64;
-  const int64_t c = c0 + t;
-  // the block's 64 chunks, staged whole: thread t loads value t of every
-  // chunk (coalesced) before the prologue, so the loads overlap it
-  double v[kChunk];
-#pragma unroll
-  for (int j = 0; j < kChunk; j++) {
-    const int64_t gi = (c0 + j) * kChunk + t;
-    v[j] = gi < n ? a[gi] : 0.0;
-  }
-  double s = 0.0;
-  SegState z;
-  int cnt = 0;
-  SegRec *out = segs + c * cap;
-  double gch = 0.0;
-  // MODE 1 walks the two runs (from g and g + u) branch-free first; a chunk
-  // whose run from g changes binade is walked again, value by value, into
-  // its segments
-  double f0 = 0.0, f1 = 0.0, fmn = 0.0, fmx = 0.0;
-  bool chg = false, fbad = false;
-  if (MODE == 1) {
-    // offset: earlier blocks' totals (any order: the guess needs no exactness)
-    double oh = 0.0, ol = 0.0;
-    for (int64_t k = t; k < (int64_t)blockIdx.x; k += 64) {
-      const double2 v = blk[k];
-      dd_add(oh, ol, v.x, v.y, oh, ol);
-    }
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) dd_shfl_xor(oh, ol, m);
-    // inclusive scan of this block's chunk totals
-    double ih = c < nch ? tot[c] : 0.0, il = 0.0;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const double ph = __shfl_up(ih, o), pl = __shfl_up(il, o);
-      if (t >= o) dd_add(ph, pl, ih, il, ih, il);
-    }
-    double eh = __shfl_up(ih, 1), el = __shfl_up(il, 1);
-    if (t == 0) eh = el = 0.0;
-    double gh, gl;
-    dd_add(oh, ol, eh, el, gh, gl);
-    gch = gh + gl;
-    if (c < nch) seg_open(z, 0, 0, 0.0, gch);
-    f0 = z.s0;
-    f1 = z.s1;
-    fmn = fmx = z.g;
-    if (t == 63) {
-      dd_add(oh, ol, ih, il, gh, gl);
-      gnx = gh + gl;  // guess of the next block's first chunk
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < kChunk; j++) tile[j][t] = v[j];
-  __syncthreads();
-  if (c < nch) {
-    const double *row = tile[t];
-    auto step = [&](double x) {
-      if (MODE == 0) {
-        s = s + x;
-      } else {
-        // the rounded partial sums bound the exact ones within half an ulp,
-        // as the pre-rounding offsets would
-        const double t0 = f0 + x, t1 = f1 + x;
-        chg = chg || segkey(t0) != z.key;
-        fbad = fbad || segkey(t1) != z.key;
-        const double lo = t0 < t1 ? t0 : t1, hi = t0 < t1 ? t1 : t0;
-        fmn = lo < fmn ? lo : fmn;
-        fmx = hi > fmx ? hi : fmx;
-        f0 = t0;
-        f1 = t1;
-      }
-    };
-    if ((c + 1) * kChunk <= n) {
-      // eight values read ahead of the chain that consumes them
-#pragma unroll
-      for (int j0 = 0; j0 < kChunk; j0 += 8) {
-        double x[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) x[j] = row[j0 + j];
-#pragma unroll
-        for (int j = 0; j < 8; j++) step(x[j]);
-      }
-    } else {
-      const int e = (int)(n - c * kChunk);
-      for (int j = 0; j < e; j++) step(row[j]);
-    }
-  }
-  if (MODE == 0) {
-    if (c < nch) tot[c] = s;
-    double h = s, l = 0.0;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) dd_shfl_xor(h, l, m);
-    if (t == 0) blk[blockIdx.x] = make_double2(h, l);
+// Partial sums between mn and mx (one binade and sign): displacements keep
+// them inside it with 4 ulps to spare; sums nearer to its ends than that, or
+// outside the ordinary range, admit none.
+__device__ __forceinline__ void keep_binade(double mn, double mx, Walk &w) {
+  const int eb = binade(mn);
+  w.emax = max(w.emax, eb);
+  const double bl = pow2_field(eb), bh = pow2_field(eb + 1), m = pow2_field(max(eb - 50, 1));
+  const double L = mn > 0.0 ? bl + m : -bh + m, U = mn > 0.0 ? bh - m : -bl - m;
+  if (!binade_ok(eb) || mn < L || mx > U) {
+    w.dlo = fmax(w.dlo, 0.0);
+    w.dhi = fmin(w.dhi, 0.0);
     return;
   }
-  if (c < nch) {
-    const int e = (int)min((int64_t)kChunk, n - c * kChunk);
-    if (!chg) {
-      // one segment: the fast walk's sums (offsets exact within one binade)
-      z.s0 = f0;
-      z.s1 = f1;
-      z.lo = fmin(0.0, fmn - z.g);
-      z.hi = fmax(0.0, fmx - z.g);
-      if (fbad) z.bad = 1;
+  w.dlo = fmax(w.dlo, L - mn);
+  w.dhi = fmin(w.dhi, U - mx);
+}
+
+// A chunk's 64 values added in order (values beyond the array are zeros,
+// which change nothing), eight at a time: the sums of a group that all share
+// the binade so far only extend its extremes.
+__device__ __forceinline__ void ordered_chunk(const double *v, Walk &w) {
+  double S = w.S, mn = 0.0, mx = 0.0;
+  int key = -1;
+  for (int j0 = 0; j0 < kChunk; j0 += 8) {
+    double x[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] = v[j0 + j];
+    double y[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      S = S + x[j];
+      y[j] = S;
+    }
+    const double lo = fmin(fmin(fmin(y[0], y[1]), fmin(y[2], y[3])),
+                           fmin(fmin(y[4], y[5]), fmin(y[6], y[7])));
+    const double hi = fmax(fmax(fmax(y[0], y[1]), fmax(y[2], y[3])),
+                           fmax(fmax(y[4], y[5]), fmax(y[6], y[7])));
+    if (segkey(lo) == key && segkey(hi) == key) {
+      mn = fmin(mn, lo);
+      mx = fmax(mx, hi);
     } else {
-      // the same walk, cut into segments where the run from g changes
-      // binade (values read eight ahead)
-      const double *row = tile[t];
-      double mn = z.g, mx = z.g;
-      for (int j0 = 0; j0 < e; j0 += 8) {
-        double x8[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) x8[j] = j0 + j < e ? row[j0 + j] : 0.0;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          if (j0 + j >= e) break;
-          const double x = x8[j];
-          const double t0 = z.s0 + x;
-          if (segkey(t0) != z.key) {
-            z.lo = fmin(0.0, mn - z.g);
-            z.hi = fmax(0.0, mx - z.g);
-            seg_close(z, j0 + j, c, out, cnt, cap);
-            seg_open(z, j0 + j, 1, x, t0);
-            mn = mx = z.g;
-          } else {
-            const double t1 = z.s1 + x;
-            const double lo = t0 < t1 ? t0 : t1, hi = t0 < t1 ? t1 : t0;
-            mn = lo < mn ? lo : mn;
-            mx = hi > mx ? hi : mx;
-            z.s0 = t0;
-            z.s1 = t1;
-            if (segkey(t1) != z.key) z.bad = 1;
-          }
+      for (int j = 0; j < 8; j++) {
+        const int k = segkey(y[j]);
+        if (k != key) {
+          if (key >= 0) keep_binade(mn, mx, w);
+          key = k;
+          mn = mx = y[j];
+        } else {
+          mn = fmin(mn, y[j]);
+          mx = fmax(mx, y[j]);
         }
       }
-      z.lo = fmin(0.0, mn - z.g);
-      z.hi = fmax(0.0, mx - z.g);
     }
-    seg_close(z, e, c, out, cnt, cap);
-    if (cnt > cap) {
-      // too many binade changes: the whole chunk is summed in order (the
-      // record keeps the chunk's guess for the window's class table)
-      SegRec r;
-      r.g = gch;
-      r.d0 = r.d1 = r.lo = r.hi = r.xh = 0.0;
-      r.chunk = (int32_t)c;
-      r.meta = 0 | (e << 9) | (1 << 19);
-      out[0] = r;
-      cnt = 1;
-    }
-    segcnt[c] = cnt;
-    first[t] = out[0];
-    fcnt[t] = cnt;
   }
+  keep_binade(mn, mx, w);
+  w.S = S;
+}
+
+// Grid steps (mod 2) between two values of one binade: the mantissas' last
+// bits.
+__device__ __forceinline__ int parity_from(double S, double g) {
+  return (__double2loint(S) ^ __double2loint(g)) & 1;
+}
+
+// A chunk's record: its guess g, the translations from g and g + u, and the
+// open range of starts whose runs stay inside g's binade (with 4 ulps to
+// spare; empty if the run from g itself leaves it).
+struct ChunkRec {
+  double g, d0, d1, lo, hi;
+};
+
+// The walk over a chunk: by its translation if its record covers S, else
+// value by value.
+__device__ __forceinline__ void walk_chunk(const ChunkRec &r, const double *v, Walk &w) {
+  if (w.S > r.lo && w.S < r.hi) {
+    w.dlo = fmax(w.dlo, r.lo - w.S);
+    w.dhi = fmin(w.dhi, r.hi - w.S);
+    w.emax = max(w.emax, binade(r.g));
+    w.S = w.S + (parity_from(w.S, r.g) ? r.d1 : r.d0);
+  } else {
+    ordered_chunk(v, w);
+  }
+}
+
+// The walk over a folded window.
+__device__ __forceinline__ void walk_comp(const SeqComp &c, Walk &w) {
+  const int p = parity_from(w.S, c.g);
+  const double lo = p ? c.lo1 : c.lo0, hi = p ? c.hi1 : c.hi0;
+  w.ok = w.ok && w.S >= lo && w.S <= hi;
+  w.dlo = fmax(w.dlo, lo - w.S);
+  w.dhi = fmin(w.dhi, hi - w.S);
+  w.emax = max(w.emax, c.eb);
+  w.S = w.S + (p ? c.d1 : c.d0);
+}
+
+// The class of start S in a table from g: grid steps away from zero, the
+// difference of the mantissas.
+__device__ __forceinline__ int class_of(double S, double g, int M) {
+  const uint32_t dm = (uint32_t)__double2loint(S) - (uint32_t)__double2loint(g);
+  return (int)(dm & (uint32_t)(max(M, 1) - 1));
+}
+
+// The walk over an entry that has a table (M classes at cls).
+__device__ __forceinline__ void walk_classes(const SeqClass *cls, double g, int M, int emax,
+                                             Walk &w) {
+  w.ok = w.ok && M > 0 && segkey(w.S) == segkey(g);
+  const SeqClass c = cls[class_of(w.S, g, M)];
+  const double delta = w.S - c.s;  // exact: one binade
+  w.ok = w.ok && delta >= c.lo && delta <= c.hi;
+  w.dlo = fmax(w.dlo, c.lo - delta);
+  w.dhi = fmin(w.dhi, c.hi - delta);
+  w.emax = max(w.emax, emax);
+  w.S = c.e + delta;
+}
+__device__ __forceinline__ void walk_tab(const SeqTab &t, Walk &w) {
+  walk_classes(t.c, t.g, t.M, t.emax, w);
+}
+
+// The same from one start, every lane alike; false if the table does not
+// cover it.
+__device__ __forceinline__ bool take_tab(const SeqTab &t, double &S) {
+  Walk w;
+  w.S = S;
+  w.ok = true;
+  w.dlo = w.dhi = 0.0;
+  w.emax = 0;
+  walk_tab(t, w);
+  if (!__ballot(w.ok)) return false;
+  S = w.S;
+  return true;
+}
+
+// Lane c's class start of a table that begins at g: c grid steps away from
+// zero, so that every class has g's binade unless it is left at once.
+__device__ __forceinline__ Walk class_start(double g) {
+  const int l = lane_id(), eb = binade(g);
+  Walk w;
+  w.ok = binade_ok(eb);
+  const double u = w.ok ? pow2_field(eb - 52) : 0.0;
+  w.S = g + (double)(g < 0.0 ? -l : l) * u;  // exact: fewer than 2^6 ulps
+  w.ok = w.ok && segkey(w.S) == segkey(g);
+  w.dlo = -0x1p1000;
+  w.dhi = 0x1p1000;
+  w.emax = eb;
+  return w;
+}
+
+// The walks' results as the table of an entry; s0: the lane's start.
+__device__ __forceinline__ void put_tab(SeqTab &t, double g, double s0, const Walk &w) {
+  const int l = lane_id(), e0 = binade(g);
+  int em = w.ok ? w.emax : e0;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) em = max(em, __shfl_xor(em, o));
+  const int lgm = 1 + em - e0;
+  int M = lgm <= 6 ? 1 << lgm : 0;
+  if (__ballot(l < M && !w.ok)) M = 0;
+  if (l < M) t.c[l] = {s0, w.S, w.dlo, w.dhi};
+  if (l == 0) {
+    t.g = g;
+    t.M = M;
+    t.emax = em;
+  }
+}
+__device__ __forceinline__ void put_exact(SeqTab &t, double S) {
+  if (lane_id() == 0) {
+    t.g = 0.0;
+    t.M = -1;
+    t.emax = 0;
+    t.c[0].e = S;
+  }
+}
+
+// ---- chunk totals -------------------------------------------------------------
+// tot[c] and blk[sg]: the totals of each chunk and segment in any order,
+// for the guesses (a wavefront takes a chunk at a time, coalesced).
+__global__ void __launch_bounds__(256) seq_totals(const double *__restrict__ a, int64_t n,
+                                                  double *__restrict__ tot,
+                                                  double *__restrict__ blk) {
+  __shared__ double part[4];
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t c0 = (int64_t)blockIdx.x * 64 + wv * 16;
+  double v[16], s = 0.0;
+#pragma unroll
+  for (int j = 0; j < 16; j++) {
+    const int64_t gi = (c0 + j) * kChunk + l;
+    v[j] = gi < n ? a[gi] : 0.0;
+  }
+#pragma unroll
+  for (int j = 0; j < 16; j++) {
+    const double t = wave_sum(v[j]);
+    s += t;
+    if (l == 0 && (c0 + j) * kChunk < n) tot[c0 + j] = t;
+  }
+  if (l == 0) part[wv] = s;
   __syncthreads();
-  // composites: the 16 lanes of DPP row w fold window w of the block, lane
-  // i taking member i: start parities by a row scan of the members' maps,
-  // translations by row scans (exact sums), intervals by row max/min
-  const int wl = t / kWin, i = t % kWin;
+  if (threadIdx.x == 0) blk[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+}
+
+// blk[k] <- the total of the segments before k (one workgroup; for sums of
+// so many segments that each segment's own loop over them would dominate)
+__global__ void __launch_bounds__(1024) seq_prefix(double *blk, int64_t nb) {
+  __shared__ double part[1024];
+  const int t = threadIdx.x;
+  const int64_t per = (nb + 1023) / 1024, b = min(nb, per * t), e = min(nb, per * (t + 1));
+  double s = 0.0;
+  for (int64_t k = b; k < e; k++) s += blk[k];
+  part[t] = s;
+  __syncthreads();
+  for (int o = 1; o < 1024; o <<= 1) {
+    const double p = t >= o ? part[t - o] : 0.0;
+    __syncthreads();
+    part[t] += p;
+    __syncthreads();
+  }
+  s = t > 0 ? part[t - 1] : 0.0;
+  for (int64_t k = b; k < e; k++) {
+    const double v = blk[k];
+    blk[k] = s;
+    s += v;
+  }
+}
+
+// ---- segments -------------------------------------------------------------------
+// ONE: the sum is this one segment; its exact value goes to dout.
+// The total before the segment comes from the chunk totals, or with blk from
+// the prefix of the segments' totals.
+// Wave 0 makes the chunks' records and folds the windows; wave k the table of
+// window k if that did not fold.
+template <bool ONE>
+__global__ void __launch_bounds__(64 * kWins) seq_segments(const double *__restrict__ a, int64_t n,
+                                                   const double *__restrict__ tot,
+                                                   const double *__restrict__ blk,
+                                                   SeqComp *__restrict__ comps,
+                                                   SeqTab *__restrict__ tabs, double *dout) {
+  __shared__ double tile[64][kChunk + 1];
+  __shared__ ChunkRec rec[64];
+  __shared__ SeqComp comp[kWins];
+  __shared__ SeqTab wtab[kWins];
+  __shared__ double before[kWins];
+  const int t = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t sg = blockIdx.x, c0 = sg * 64, c = c0 + t, nch = (n + kChunk - 1) / kChunk;
+  {
+    constexpr int PER = kSegVals / (64 * kWins);
+    double v[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int64_t gi = sg * kSegVals + (j * kWins + wv) * 64 + t;
+      v[j] = gi < n ? a[gi] : 0.0;
+    }
+    if (!ONE) {
+      double s = 0.0;
+      if (blk) {
+        if (threadIdx.x == 0) s = blk[sg];
+      } else {
+        // sixteen totals a thread in flight
+        for (int64_t k = threadIdx.x; k < c0; k += 16 * 64 * kWins) {
+          double q[16];
+#pragma unroll
+          for (int j = 0; j < 16; j++) {
+            const int64_t kj = k + j * 64 * kWins;
+            q[j] = kj < c0 ? tot[kj] : 0.0;
+          }
+#pragma unroll
+          for (int j = 0; j < 16; j++) s += q[j];
+        }
+      }
+      s = wave_sum(s);
+      if (t == 0) before[wv] = s;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) tile[j * kWins + wv][t] = v[j];
+  }
+  const int nwin = (int)min((int64_t)kWins, (nch - c0 + kWin - 1) / kWin);
+  double tc = !ONE && wv == 0 && c < nch ? tot[c] : 0.0;
+  __syncthreads();
+  if (wv == 0) {
+  double off = 0.0;  // the total before this segment
+  if (ONE) {
+    const double *row = tile[t];
+#pragma unroll 16
+    for (int j = 0; j < kChunk; j++) tc += row[j];
+  } else {
+#pragma unroll
+    for (int k = 0; k < kWins; k++) off += before[k];
+  }
+  // guess of the chunk's start, and of the one after it
+  const double gnext = off + wave_incl_add(tc);
+  double g = __shfl_up(gnext, 1);
+  if (t == 0) g = off;
+  // the runs from g and g + u, branch-free: the rounded partial sums bound
+  // the exact ones within half an ulp, and in one binade the second run
+  // stays 0 to 2 u above the first
+  const int eb = binade(g), key = segkey(g);
+  const bool eb_ok = binade_ok(eb);
+  const double u = eb_ok ? pow2_field(eb - 52) : 0.0, ui = eb_ok ? pow2_field(2098 - eb) : 0.0;
+  double f0 = g, f1 = g + u, mn = g, mx = g;
+  bool in = eb_ok && segkey(f1) == key;
+  const double *row = tile[t];
+#pragma unroll
+  for (int j0 = 0; j0 < kChunk; j0 += 8) {
+    double x[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] = row[j0 + j];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      f0 = f0 + x[j];
+      f1 = f1 + x[j];
+      mn = fmin(mn, f0);
+      mx = fmax(mx, f0);
+    }
+  }
+  mx = mx + 2.0 * u;
+  // extremes in g's binade: then so is every partial sum
+  in = in && segkey(mn) == key && segkey(mx) == key && segkey(f1) == key;
+  const double d0 = f0 - g, d1 = f1 - (g + u), rlo0 = mn - g, rhi0 = mx - g;
+  const bool rok = in && run_inside(g, eb, rlo0, rhi0);
+  {
+    const double bl = eb_ok ? pow2_field(eb) : 0.0, m4 = 4.0 * u, bh = 2.0 * bl;
+    ChunkRec R;
+    R.g = g;
+    R.d0 = d0;
+    R.d1 = d1;
+    R.lo = !rok ? 1.0 : (g > 0.0 ? bl + m4 : m4 - bh) - rlo0;
+    R.hi = !rok ? 0.0 : (g > 0.0 ? bh - m4 : -bl - m4) - rhi0;
+    rec[t] = R;
+  }
+  // windows: the 16 lanes of DPP row w fold window w, lane i taking member
+  // i: start parities by a row scan of the members' maps, translations by
+  // row scans (exact sums), intervals by row max/min
+  const int wl = t / kWin, rl = t & 15;
   const int64_t w0 = c0 + (int64_t)wl * kWin;
   const int nm = w0 < nch ? (int)min((int64_t)kWin, nch - w0) : 0;
-  const bool mem = i < nm;
-  const int fc = mem ? fcnt[t] : 1;
-  const bool single = __ballot(!(fc == 1)) >> (wl * kWin) & 0xffff ? false : true;
-  uint64_t cn = mem ? (uint64_t)fc << (4 * i) : 0;
-#pragma unroll
-  for (int m = 1; m < kWin; m <<= 1) cn |= __shfl_xor(cn, m);
-  const SegRec A = first[wl * kWin];
-  const SegRec Ri = first[t];
-  const int key = segkey(A.g), eb = binade(A.g);
-  const bool ok0 = !((A.meta >> 18) & 3) && eb >= 64 && eb <= 2045;
-  const double ui = ok0 ? pow2_field(2098 - eb) : 0.0;
-  const double sig = A.g < 0.0 ? -1.0 : 1.0;
-  const double G1 = ok0 ? (fabs(A.g) - pow2_field(eb)) * ui : 0.0;
-  bool okm = true;
+  const bool mem = rl < nm;
+  const int src0 = wl * kWin;
+  const double gA = __shfl(g, src0);
+  const int kA = __shfl(key, src0);
+  const double sig = gA < 0.0 ? -1.0 : 1.0;
+  bool fold = mem ? rok && key == kA : true;
   int mapm = 2;  // identity
   double d0m = 0.0, d1m = 0.0, Li = -0x1p60, Ui = 0x1p60;
-  if (mem && single && ok0) {
-    okm = (i == 0 || (((Ri.meta >> 18) & 3) == 0 && segkey(Ri.g) == key)) &&
-          run_inside(Ri.g, eb, Ri.lo, Ri.hi);
-    const double rlo = sig > 0.0 ? Ri.lo : -Ri.hi;
-    const double rhi = sig > 0.0 ? Ri.hi : -Ri.lo;
+  if (mem && fold) {
+    const double rlo = sig > 0.0 ? rlo0 : -rhi0, rhi = sig > 0.0 ? rhi0 : -rlo0;
     Li = ceil(5.0 - rlo * ui) + 1.0;
     Ui = floor(0x1p52 - 5.0 - rhi * ui) - 1.0;
-    const bool last = i + 1 == nm;
-    const bool has_next = w0 + nm < nch;
-    const double gn = !last ? first[t + 1].g : ((wl + 1) * kWin < 64 ? first[(wl + 1) * kWin].g : gnx);
-    const int am = (!last || has_next) ? parity_of((Ri.g + Ri.d0) - gn, ui) : 0;
-    const int bm = parity_of(Ri.d1 - Ri.d0, ui);
+    // parity towards the next member (a run that leaves the binade there
+    // does not fold)
+    const int am = rl + 1 < nm ? parity_of((g + d0) - gnext, ui) : 0;
+    const int bm = parity_of(d1 - d0, ui);
     mapm = ((bm ? 0 : 1) << 1) | am;  // p -> bm ? am : p ^ am
-    d0m = Ri.d0;
-    d1m = Ri.d1;
+    d0m = d0;
+    d1m = d1;
   }
-  // start parity of member i for window start parity 0 and 1
-  const int rl = t & 15;
   const int incl = row_incl_map(mapm);
   int ex = dpp_i<0x111>(incl);
   if (rl == 0) ex = 2;
-  const int pa = (ex >> 1) ? (0 ^ (ex & 1)) : (ex & 1);
-  const int pb = (ex >> 1) ? (1 ^ (ex & 1)) : (ex & 1);
-  const double da = mem ? (pa ? d1m : d0m) : 0.0, db = mem ? (pb ? d1m : d0m) : 0.0;
-  const double ia = row_incl_add(da), ib = row_incl_add(db);
+  const int pa = ex & 1, pb = (ex >> 1) ? (1 ^ (ex & 1)) : (ex & 1);
+  const double ia = row_incl_add(mem ? (pa ? d1m : d0m) : 0.0);
+  const double ib = row_incl_add(mem ? (pb ? d1m : d0m) : 0.0);
   double xa = dpp_d<0x111>(ia), xb = dpp_d<0x111>(ib);
   if (rl == 0) xa = xb = 0.0;
   // admissible start offsets: member i's start is G1 + delta + sig D / u
   double lo0 = -0x1p60, hi0 = 0x1p60, lo1 = -0x1p60, hi1 = 0x1p60;
-  if (mem && single && ok0) {
+  if (mem && fold) {
+    const double G1 = (fabs(gA) - pow2_field(eb)) * ui;
     const double Oa = sig * xa * ui, Ob = sig * xb * ui;
     lo0 = Li - G1 - Oa;
     hi0 = Ui - G1 - Oa;
     lo1 = Li - G1 - Ob;
     hi1 = Ui - G1 - Ob;
     // partial translations stay well inside 2^53 u, so every sum is exact
-    if (fabs(ia) * ui > 0x1p51 || fabs(ib) * ui > 0x1p51) okm = false;
+    if (fabs(ia) * ui > 0x1p51 || fabs(ib) * ui > 0x1p51) fold = false;
   }
 #pragma unroll
   for (int m = 1; m < kWin; m <<= 1) {
@@ -480,569 +562,364 @@ __global__ void __launch_bounds__(64) seq_chunks(const double *__restrict__ a, i
     lo1 = fmax(lo1, __shfl_xor(lo1, m));
     hi1 = fmin(hi1, __shfl_xor(hi1, m));
   }
-  const bool ok = single && ok0 && ((__ballot(!okm) >> (wl * kWin)) & 0xffff) == 0;
-  // totals and the whole window's map sit in member nm - 1's lane
-  const int src = wl * kWin + (nm > 0 ? nm - 1 : 0);
-  const double Da = __shfl(ia, src), Db = __shfl(ib, src);
-  const int mw = __shfl(incl, src);
-  if (i == 0 && nm > 0) {
-    CompRec C;
-    if (single) {
-      const int pn0 = (mw >> 1) ? (0 ^ (mw & 1)) : (mw & 1);
-      const int pn1 = (mw >> 1) ? (1 ^ (mw & 1)) : (mw & 1);
-      C.g = A.g;
-      C.d0 = Da;
-      C.d1 = Db;
-      C.lo0 = lo0;
-      C.hi0 = hi0;
-      C.lo1 = lo1;
-      C.hi1 = hi1;
-      C.meta = nm | ((ok ? 1 : 0) << 5) | ((((pn0 ^ pn1) << 1) | pn0) << 6);
-    } else {
-      C.g = C.d0 = C.d1 = C.lo0 = C.hi0 = C.lo1 = C.hi1 = 0.0;
-      C.meta = nm;
-    }
-    C.win = (int32_t)(w0 / kWin);
-    C.cnts = cn;
-    cps[w0 / kWin] = C;
+  const uint64_t foldm = __ballot(fold);
+  const int last = src0 + (nm > 0 ? nm - 1 : 0);  // its lane holds the totals
+  const double Da = __shfl(ia, last), Db = __shfl(ib, last);
+  if (rl == 0) {
+    SeqComp C;
+    C.g = gA;
+    C.d0 = Da;
+    C.d1 = Db;
+    // from grid steps towards larger magnitude to starts (the steps' margins
+    // cover the roundings here)
+    C.lo0 = gA + (sig > 0.0 ? lo0 : -hi0) * u;
+    C.hi0 = gA + (sig > 0.0 ? hi0 : -lo0) * u;
+    C.lo1 = gA + (sig > 0.0 ? lo1 : -hi1) * u;
+    C.hi1 = gA + (sig > 0.0 ? hi1 : -lo1) * u;
+    C.ok = nm > 0 && ((foldm >> src0) & 0xffff) == 0xffff;
+    C.eb = eb;
+    comp[wl] = C;
+    if (!ONE) comps[sg * kWins + wl] = C;
   }
-}
-
-// Exact sequential sum of a[b, e) (e - b <= 2 * 64) starting from S: the
-// wavefront loads the values, then adds them in order (the values reach
-// the adder through readlane, so the chain is one dependent add per value).
-__device__ double lane_seq(const double *__restrict__ a, int64_t b, int64_t e, double S) {
-  const int l = lane_id();
-  const int cnt = (int)(e - b);
-  const double x0 = l < cnt ? a[b + l] : 0.0;
-  const double x1 = 64 + l < cnt ? a[b + 64 + l] : 0.0;
-  const int c0 = cnt < 64 ? cnt : 64;
-  for (int i = 0; i < c0; i++) S = S + readlane_d(x0, i);
-  for (int i = 64; i < cnt; i++) S = S + readlane_d(x1, i - 64);
-  return S;
-}
-
-// The member chain over up to 64 compacted records (one per lane).  Runs
-// of at most kWalk records are walked one record at a time (a handful of
-// dependent operations each); longer runs take the wavefront scans.
-static constexpr int kWalk = 4;
-
-__device__ void chain_group(const double *__restrict__ a, const SegRec &R, int nv, double &S) {
-  const int l = lane_id();
-  const bool valid = l < nv;
-  const int head = valid ? (R.meta >> 18) & 1 : 0;
-  const int rep = valid ? (R.meta >> 19) & 1 : 0;
-  const int key = segkey(R.g);
-  const double gn = dpp_d<0x130>(R.g);  // next lane's guess (wave_shl:1)
-  // Everything that depends on the lane's own record only, computed once:
-  // 1/u = 2^(52 - E) of its binade (exact; used only while in range), its
-  // parity map p -> b ? a : p ^ a towards the next lane (used only when the
-  // next lane continues the run, hence shares the binade), and whether the
-  // guessed run itself keeps the margins.
-  const int eb = binade(R.g);
-  const bool eb_ok = eb >= 2 && eb <= 2045;
-  const double ui = eb_ok ? pow2_field(2098 - eb) : 0.0;
-  const int map_own = ((parity_of(R.d1 - R.d0, ui) ? 0 : 1) << 1) |
-                      parity_of((R.g + R.d0) - gn, ui);
-  const bool g_inside = eb_ok && run_inside(R.g, eb, R.lo, R.hi);
-  int q = 0;
-  while (q < nv) {
-    const int meta_q = __builtin_amdgcn_readlane(R.meta, q);
-    const int64_t chunk_q = (int64_t)__builtin_amdgcn_readlane(R.chunk, q);
-    if ((meta_q >> 19) & 1) {
-      const int64_t b = chunk_q * kChunk + (meta_q & 511);
-      const int64_t e = chunk_q * kChunk + ((meta_q >> 9) & 511);
-      S = lane_seq(a, b, e, S);
-      q++;
-      continue;
-    }
-    if ((meta_q >> 18) & 1) S = S + readlane_d(R.xh, q);
-    const int key_q = __builtin_amdgcn_readlane(key, q);
-    // the run: lanes q .. h-1 without a head, replay or binade change
-    const uint64_t stop = __ballot(valid && l > q && (head || rep || key != key_q));
-    const int h = stop ? __ffsll((unsigned long long)stop) - 1 : nv;
-    if (h - q <= kWalk) {
-      // a short run (the records between binade crossings): each record is
-      // checked and translated on its own, S being exact at its start
-      for (int r = q; r < h; r++) {
-        const double g_r = readlane_d(R.g, r), d0_r = readlane_d(R.d0, r);
-        const double d1_r = readlane_d(R.d1, r), lo_r = readlane_d(R.lo, r);
-        const double hi_r = readlane_d(R.hi, r), ui_r = readlane_d(ui, r);
-        const int gin_r = __builtin_amdgcn_readlane((int)g_inside, r);
-        if (gin_r && segkey(S) == key_q && run_inside(S, binade(g_r), lo_r, hi_r)) {
-          S = S + (parity_of(S - g_r, ui_r) ? d1_r : d0_r);
-        } else {
-          const int64_t chunk_r = (int64_t)__builtin_amdgcn_readlane(R.chunk, r);
-          const int meta_r = __builtin_amdgcn_readlane(R.meta, r);
-          const int64_t b = chunk_r * kChunk + (meta_r & 511) + ((meta_r >> 18) & 1);
-          const int64_t e = chunk_r * kChunk + ((meta_r >> 9) & 511);
-          S = lane_seq(a, b, e, S);
-        }
+  }
+  __syncthreads();
+  if (ONE || sg == 0) {
+    if (wv != 0) return;
+    // the first segment starts at exactly +0: every lane walks it
+    Walk w;
+    w.S = 0.0;
+    w.dlo = -0x1p1000;
+    w.dhi = 0x1p1000;
+    w.emax = 0;
+    for (int k = 0; k < nwin; k++) {
+      Walk z = w;
+      z.ok = comp[k].ok;
+      if (z.ok) walk_comp(comp[k], z);
+      if (z.ok) {
+        w = z;
+        continue;
       }
-      q = h;
-      continue;
+      const int m = (int)min((int64_t)kWin, nch - c0 - k * kWin);
+      for (int i = k * kWin; i < k * kWin + m; i++)
+        walk_chunk(rec[i], tile[i], w);
     }
-    const bool in = l >= q && l < h;
-    const double g_q = readlane_d(R.g, q);
-    const double ui_q = readlane_d(ui, q);
-    // start parities: p_(l+1) = b_l ? a_l : p_l ^ a_l, a GF(2) affine scan
-    const int mp = (in && l + 1 < h) ? map_own : 2;  // 2: identity
-    const int incl_m = wave_incl_map(mp);
-    int ex_m = dpp_i<0x138>(incl_m);
-    if (l == 0) ex_m = 2;
-    // maps of lanes < q are identities, so each prefix starts at lane q
-    const int p_q = segkey(S) == key_q ? parity_of(S - g_q, ui_q) : 0;
-    const int p = (ex_m >> 1) ? (p_q ^ (ex_m & 1)) : (ex_m & 1);
-    const double d = in ? (p ? R.d1 : R.d0) : 0.0;
-    // lanes < q add zeros, so lane l's exclusive partial covers [q, l)
-    const double excl = wave_prev_d(wave_incl_add(d));
-    const double Sl = S + excl;
-    bool acc = false;
-    if (in) {
-      acc = g_inside && segkey(Sl) == key && run_inside(Sl, eb, R.lo, R.hi) &&
-            parity_of(Sl - R.g, ui) == p;
+    if (ONE) {
+      if (t == 0) *dout = w.S;
+    } else {
+      put_exact(tabs[0], w.S);
     }
-    const uint64_t rej = __ballot(in && !acc);
-    if (rej == 0) {
-      S = readlane_d(Sl + d, h - 1);
-      q = h;
-      continue;
-    }
-    const int f = __ffsll((unsigned long long)rej) - 1;
-    const double Sf = readlane_d(Sl, f);
-    const int64_t chunk_f = (int64_t)__builtin_amdgcn_readlane(R.chunk, f);
-    const int meta_f = __builtin_amdgcn_readlane(R.meta, f);
-    const int64_t b = chunk_f * kChunk + (meta_f & 511) + ((meta_f >> 18) & 1);
-    const int64_t e = chunk_f * kChunk + ((meta_f >> 9) & 511);
-    S = lane_seq(a, b, e, Sf);
-    q = f + 1;
-  }
-}
-
-// Records of window win (chunks kWin win .. + nm, counts packed in cnts),
-// one per lane in order, summed by the member chain from S.
-__device__ void member_level(const double *__restrict__ a, const SegRec *__restrict__ sg, int cap,
-                             int64_t win, int nm, uint64_t cnts, double &S) {
-  const int l = lane_id();
-  const int64_t c0 = win * kWin;
-  // lane r takes record r: chunk i with off_i <= r < off_i + cnt_i
-  int ch = 0, k = l, tot = 0;
-  for (int i = 0; i < nm; i++) {
-    if (l >= tot) {
-      ch = i;
-      k = l - tot;
-    }
-    tot += (cnts >> (4 * i)) & 15;
-  }
-  SegRec R;
-  if (l < tot) {
-    R = sg[(c0 + ch) * cap + k];
-  } else {
-    R.meta = 0, R.g = 0.0, R.d0 = R.d1 = R.lo = R.hi = R.xh = 0.0, R.chunk = 0;
-  }
-  chain_group(a, R, tot, S);
-}
-
-// ---- class tables of the windows that did not fold -------------------------
-// A window whose guessed run crosses binades (heads) is a translation only
-// per residue class of the start: for a start S = G_c + Delta, G_c = g + c u
-// (g the window's first guess, u the grid of g's binade, c < M) and Delta a
-// multiple of M u = 2 u_max (u_max the coarsest grid the run visits), every
-// rounding of the run from S happens on the grid it happens on from G_c,
-// displaced by Delta, as long as every partial sum stays in its binade:
-// the run then ends exactly at E_c + Delta.  seq_classes walks the window's
-// records from the 32 starts G_0..G_31 (one lane each, heads added, rejected
-// records summed in order), intersecting the admissible Delta interval over
-// every step (4-ulp margins, as run_inside).  The chain then resolves such a
-// window with one lookup: c from the low mantissa bits of S - g, Delta =
-// S - G_c, a range check, S = E_c + Delta; a start outside its interval, or
-// a window whose run climbs more than 4 binades (M > 32), takes the member
-// chain.
-static constexpr int kClasses = 32;
-
-struct ClassTab {
-  double e[kClasses], gs[kClasses], lo[kClasses], hi[kClasses];
-};
-
-// Delta keeps y + Delta in y's binade (margins of 4 ulps); a power of two or
-// a value outside the normal range admits Delta = 0 only.
-__device__ __forceinline__ void keep_binade(double y, double &dlo, double &dhi, int &emax) {
-  const uint64_t bits = (uint64_t)__double_as_longlong(y);
-  const int eb = (int)((bits >> 52) & 0x7ff);
-  if (eb < 64 || eb > 2045 || (bits & 0xfffffffffffffull) == 0) {
-    dlo = fmax(dlo, 0.0);
-    dhi = fmin(dhi, 0.0);
-    emax = max(emax, eb);
     return;
   }
-  const double bl = pow2_field(eb), bh = pow2_field(eb + 1), m = pow2_field(eb - 50);
-  const double L = y > 0.0 ? bl + m : -bh + m, U = y > 0.0 ? bh - m : -bl - m;
-  dlo = fmax(dlo, L - y);
-  dhi = fmin(dhi, U - y);
-  emax = max(emax, eb);
+  if (wv < nwin && !comp[wv].ok) {
+    const double gk = rec[wv * kWin].g;
+    Walk w = class_start(gk);
+    const double s0 = w.S;
+    const int m = (int)min((int64_t)kWin, nch - c0 - wv * kWin);
+    for (int i = wv * kWin; i < wv * kWin + m && __ballot(w.ok); i++)
+      walk_chunk(rec[i], tile[i], w);
+    put_tab(wtab[wv], gk, s0, w);
+  }
+  __syncthreads();
+  if (wv != 0) return;
+  // the segment's table
+  const double gs = rec[0].g;
+  Walk w = class_start(gs);
+  const double s0 = w.S;
+  for (int k = 0; k < nwin; k++) {
+    if (comp[k].ok) walk_comp(comp[k], w);
+    else walk_tab(wtab[k], w);
+  }
+  put_tab(tabs[sg], gs, s0, w);
 }
 
-// The values a[b, e) added in order to S, with the binade constraints.
-__device__ __forceinline__ double ordered_steps(const double *__restrict__ a, int64_t b, int64_t e,
-                                               double S, double &dlo, double &dhi, int &emax) {
-  for (int64_t i = b; i < e; i++) {
-    S = S + a[i];
-    keep_binade(S, dlo, dhi, emax);
+// Sixteen entries of a level to one of the next: a wavefront per entry.
+__global__ void __launch_bounds__(64) seq_fold(const SeqTab *__restrict__ in, int64_t nin,
+                                               SeqTab *__restrict__ out) {
+  __shared__ SeqTab t[kFold];
+  const int l = threadIdx.x;
+  const int64_t i0 = (int64_t)blockIdx.x * kFold;
+  const int m = (int)min((int64_t)kFold, nin - i0);
+  // every class of every entry in flight at once (those beyond an entry's M
+  // are not used)
+  SeqClass c[kFold];
+#pragma unroll
+  for (int k = 0; k < kFold; k++) c[k] = in[i0 + min(k, m - 1)].c[l];
+  if (l < m) {
+    t[l].g = in[i0 + l].g;
+    t[l].M = in[i0 + l].M;
+    t[l].emax = in[i0 + l].emax;
+  }
+#pragma unroll
+  for (int k = 0; k < kFold; k++)
+    if (k < m) t[k].c[l] = c[k];
+  __syncthreads();
+  const bool first = blockIdx.x == 0;  // starts at the sum's beginning
+  Walk w = class_start(t[0].g);
+  if (first) {
+    w.S = t[0].c[0].e;
+    w.ok = true;
+  }
+  const double s0 = w.S;
+  for (int k = first ? 1 : 0; k < m; k++) walk_tab(t[k], w);
+  if (first && w.ok) put_exact(out[0], w.S);
+  else if (first) {
+    if (l == 0) out[0].M = 0;
+  } else {
+    put_tab(out[blockIdx.x], t[0].g, s0, w);
+  }
+}
+
+// ---- the chain --------------------------------------------------------------------
+struct SeqLevels {
+  const SeqTab *tab[kMaxLevels];
+  int64_t n[kMaxLevels];
+  int top;  // the level that the chain takes
+};
+
+// Orders the calling wavefront's LDS accesses.
+__device__ __forceinline__ void seq_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Window k of segment sg from S: folded, or its values added in order
+// (staged through LDS, a dependent add of 4.3 ns each).
+__device__ double resolve_window(const double *__restrict__ a, int64_t n, int64_t win,
+                                 const SeqComp *__restrict__ comps, double S, double *lds) {
+  const int l = lane_id();
+  const SeqComp C = comps[win];
+  const int p = parity_from(S, C.g);
+  if (__ballot(C.ok && S >= (p ? C.lo1 : C.lo0) && S <= (p ? C.hi1 : C.hi0)))
+    return S + (p ? C.d1 : C.d0);
+  const int64_t b = win * (int64_t)(kWin * kChunk);
+  seq_wave_sync();
+  for (int j = l; j < kWin * kChunk; j += 64) lds[j] = b + j < n ? a[b + j] : 0.0;
+  seq_wave_sync();
+  for (int j0 = 0; j0 < kWin * kChunk; j0 += 16) {
+    double x[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) x[j] = lds[j0 + j];
+#pragma unroll
+    for (int j = 0; j < 16; j++) S = S + x[j];
   }
   return S;
 }
 
-__global__ void __launch_bounds__(64) seq_classes(const double *__restrict__ a,
-                                                  const SegRec *__restrict__ sg, int cap,
-                                                  CompRec *__restrict__ cp, int64_t nw,
-                                                  int32_t *__restrict__ tab_m,
-                                                  ClassTab *__restrict__ tab) {
-  const int64_t w = blockIdx.x;
-  const CompRec C = cp[w];
-  if ((C.meta >> 5) & 1) return;  // folded: no table needed
-  const int l = threadIdx.x, nm = C.meta & 31;
-  const int64_t c0 = w * kWin;
-  // lane r holds record r of the window (as the member chain)
-  int ch = 0, k = l, tot = 0;
-  for (int i = 0; i < nm; i++) {
-    if (l >= tot) {
-      ch = i;
-      k = l - tot;
-    }
-    tot += (C.cnts >> (4 * i)) & 15;
-  }
-  SegRec R;
-  if (l < tot) {
-    R = sg[(c0 + ch) * cap + k];
-  } else {
-    R.meta = 0, R.g = 0.0, R.d0 = R.d1 = R.lo = R.hi = R.xh = 0.0, R.chunk = 0;
-  }
-  const double g = readlane_d(R.g, 0);
-  const int e0 = binade(g);
-  // (a replay record carries its chunk's guess, so a table can start there)
-  bool ok = tot > 0 && e0 >= 64 && e0 <= 2045;
-  const double u = ok ? pow2_field(e0) * 0x1p-52 : 0.0;
-  const int c = l < kClasses ? l : 0;
-  double S = g + (double)c * u;  // exact: c < 2^5 ulps
-  ok = ok && segkey(S) == segkey(g);
-  double dlo = -0x1p1000, dhi = 0x1p1000;
-  int emax = e0;
-  // per-record quantities that do not depend on the start
-  const int ebr = binade(R.g);
-  const bool ebr_ok = ebr >= 2 && ebr <= 2045;
-  const double uir = ebr_ok ? pow2_field(2098 - ebr) : 0.0;
-  const bool gin = ebr_ok && run_inside(R.g, ebr, R.lo, R.hi);
-  for (int r = 0; r < tot && __ballot(ok); r++) {
-    const int meta = __builtin_amdgcn_readlane(R.meta, r);
-    const int64_t base = (int64_t)__builtin_amdgcn_readlane(R.chunk, r) * kChunk;
-    const int64_t b = base + (meta & 511), e = base + ((meta >> 9) & 511);
-    if ((meta >> 19) & 1) {
-      S = ordered_steps(a, b, e, S, dlo, dhi, emax);
+// Entry i of level lev from S, by its table or by its parts.
+__device__ double resolve(const double *__restrict__ a, int64_t n, const SeqLevels &L, int lev,
+                          int64_t i, const SeqComp *__restrict__ comps, double S, double *lds) {
+  // the entries still to take, a depth-first descent: at most kFold - 1
+  // siblings a level
+  int64_t at[kMaxLevels], end[kMaxLevels];
+  at[lev] = i;
+  end[lev] = i + 1;
+  int k = lev;
+  for (;;) {
+    while (k <= lev && at[k] >= end[k]) k++;
+    if (k > lev) return S;
+    const int64_t j = at[k]++;
+    const SeqTab &t = L.tab[k][j];
+    const int M = t.M;
+    if (M < 0) {
+      S = t.c[0].e;
       continue;
     }
-    const int head = (meta >> 18) & 1;
-    if (head) {
-      S = S + readlane_d(R.xh, r);
-      keep_binade(S, dlo, dhi, emax);
+    if (M > 0 && take_tab(t, S)) continue;
+    if (k > 0) {
+      k--;
+      at[k] = j * kFold;
+      end[k] = min(L.n[k], (j + 1) * kFold);
+      continue;
     }
-    const double gr = readlane_d(R.g, r), lor = readlane_d(R.lo, r), hir = readlane_d(R.hi, r);
-    const int eb = binade(gr);
-    if (__builtin_amdgcn_readlane((int)gin, r) && segkey(S) == segkey(gr) &&
-        run_inside(S, eb, lor, hir)) {
-      // the record's run from S + Delta is its run from S displaced: the
-      // range of run_inside, relative to S
-      const double bl = pow2_field(eb), bh = pow2_field(eb + 1), m = 4.0 * bl * 0x1p-52;
-      const double rlo = S < 0.0 ? -hir : lor, rhi = S < 0.0 ? -lor : hir;
-      const double ax = fabs(S);
-      const double alo = (bl + m - rlo) - ax, ahi = (bh - m - rhi) - ax;  // on |S|
-      dlo = fmax(dlo, S < 0.0 ? -ahi : alo);
-      dhi = fmin(dhi, S < 0.0 ? -alo : ahi);
-      emax = max(emax, eb);
-      const int p = parity_of(S - gr, readlane_d(uir, r));
-      S = S + (p ? readlane_d(R.d1, r) : readlane_d(R.d0, r));
-    } else {
-      S = ordered_steps(a, b + head, e, S, dlo, dhi, emax);
-    }
+    const int64_t nwin = (n + kWin * kChunk - 1) / (kWin * kChunk);
+    for (int64_t wn = j * kWins; wn < min(nwin, (j + 1) * kWins); wn++)
+      S = resolve_window(a, n, wn, comps, S, lds);
   }
-  // M u = 2 u_max over every lane's run
-  int em = emax;
+}
+
+// The top level's entries in order.  Each of the workgroup's wavefronts folds
+// its kGroup or fewer consecutive entries into one table (their classes
+// brought into LDS first if they fit its share); wavefront 0 takes the
+// sixteen tables.  A start that a table does not cover descends to the
+// group's entries.
+static constexpr int kShare = 192;  // classes in LDS per wavefront
+struct ChainLds {
+  SeqTab group[kChainWaves];
+  SeqClass cls[kChainWaves][kShare];
+  double vals[kWin * kChunk];
+};
+__global__ void __launch_bounds__(64 * kChainWaves) seq_chain(const double *__restrict__ a,
+                                                              int64_t n, SeqLevels L,
+                                                              const SeqComp *__restrict__ comps,
+                                                              double *dout) {
+  extern __shared__ __align__(16) unsigned char chain_raw[];
+  ChainLds &C = *(ChainLds *)chain_raw;
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, m = (int)L.n[L.top];
+  const SeqTab *tab = L.tab[L.top];
+  const int per = (m + kChainWaves - 1) / kChainWaves, k0 = wv * per, ke = min(m, k0 + per);
+  if (k0 < m) {
+    // lane i: the head of entry k0 + i
+    const bool have = l < ke - k0;
+    const int Mi = have ? tab[k0 + l].M : 0, ei = have ? tab[k0 + l].emax : 0;
+    const double gi = have ? tab[k0 + l].g : 0.0;
+    const int cnt = abs(Mi);
+    int incl = cnt;
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) em = max(em, __shfl_xor(em, o));
-  const int lgm = 1 + em - e0;
-  const int M = (lgm >= 1 && lgm <= 5) ? (1 << lgm) : 0;
-  const bool all_ok = __ballot(l < M && !ok) == 0;
-  if (l < kClasses) {
-    tab[w].e[l] = S;
-    tab[w].gs[l] = g + (double)c * u;
-    tab[w].lo[l] = dlo;
-    tab[w].hi[l] = dhi;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(incl, o);
+      if (l >= o) incl += u;
+    }
+    const int first = incl - cnt;
+    const bool fits = __shfl(incl, 63) <= kShare;
+    if (fits) {
+      SeqClass c[kGroup];
+#pragma unroll
+      for (int j = 0; j < kGroup; j++)
+        if (l < __builtin_amdgcn_readlane(cnt, j)) c[j] = tab[k0 + j].c[l];
+#pragma unroll
+      for (int j = 0; j < kGroup; j++)
+        if (l < __builtin_amdgcn_readlane(cnt, j))
+          C.cls[wv][__builtin_amdgcn_readlane(first, j) + l] = c[j];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    const double g0 = readlane_f64(gi, 0);
+    Walk w = class_start(g0);
+    if (k0 == 0) {  // the sum's beginning: one exact start
+      w.S = tab[0].c[0].e;
+      w.ok = __builtin_amdgcn_readlane(Mi, 0) < 0;
+    }
+    const double s0 = w.S;
+    for (int j = k0 == 0 ? 1 : 0; j < ke - k0; j++) {
+      const int M = __builtin_amdgcn_readlane(Mi, j), em = __builtin_amdgcn_readlane(ei, j);
+      const double g = readlane_f64(gi, j);
+      if (fits) walk_classes(C.cls[wv] + __builtin_amdgcn_readlane(first, j), g, M, em, w);
+      else walk_classes(tab[k0 + j].c, g, M, em, w);
+    }
+    if (k0 > 0) put_tab(C.group[wv], g0, s0, w);
+    else if (w.ok) put_exact(C.group[0], w.S);
+    else if (l == 0) C.group[0].M = 0;
   }
-  const bool valid = M > 0 && all_ok && __ballot(ok) != 0;
-  if (l == 0) tab_m[w] = valid ? M : 0;
-  // Two classes whose runs end in g's binade: the window is a composite of
-  // the ordinary kind (start parity = class, translations E_c - G_c exact
-  // in one binade, the class intervals in units of u), so the chain's scan
-  // takes it without a break.
-  if (valid && M == 2) {
-    const double E0 = readlane_d(S, 0), E1 = readlane_d(S, 1);
-    const double lo0 = readlane_d(dlo, 0), hi0 = readlane_d(dhi, 0);
-    const double lo1 = readlane_d(dlo, 1), hi1 = readlane_d(dhi, 1);
-    const int key = segkey(g);
-    if (segkey(E0) == key && segkey(E1) == key && l == 0) {
-      const double ui = pow2_field(2098 - e0);  // 1/u of g's binade
-      const double g1 = g + u;
-      int pn0 = 0, pn1 = 0;
-      if (w + 1 < nw) {
-        const double gn = sg[(w + 1) * kWin * cap].g;
-        if (segkey(gn) == key) {
-          pn0 = parity_of(E0 - gn, ui);
-          pn1 = parity_of(E1 - gn, ui);
-        }
-      }
-      CompRec D = C;
-      D.g = g;
-      D.d0 = E0 - g;
-      D.d1 = E1 - g1;
-      // delta = sign(g) (S - g) / u is an integer: the class intervals,
-      // tightened to integers
-      if (g > 0.0) {
-        D.lo0 = ceil(lo0 * ui);
-        D.hi0 = floor(hi0 * ui);
-        D.lo1 = ceil(1.0 + lo1 * ui);
-        D.hi1 = floor(1.0 + hi1 * ui);
-      } else {
-        D.lo0 = ceil(-(hi0 * ui));
-        D.hi0 = floor(-(lo0 * ui));
-        D.lo1 = ceil(-(1.0 + hi1 * ui));
-        D.hi1 = floor(-(1.0 + lo1 * ui));
-      }
-      D.meta = nm | (1 << 5) | ((((pn0 ^ pn1) << 1) | pn0) << 6);
-      cp[w] = D;
-    }
-  }
-}
-
-// The window's run from S by its class table; false when the table does
-// not cover S (the caller then takes the member chain).
-__device__ __forceinline__ bool class_lookup(const int32_t *__restrict__ tab_m,
-                                             const ClassTab *__restrict__ tab,
-                                             const SegRec *__restrict__ sg, int cap, int64_t win,
-                                             double &S) {
-  const int M = tab_m[win];
-  if (M == 0) return false;
-  const int l = lane_id();
-  const ClassTab &T = tab[win];
-  const double e = l < kClasses ? T.e[l] : 0.0, gs = l < kClasses ? T.gs[l] : 0.0;
-  const double lo = l < kClasses ? T.lo[l] : 0.0, hi = l < kClasses ? T.hi[l] : 0.0;
-  const double g = readlane_d(gs, 0);
-  if (segkey(S) != segkey(g)) return false;
-  // k = (S - g) / u: the difference of the mantissas, negated for g < 0
-  const int dm = (int)((uint32_t)__double2loint(S) - (uint32_t)__double2loint(g));
-  const int c = (g < 0.0 ? -dm : dm) & (M - 1);
-  const double delta = S - readlane_d(gs, c);  // exact: one binade
-  if (!(delta >= readlane_d(lo, c) && delta <= readlane_d(hi, c))) return false;
-  S = readlane_d(e, c) + delta;
-  return true;
-}
-
-// A window that did not fold: its class table, else the member chain.
-__device__ void window_level(const double *__restrict__ a, const SegRec *__restrict__ sg, int cap,
-                             const int32_t *__restrict__ tab_m, const ClassTab *__restrict__ tab,
-                             int64_t win, int nm, uint64_t cnts, double &S) {
-  if (class_lookup(tab_m, tab, sg, cap, win, S)) return;
-  member_level(a, sg, cap, win, nm, cnts, S);
-}
-
-// The chain over 64 windows: as chain_group, with each composite's parity
-// map, translations and admissible intervals; windows that did not fold,
-// and the first rejected one, go to the member chain.
-__device__ void chain_comp(const double *__restrict__ a, const SegRec *__restrict__ sg, int cap,
-                           const int32_t *__restrict__ tab_m, const ClassTab *__restrict__ tab,
-                           const CompRec &C, int nv, double &S) {
-  const int l = lane_id();
-  const bool valid = l < nv;
-  const int ok = valid ? (C.meta >> 5) & 1 : 0;
-  const int key = segkey(C.g);
-  int q = 0;
-  while (q < nv) {
-    const int meta_q = __builtin_amdgcn_readlane(C.meta, q);
-    const int win_q = __builtin_amdgcn_readlane(C.win, q);
-    if (!((meta_q >> 5) & 1)) {
-      window_level(a, sg, cap, tab_m, tab, win_q, meta_q & 31, readlane_u64(C.cnts, q), S);
-      q++;
-      continue;
-    }
-    const int key_q = __builtin_amdgcn_readlane(key, q);
-    const uint64_t stop = __ballot(valid && l > q && (!ok || key != key_q));
-    const int h = stop ? __ffsll((unsigned long long)stop) - 1 : nv;
-    const bool in = l >= q && l < h;
-    const double g_q = readlane_d(C.g, q);
-    const int eq = binade(g_q);
-    const double ui = (eq >= 2 && eq <= 2045) ? pow2_field(2098 - eq) : 0.0;
-    const int mp = (in && l + 1 < h) ? (C.meta >> 6) & 3 : 2;
-    const int incl_m = wave_incl_map(mp);
-    int ex_m = dpp_i<0x138>(incl_m);
-    if (l == 0) ex_m = 2;
-    const int p_q = segkey(S) == key_q ? parity_of(S - g_q, ui) : 0;
-    const int p = (ex_m >> 1) ? (p_q ^ (ex_m & 1)) : (ex_m & 1);
-    const double d = in ? (p ? C.d1 : C.d0) : 0.0;
-    const double excl = wave_prev_d(wave_incl_add(d));
-    const double Sl = S + excl;
-    bool acc = false;
-    if (in && segkey(Sl) == key) {
-      const double off = Sl - C.g;  // exact: one binade
-      const double delta = (C.g < 0.0 ? -off : off) * ui;
-      acc = parity_of(off, ui) == p && delta >= (p ? C.lo1 : C.lo0) &&
-            delta <= (p ? C.hi1 : C.hi0);
-    }
-    const uint64_t rej = __ballot(in && !acc);
-    if (rej == 0) {
-      S = readlane_d(Sl + d, h - 1);
-      q = h;
-      continue;
-    }
-    const int f = __ffsll((unsigned long long)rej) - 1;
-    S = readlane_d(Sl, f);
-    const int meta_f = __builtin_amdgcn_readlane(C.meta, f);
-    const int win_f = __builtin_amdgcn_readlane(C.win, f);
-    window_level(a, sg, cap, tab_m, tab, win_f, meta_f & 31, readlane_u64(C.cnts, f), S);
-    q = f + 1;
-  }
-}
-
-// Level 2: the chain over the windows.  Wave 0 runs the chain; waves 1-3
-// stream the next block of composites into LDS meanwhile (double buffered,
-// one barrier per block).
-static constexpr int kBlockComps = 256;
-
-__global__ void __launch_bounds__(256) seq_chain(const double *__restrict__ a,
-                                                 const SegRec *__restrict__ sg, int cap,
-                                                 const CompRec *__restrict__ cp, int64_t M,
-                                                 const int32_t *__restrict__ tab_m,
-                                                 const ClassTab *__restrict__ tab, double *out) {
-  __shared__ CompRec buf[2][kBlockComps];
-  __shared__ int sink;
-  const int t = threadIdx.x, w = t >> 6;
-  const int64_t nblk = (M + kBlockComps - 1) / kBlockComps;
-  double S = 0.0;  // the reference's accumulator starts at +0
-  for (int j = t; j < kBlockComps; j += 256)
-    if (j < M) buf[0][j] = cp[j];
   __syncthreads();
-  for (int64_t k = 0; k < nblk; k++) {
-    if (w != 0) {
-      const int64_t b1 = (k + 1) * kBlockComps;
-      uint64_t touched = 0;
-      for (int j = t - 64; j < kBlockComps; j += 192) {
-        if (b1 + j >= M) break;
-        const CompRec C = cp[b1 + j];
-        buf[(k + 1) & 1][j] = C;
-        if (!((C.meta >> 5) & 1)) {
-          // the member chain will read this window's records: one load per
-          // 128-byte line brings them into this CU's caches meanwhile
-          const char *base = (const char *)(sg + (int64_t)C.win * kWin * cap);
-          const int bytes = (C.meta & 31) * cap * (int)sizeof(SegRec);
-          for (int o = 0; o < bytes; o += 128) touched ^= *(const uint64_t *)(base + o);
-        }
-      }
-      if (touched == 0x7ff4dead0badf00dull) sink = 1;  // keeps the loads
-    } else {
-      const int64_t b0 = k * kBlockComps;
-      for (int g0 = 0; g0 < kBlockComps && b0 + g0 < M; g0 += 64) {
-        const int nv = (int)min((int64_t)64, M - b0 - g0);
-        CompRec C;
-        if (t < nv) {
-          C = buf[k & 1][g0 + t];
-        } else {
-          C.g = C.d0 = C.d1 = C.lo0 = C.hi0 = C.lo1 = C.hi1 = 0.0;
-          C.win = 0;
-          C.meta = 0;
-          C.cnts = 0;
-        }
-        chain_comp(a, sg, cap, tab_m, tab, C, nv, S);
-      }
+  if (wv != 0) return;
+  double S = 0.0;  // the reference's accumulator starts at +0
+  for (int q = 0; q * per < m; q++) {
+    const int M = C.group[q].M;
+    if (M < 0) {
+      S = C.group[q].c[0].e;
+      continue;
     }
-    __syncthreads();
+    if (M > 0 && take_tab(C.group[q], S)) continue;
+    for (int k = q * per; k < min(m, (q + 1) * per); k++)
+      S = resolve(a, n, L, L.top, k, comps, S, C.vals);
   }
-  if (t == 0) *out = S;
+  if (l == 0) *dout = S;
 }
 
 __global__ void seq_zero(double *out) {
   if (threadIdx.x == 0) *out = 0.0;
 }
 
-// records per chunk (a window of kWin chunks must fit one wavefront); very
-// long arrays keep 2 to bound the work space
-static int seg_cap(int64_t nch) { return nch <= 65536 ? 64 / kWin : 2; }
-
 struct SeqLayout {
-  int64_t nch, nb, nw, tot, blk, segs, cnt, cps, tabm, tab, bytes;
-  int cap;
+  int64_t nch, nseg, tot, blk, comps, tabs[kMaxLevels], n[kMaxLevels], bytes;
+  int top;
 };
 
 static SeqLayout seq_layout(int64_t n) {
   SeqLayout L;
   L.nch = (n + kChunk - 1) / kChunk;
-  L.nb = (L.nch + 63) / 64;
-  L.nw = (L.nch + kWin - 1) / kWin;
-  L.cap = seg_cap(L.nch);
+  L.nseg = (n + kSegVals - 1) / kSegVals;
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
   L.tot = 0;
   L.blk = al(L.tot + 8 * L.nch);
-  L.segs = al(L.blk + 16 * L.nb);
-  L.cnt = al(L.segs + (int64_t)sizeof(SegRec) * L.nch * L.cap);
-  L.cps = al(L.cnt + 4 * L.nch);
-  L.tabm = al(L.cps + (int64_t)sizeof(CompRec) * L.nw);
-  L.tab = al(L.tabm + 4 * L.nw);
-  L.bytes = al(L.tab + (int64_t)sizeof(ClassTab) * L.nw);
+  L.comps = al(L.blk + 8 * L.nseg);
+  int64_t at = al(L.comps + (int64_t)sizeof(SeqComp) * kWins * L.nseg);
+  // 2^31 nodes' worth of values (the largest array any caller has) needs
+  // five levels
+  int64_t m = L.nseg;
+  for (L.top = 0;; L.top++) {
+    L.n[L.top] = m;
+    L.tabs[L.top] = at;
+    at = al(at + (int64_t)sizeof(SeqTab) * m);
+    if (m <= kTop || L.top == kMaxLevels - 1) break;
+    m = (m + kFold - 1) / kFold;
+  }
+  L.bytes = at;
   return L;
 }
 
-// The four launches of one sum over a work area laid out by seq_layout(n).
+// The launches of one sum over a work area laid out by seq_layout(n).
+// totals: the chunk totals, where the array's producer has made them.
 static int seqsum_launch(const double *a, int64_t n, double *dout, char *w, const SeqLayout &L,
-                         hipStream_t s) {
-  double *tot = (double *)(w + L.tot);
-  double2 *blk = (double2 *)(w + L.blk);
-  SegRec *segs = (SegRec *)(w + L.segs);
-  int32_t *cnt = (int32_t *)(w + L.cnt);
-  CompRec *cps = (CompRec *)(w + L.cps);
-  int32_t *tabm = (int32_t *)(w + L.tabm);
-  ClassTab *tab = (ClassTab *)(w + L.tab);
+                         hipStream_t s, const double *totals = nullptr) {
   if (n == 0) {
     hipLaunchKernelGGL(seq_zero, dim3(1), dim3(64), 0, s, dout);
     HYD_HIP(hipGetLastError());
     return HYD_OK;
   }
-  hipLaunchKernelGGL(seq_chunks<0>, dim3((unsigned)L.nb), dim3(64), 0, s, a, n, L.nch, tot, blk,
-                     segs, cnt, cps, L.cap);
-  hipLaunchKernelGGL(seq_chunks<1>, dim3((unsigned)L.nb), dim3(64), 0, s, a, n, L.nch, tot, blk,
-                     segs, cnt, cps, L.cap);
-  hipLaunchKernelGGL(seq_classes, dim3((unsigned)L.nw), dim3(64), 0, s, a, segs, L.cap, cps, L.nw,
-                     tabm, tab);
-  hipLaunchKernelGGL(seq_chain, dim3(1), dim3(256), 0, s, a, segs, L.cap, cps, L.nw, tabm, tab,
-                     dout);
+  if (L.nseg == 1) {
+    hipLaunchKernelGGL(seq_segments<true>, dim3(1), dim3(64 * kWins), 0, s, a, n, nullptr,
+                       nullptr, nullptr, nullptr, dout);
+    HYD_HIP(hipGetLastError());
+    return HYD_OK;
+  }
+  if (L.n[L.top] > kTop) {
+    set_error("seqsum: array too long");
+    return HYD_EARG;
+  }
+  double *tot = (double *)(w + L.tot);
+  double *blk = (double *)(w + L.blk);
+  SeqComp *comps = (SeqComp *)(w + L.comps);
+  SeqLevels lv;
+  lv.top = L.top;
+  for (int k = 0; k <= L.top; k++) {
+    lv.tab[k] = (const SeqTab *)(w + L.tabs[k]);
+    lv.n[k] = L.n[k];
+  }
+  // up to 512 segments (kSeqOwnTotals) each one adds the chunk totals before
+  // it (at most 128 loads a thread); beyond, a launch of the prefix is shorter
+  const bool prefixed = n > kSeqOwnTotals;
+  if (!totals || prefixed)
+    hipLaunchKernelGGL(seq_totals, dim3((unsigned)L.nseg), dim3(256), 0, s, a, n, tot, blk);
+  if (prefixed) hipLaunchKernelGGL(seq_prefix, dim3(1), dim3(1024), 0, s, blk, L.nseg);
+  hipLaunchKernelGGL(seq_segments<false>, dim3((unsigned)L.nseg), dim3(64 * kWins), 0, s, a, n,
+                     totals && !prefixed ? totals : tot, prefixed ? blk : nullptr, comps,
+                     (SeqTab *)(w + L.tabs[0]), nullptr);
+  for (int k = 1; k <= L.top; k++)
+    hipLaunchKernelGGL(seq_fold, dim3((unsigned)L.n[k]), dim3(64), 0, s, lv.tab[k - 1], L.n[k - 1],
+                       (SeqTab *)(w + L.tabs[k]));
+  constexpr size_t shm = sizeof(ChainLds);
+  static_assert(shm <= 160 * 1024, "the chain's LDS");
+  static std::atomic<bool> raised{false};  // more than 64 KiB of LDS must be requested
+  if (!raised.load(std::memory_order_acquire)) {
+    HYD_HIP(hipFuncSetAttribute((const void *)seq_chain,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    raised.store(true, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(seq_chain, dim3(1), dim3(64 * kChainWaves), shm, s, a, n, lv, comps, dout);
   HYD_HIP(hipGetLastError());
   return HYD_OK;
 }
 
-int seqsum(Ctx &c, const double *a, int64_t n, double *dout) {
+int seqsum(Ctx &c, const double *a, int64_t n, double *dout, const double *totals) {
   const SeqLayout L = seq_layout(n);
   if (L.nch > c.seq_cap || seq_layout((int64_t)c.seq_cap * kChunk).bytes < L.bytes) {
     set_error("seqsum: array longer than the context's work space");
     return HYD_ECAPACITY;
   }
   KTimer t(c, "seqsum", 8 * n);
-  return seqsum_launch(a, n, dout, (char *)c.seq_work, L, c.s);
+  return seqsum_launch(a, n, dout, (char *)c.seq_work, L, c.s, totals);
 }
 
 // ---- the sequential sum without allocation ---------------------------------
 // Work area in a file-scope device array: each GPU the library runs on holds
-// its own copy (19.06 MiB used of 24 MiB for the largest sum, 2^22 values)
+// its own copy (3.1 MiB used of 4 MiB for the largest sum, 2^22 values)
 // until the process ends.  Host code never passes `scratch` itself to a
 // kernel (in host code the name is a host-side stand-in): each device's
 // address comes from hipGetSymbolAddress, taken once per device, with that
 // device current, on the first call there.
 static constexpr int64_t kNoAllocMaxN = (int64_t)1 << 22;
-static constexpr int64_t kNoAllocBytes = (int64_t)24 << 20;
+static constexpr int64_t kNoAllocBytes = (int64_t)4 << 20;
 static __device__ __align__(256) char scratch[kNoAllocBytes];
 
 static constexpr int kMaxDevices = 64;

@@ -74,11 +74,13 @@ PW_KERNEL(k_qq_kd, (double *__restrict__ ss, const double *__restrict__ qq,
 
 // zz = zz**2 and the maxima of zz**2 and uu**2+vv**2 (evolution.f90:552-556),
 // one pair of maxima per block in mx[2 b], mx[2 b + 1] (k_adapt_scalars
-// takes the maximum over the blocks: no same-address atomics)
+// takes the maximum over the blocks: no same-address atomics); tot: the sum
+// of each 64 values of zz**2, in any order, for the sequential sum's guesses
 __global__ void __launch_bounds__(256) k_adapt_reduce(double *__restrict__ zz,
                                                       const double *__restrict__ uu,
                                                       const double *__restrict__ vv, int64_t n,
-                                                      unsigned long long *__restrict__ mx) {
+                                                      unsigned long long *__restrict__ mx,
+                                                      double *__restrict__ tot) {
   double z2m = 0.0, u2m = 0.0;
   // four elements per thread and pass, all loads in flight before any use
   constexpr int U = 4;
@@ -98,6 +100,10 @@ __global__ void __launch_bounds__(256) k_adapt_reduce(double *__restrict__ zz,
       const int64_t k = k0 + j * stride;
       const double z2 = z[j] * z[j];
       if (k < n) zz[k] = z2;
+      double s = k < n ? z2 : 0.0;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
+      if ((threadIdx.x & 63) == 0 && k < n) tot[k >> 6] = s;
       z2m = fmax(z2m, z2);
       u2m = fmax(u2m, u[j] * u[j] + v[j] * v[j]);
     }
@@ -505,9 +511,9 @@ int adapt(Ctx &c) {
   {
     KTimer t(c, "adapt_reduce", 32 * N);
     hipLaunchKernelGGL(k_adapt_reduce, dim3((unsigned)nb), dim3(256), 0, c.s, zz, c.uu, c.vv, N,
-                       c.amax);
+                       c.amax, c.seq_tot);
   }
-  HYD_CHECK(seqsum(c, zz, N, c.dsum + 1));
+  HYD_CHECK(seqsum(c, zz, N, c.dsum + 1, c.seq_tot));
   AdaptArgs a;
   a.dsumi = c.c.dsumi;
   a.small = c.c.small;

@@ -158,6 +158,40 @@ def test_sum_sequential_binade_walks_bitwise():
     h.close()
 
 
+@pytest.fixture(scope="module")
+def hyd_2048():
+    from hydra_amd import Hydra
+    h = Hydra(2048)
+    yield h
+    h.close()
+
+
+# one launch up to 4096 values, one chained level up to 64 segments of 4096,
+# then one and two folded levels; beyond 512 segments prefixed totals
+@pytest.mark.parametrize("n", [1, 64, 4095, 4096, 4097, 64 * 4096, 64 * 4096 + 1, 512 * 4096 + 1,
+                               1024 * 4096, 1024 * 4096 + 1, 4 * 2048 * 2048])
+def test_sum_sequential_level_edges_bitwise(n, hyd_2048):
+    import ctypes as C
+    from oracle.hyo import lib
+    ol = lib()
+    ol.hyo_sum_seq.restype = C.c_double
+    ol.hyo_sum_seq.argtypes = [np.ctypeslib.ndpointer(dtype=np.float64), C.c_int64]
+    rng = np.random.default_rng(n)
+    walk = rng.standard_normal(n) * 10.0 ** rng.integers(-3, 3, n)
+    level = np.full(n, 0.1)                       # no crossing for long
+    jumps = rng.standard_normal(n)
+    jumps[::1021] *= 1e12                         # starts far from any guess
+    for a in (walk, level, jumps):
+        want = np.float64(ol.hyo_sum_seq(a, n))
+        got = np.float64(hyd_2048.sum_sequential(a))
+        assert got.view(np.int64) == want.view(np.int64), (got, want)
+    for bad in (np.inf, -np.inf, np.nan):
+        a = walk.copy()
+        a[n // 2] = bad
+        want, got = ol.hyo_sum_seq(a, n), hyd_2048.sum_sequential(a)
+        assert (np.isnan(got) and np.isnan(want)) or got == want
+
+
 @pytest.mark.parametrize("ng", [32, 64])
 def test_advance_bitwise(ng):
     """Several RK4 steps of the device-resident state, every field and node
