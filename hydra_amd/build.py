@@ -19,7 +19,8 @@ LIB = os.path.join(HERE, "libhydra_amd.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("HYDRA_AMD_ARCH", "gfx950")
 
-SOURCES = ["tables.cpp", "fft.hip", "con2grid.hip", "seqsum.hip", "nodes.hip", "step.hip",
+SOURCES = ["tables.cpp", "fft.hip", "fft64_lo.hip", "fft64_hi.hip", "fft32_lo.hip",
+           "fft32_hi.hip", "con2grid.hip", "seqsum.hip", "nodes.hip", "step.hip",
            "renode.hip", "congen.hip", "surgery.hip", "capi.hip", "cnn.hip", "diag.hip"]
 
 FLAGS = [
@@ -50,7 +51,8 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
     os.makedirs(objdir, exist_ok=True)
     jobs = jobs or min(8, os.cpu_count() or 1)
     # longest compiles first so the pool finishes together
-    order = sorted(SOURCES, key=lambda f: -os.path.getsize(os.path.join(CSRC, f)))
+    order = sorted(SOURCES, key=lambda f: (not f.startswith("fft"),
+                                           -os.path.getsize(os.path.join(CSRC, f))))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         done = dict(zip(order, ex.map(lambda f: _compile(f, objdir, verbose), order)))
     objs = [done[f] for f in SOURCES]

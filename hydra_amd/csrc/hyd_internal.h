@@ -238,6 +238,9 @@ struct Ctx {
   // the GPU and the second stream's work overlaps the single-workgroup
   // sequential mean instead); con2grid runs and clears it
   std::function<int()> after_sweep;
+  // work that the plain step queues just before a contour grid is combined
+  // with the fields
+  std::function<int()> before_combine;
   double *seq_tot = nullptr;  // chunk totals that a sum's producer makes for it
   void *seq_work = nullptr; // chunk table of seqsum
   int64_t seq_cap = 0;      // chunks it holds
@@ -262,19 +265,17 @@ int fft_ptospc(Ctx &c, const double *rvar, double *svar);
 int fft_ptospc_mean(Ctx &c, const double *rvar, const double *sum, double ndiv, double *svar);
 int fft_spctop(Ctx &c, const double *svar, double *rvar, int pre, double post_sign,
                double *tmp);
-int fft_forward_1d(Ctx &c, double *x, int m);   // forfft(m, ng, x)
 // One batched 1D pass in stafft's layout (m vectors of length n, the
 // vector index fastest) in place on device memory: forfft or revfft
 // (stafft.f90:187-406) with the caller's trig table (device copy).
 int fft_1d(Ctx &c, bool fwd, int m, int n, double *x, const double *trig);
-int fft_ptospc32(Ctx &c, const float *rvar, double *svar);
 int fft_spctop_n(Ctx &c, int F, const double *const *svar, double *const *rvar, const int *pre,
                  const double *post_sign, double *const *tmp);
 int fft_ptospc_n(Ctx &c, int F, const double *const *rvar, double *const *svar);
 int fft_spctop32_n(Ctx &c, int F, const double *const *svar, float *const *rvar, const int *pre,
                    const double *post_sign, float *const *tmp);
 int fft_ptospc32_n(Ctx &c, int F, const float *const *rvar, double *const *svar,
-                   float *const *tmp);
+                   float *const *tmp, const double *mean = nullptr);
 int fft_spctop32(Ctx &c, const double *svar, float *rvar, int pre, double post_sign);
 int con2grid_mixed(Ctx &c, float *qc, bool defer_mean = false);
 int fft_ptospc32_mean(Ctx &c, const float *rvar, const double *mean, double *svar);
@@ -282,7 +283,6 @@ int advance_mixed(Ctx &c);
 int advance_mixed_head(Ctx &c);
 int advance_mixed_tail(Ctx &c);
 int fft_autotune(Ctx &c);
-int fft_reverse_1d(Ctx &c, double *x, int m);   // revfft(m, ng, x)
 
 int main_invert_dev(Ctx &c, const double *qq, double *uu, double *vv, double *pp, double *tmp);
 int gradient_dev(Ctx &c, const double *ff, double *fx, double *fy, double *tmp);

@@ -30,37 +30,10 @@ int rk_nodes(Ctx &c, int stage);
     body;                                                               \
   }
 
-// qq = flo*(qs-qc)+qc+qd  (evolution.f90:514)
-PW_KERNEL(k_combine_qq,
-          (double *__restrict__ qq, const double *__restrict__ flo, const double *__restrict__ qs,
-           const double *__restrict__ qc, const double *__restrict__ qd, int64_t n),
-          { qq[k] = flo[k] * (qs[k] - qc[k]) + qc[k] + qd[k]; })
-
-// qq as k_combine_qq, then pp = green*qq (spectral.f90:321-325), one pass
-PW_KERNEL(k_combine_green,
-          (double *__restrict__ qq, double *__restrict__ pp, const double *__restrict__ flo,
-           const double *__restrict__ green, const double *__restrict__ qs,
-           const double *__restrict__ qc, const double *__restrict__ qd, int64_t n),
-          {
-            const double q = flo[k] * (qs[k] - qc[k]) + qc[k] + qd[k];
-            qq[k] = q;
-            pp[k] = green[k] * q;
-          })
-
 // pp = green*qq  (spectral.f90:321-325)
 PW_KERNEL(k_green, (double *__restrict__ pp, const double *__restrict__ green,
                     const double *__restrict__ qq, int64_t n),
           { pp[k] = green[k] * qq[k]; })
-
-// qs = flo*(qs-qc)+qc+qd ; qd = fhi*(qs-qc)  (evolution.f90:199-200, 126)
-PW_KERNEL(k_reset, (double *__restrict__ qs, double *__restrict__ qd,
-                    const double *__restrict__ qc, const double *__restrict__ flo,
-                    const double *__restrict__ fhi, int64_t n),
-          {
-            const double s = flo[k] * (qs[k] - qc[k]) + qc[k] + qd[k];
-            qs[k] = s;
-            qd[k] = fhi[k] * (s - qc[k]);
-          })
 
 // qd = fhi*(qs-qc)  (evolution.f90:126)
 PW_KERNEL(k_init_qd, (double *__restrict__ qd, const double *__restrict__ qs,
@@ -189,68 +162,119 @@ PW_KERNEL(k_expand_epq, (double *__restrict__ epq, double *__restrict__ emq,
             emq[k] = 1.0 / v;
           })
 
-// qqx = -uu*qqx - vv*qqy  (evolution.f90:449, 460) / with beta (458)
-PW_KERNEL(k_advect_prod, (double *__restrict__ qqx, const double *__restrict__ qqy,
-                          const double *__restrict__ uu, const double *__restrict__ vv,
-                          double beta, int withbeta, int64_t n),
-          {
-            if (withbeta)
-              qqx[k] = -uu[k] * qqx[k] - vv[k] * (qqy[k] + beta);
-            else
-              qqx[k] = -uu[k] * qqx[k] - vv[k] * qqy[k];
-          })
-
-// sqd = sqd - rekman*(qq+kdsq*pp), then the integrating factor (476, 483-487)
-PW_KERNEL(k_source_finish, (double *__restrict__ sqd, const double *__restrict__ qq,
-                            const double *__restrict__ pp, const double *__restrict__ epq,
-                            double rekman, double kdsq, int lev, int64_t n),
-          {
-            double s = sqd[k] - rekman * (qq[k] + kdsq * pp[k]);
-            if (lev == 1) s = epq[k] * s;
-            else if (lev == 2) s = epq[k] * epq[k] * s;
-            sqd[k] = s;
-          })
-
-// spectral RK updates, evolution.f90:228-233, 259-262, 287-291, 313-314
-__global__ void k_rk_fields(double *__restrict__ qs, double *__restrict__ qd,
-                            double *__restrict__ qsi, double *__restrict__ qsf,
-                            double *__restrict__ qdi, double *__restrict__ qdf,
-                            const double *__restrict__ sqs, const double *__restrict__ sqd,
-                            double *__restrict__ emq, int stage, const Scalars *__restrict__ sc,
-                            int64_t n) {
+// The sources finished (evolution.f90:476, 483-487) and the spectral RK
+// updates (228-233, 259-262, 287-291, 313-314), one pass.  Bound by memory.
+// Doing this, the products below or k_combine in the transforms' own passes
+// saves the traffic but not time: a pass has half a wavefront per SIMD at
+// 1024^2 and waits for the operands, the pointwise kernels fill the device.
+// The combination fused into qc's y-pass took 21-32 us at 1024^2, by itself
+// it takes 11 on a pass of 9.
+struct RkArgs {
+  double *qs, *qd, *qsi, *qsf, *qdi, *qdf, *emq;
+  const double *sqs, *sqd, *epq, *qq, *pp;
+  double rekman, kdsq;
+  const Scalars *sc;
+};
+template <int STAGE>
+__global__ void __launch_bounds__(256) k_rk(RkArgs a, int64_t n) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  const double dt = sc->dt, dt2 = sc->dt2, dt3 = sc->dt3, dt6 = sc->dt6;
-  if (stage == 1) {
-    const double s0 = qs[k], d0 = qd[k];
-    qsi[k] = s0;
-    qs[k] = s0 + dt2 * sqs[k];
-    qsf[k] = s0 + dt6 * sqs[k];
-    qdi[k] = d0;
-    qd[k] = emq[k] * (d0 + dt2 * sqd[k]);
-    qdf[k] = d0 + dt6 * sqd[k];
-  } else if (stage == 2) {
-    qs[k] = qsi[k] + dt2 * sqs[k];
-    qsf[k] = qsf[k] + dt3 * sqs[k];
-    qd[k] = emq[k] * (qdi[k] + dt2 * sqd[k]);
-    qdf[k] = qdf[k] + dt3 * sqd[k];
-  } else if (stage == 3) {
-    qs[k] = qsi[k] + dt * sqs[k];
-    qsf[k] = qsf[k] + dt3 * sqs[k];
-    const double e = emq[k] * emq[k];
-    emq[k] = e;
-    qd[k] = e * (qdi[k] + dt * sqd[k]);
-    qdf[k] = qdf[k] + dt3 * sqd[k];
+  const double h = STAGE <= 2 ? a.sc->dt2 : a.sc->dt;
+  const double w = STAGE == 1 || STAGE == 4 ? a.sc->dt6 : a.sc->dt3;
+  const double ss = a.sqs[k], qq = a.qq[k], pp = a.pp[k], ep = STAGE > 1 ? a.epq[k] : 1.0;
+  double sd = a.sqd[k] - a.rekman * (qq + a.kdsq * pp);
+  if (STAGE == 2 || STAGE == 3) sd = ep * sd;
+  else if (STAGE == 4) sd = ep * ep * sd;
+  double em = a.emq[k];
+  if (STAGE == 1) {
+    const double s0 = a.qs[k], d0 = a.qd[k];
+    a.qsi[k] = s0;
+    a.qs[k] = s0 + h * ss;
+    a.qsf[k] = s0 + w * ss;
+    a.qdi[k] = d0;
+    a.qd[k] = em * (d0 + h * sd);
+    a.qdf[k] = d0 + w * sd;
+  } else if (STAGE < 4) {
+    const double si = a.qsi[k], sf = a.qsf[k], di = a.qdi[k], df = a.qdf[k];
+    if (STAGE == 3) {
+      em = em * em;
+      a.emq[k] = em;
+    }
+    a.qs[k] = si + h * ss;
+    a.qsf[k] = sf + w * ss;
+    a.qd[k] = em * (di + h * sd);
+    a.qdf[k] = df + w * sd;
   } else {
-    qs[k] = qsf[k] + dt6 * sqs[k];
-    qd[k] = emq[k] * (qdf[k] + dt6 * sqd[k]);
+    const double sf = a.qsf[k], df = a.qdf[k];
+    a.qs[k] = sf + w * ss;
+    a.qd[k] = em * (df + w * sd);
   }
+}
+
+// -uu qqx - vv qqy of qd and qs (evolution.f90:449, 460; beta enters qs's,
+// 458), over qqx
+struct ProdArgs {
+  void *qx[2];
+  const void *qy[2], *uu, *vv;
+  double beta;
+  int with_beta;
+};
+template <class T>
+__global__ void __launch_bounds__(256) k_prod(ProdArgs a, int64_t n) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const T u = ((const T *)a.uu)[k], v = ((const T *)a.vv)[k];
+  const T x0 = ((T *)a.qx[0])[k], x1 = ((T *)a.qx[1])[k];
+  const T y0 = ((const T *)a.qy[0])[k];
+  T y1 = ((const T *)a.qy[1])[k];
+  if (a.with_beta) y1 = y1 + (T)a.beta;
+  ((T *)a.qx[0])[k] = -u * x0 - v * y0;
+  ((T *)a.qx[1])[k] = -u * x1 - v * y1;
 }
 
 static inline dim3 grid1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
-// The contour part of inversion: qc = ptospc(con2grid) (evolution.f90:507-508).
-static int contour_grid(Ctx &c) {
+// qq = flo*(qs-qc)+qc+qd (evolution.f90:514) and pp = green*qq
+// (spectral.f90:321-325) in one pass; RESET: also the step's start, qs = qq
+// and qd = fhi*(qs-qc) (evolution.f90:199-200, 126).
+struct CombineArgs {
+  const double *flo, *green, *fhi, *qc;
+  double *qs, *qd, *qq, *pp;
+};
+template <bool RESET>
+__global__ void k_combine(CombineArgs a, int64_t n) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const double qc = a.qc[k], flo = a.flo[k], gr = a.green[k], fhi = RESET ? a.fhi[k] : 0.0;
+  const double q = flo * (a.qs[k] - qc) + qc + a.qd[k];
+  a.qq[k] = q;
+  a.pp[k] = gr * q;
+  if (RESET) {
+    a.qs[k] = q;
+    a.qd[k] = fhi * (q - qc);
+  }
+}
+
+// The combination of an inversion once qc is there.  wait: an event that qs
+// and qd wait for.
+static int combine(Ctx &c, bool reset, hipEvent_t wait) {
+  if (c.before_combine) {
+    auto fn = std::move(c.before_combine);
+    c.before_combine = nullptr;
+    HYD_CHECK(fn());
+  }
+  if (wait) HYD_HIP(hipStreamWaitEvent(c.s, wait, 0));
+  KTimer t(c, "combine_qq", (reset ? 80 : 56) * c.N);
+  const CombineArgs a = {c.flo, c.green, c.fhi, c.qc, c.qs, c.qd, c.qq, c.pp};
+  if (reset) hipLaunchKernelGGL(k_combine<true>, grid1(c.N), dim3(256), 0, c.s, a, c.N);
+  else hipLaunchKernelGGL(k_combine<false>, grid1(c.N), dim3(256), 0, c.s, a, c.N);
+  HYD_HIP(hipGetLastError());
+  return HYD_OK;
+}
+
+// The contour part of inversion: qc = ptospc(con2grid) (evolution.f90:507-508),
+// then qq and pp.
+static int contour_grid(Ctx &c, bool reset, hipEvent_t wait) {
   // with per-launch timing (one stream) the deferred work runs first, so
   // that the contour grid's records hold its own kernels only
   if ((c.nptq == 0 || c.timing) && c.after_sweep) {
@@ -260,34 +284,26 @@ static int contour_grid(Ctx &c) {
   }
   if (c.nptq == 0) {
     HYD_CHECK(con2grid(c, c.xq, c.yq, c.nextq, c.nptq, c.c2g_q, nullptr));
-    return fft_ptospc(c, c.c2g_q, c.qc);
+    HYD_CHECK(fft_ptospc(c, c.c2g_q, c.qc));
+  } else {
+    HYD_CHECK(con2grid(c, c.xq, c.yq, c.nextq, c.nptq, nullptr, nullptr, true));
+    HYD_CHECK(fft_ptospc_mean(c, c.c2g_w, c.dsum, (double)c.N, c.qc));
   }
-  HYD_CHECK(con2grid(c, c.xq, c.yq, c.nextq, c.nptq, nullptr, nullptr, true));
-  return fft_ptospc_mean(c, c.c2g_w, c.dsum, (double)c.N, c.qc);
+  return combine(c, reset, wait);
 }
 
-// The field part of inversion: qq, pp and the velocity (evolution.f90:510-520).
+// The velocity of pp (evolution.f90:510-520, main_invert): vv =
+// spctop(xderiv(pp)), uu = -spctop(yderiv(pp)), one batch.
 static int inversion_fields(Ctx &c) {
-  const int64_t N = c.N;
-  {
-    KTimer t(c, "combine_qq", 56 * N);
-    hipLaunchKernelGGL(k_combine_green, grid1(N), dim3(256), 0, c.s, c.qq, c.pp, c.flo, c.green,
-                       c.qs, c.qc, c.qd, N);
-  }
-  HYD_HIP(hipGetLastError());
-  // main_invert: vv = spctop(xderiv(pp)), uu = -spctop(yderiv(pp)), one batch
-  {
-    const double *in[2] = {c.pp, c.pp};
-    double *out[2] = {c.vv, c.uu};
-    const int pre[2] = {PRE_XDERIV, PRE_YDERIV};
-    const double sg[2] = {1.0, -1.0};
-    HYD_CHECK(fft_spctop_n(c, 2, in, out, pre, sg, c.t4));
-  }
-  return HYD_OK;
+  const double *in[2] = {c.pp, c.pp};
+  double *out[2] = {c.vv, c.uu};
+  const int pre[2] = {PRE_XDERIV, PRE_YDERIV};
+  const double sg[2] = {1.0, -1.0};
+  return fft_spctop_n(c, 2, in, out, pre, sg, c.t4);
 }
 
 int inversion(Ctx &c) {
-  HYD_CHECK(contour_grid(c));
+  HYD_CHECK(contour_grid(c, false, nullptr));
   return inversion_fields(c);
 }
 
@@ -562,9 +578,9 @@ int adapt_finish(Ctx &c) {
   return HYD_OK;
 }
 
-int source(Ctx &c, int lev) {
-  const int64_t N = c.N;
-  const int wb = c.c.beffect ? 1 : 0;
+// source (evolution.f90:432-490) up to its last line, which the field update
+// does (rk_fields).
+static int source(Ctx &c) {
   // the four gradients (qd and qs, x and y) in one batch
   {
     const double *in[4] = {c.qd, c.qd, c.qs, c.qs};
@@ -574,39 +590,34 @@ int source(Ctx &c, int lev) {
     HYD_CHECK(fft_spctop_n(c, 4, in, out, pre, sg, c.t4));
   }
   {
-    KTimer t(c, "advect_prod", 80 * N);
-    hipLaunchKernelGGL(k_advect_prod, grid1(N), dim3(256), 0, c.s, c.wa, c.wb, c.uu, c.vv,
-                       c.p.beta, 0, N);
-    hipLaunchKernelGGL(k_advect_prod, grid1(N), dim3(256), 0, c.s, c.wc, c.wd, c.uu, c.vv,
-                       c.p.beta, wb, N);
-  }
-  {
-    const double *in[2] = {c.wa, c.wc};
-    double *out[2] = {c.sqd, c.sqs};
-    HYD_CHECK(fft_ptospc_n(c, 2, in, out));
-  }
-  {
-    KTimer t(c, "source_finish", 40 * N);
-    hipLaunchKernelGGL(k_source_finish, grid1(N), dim3(256), 0, c.s, c.sqd, c.qq, c.pp, c.epq,
-                       c.p.rekman, c.c.kdsq, lev, N);
+    KTimer t(c, "advect_prod", 64 * c.N);
+    const ProdArgs a = {{c.wa, c.wc}, {c.wb, c.wd}, c.uu, c.vv, c.p.beta, c.c.beffect ? 1 : 0};
+    hipLaunchKernelGGL(k_prod<double>, grid1(c.N), dim3(256), 0, c.s, a, c.N);
   }
   HYD_HIP(hipGetLastError());
-  return HYD_OK;
+  const double *in[2] = {c.wa, c.wc};
+  double *out[2] = {c.sqd, c.sqs};
+  return fft_ptospc_n(c, 2, in, out);
 }
 
 static int rk_fields(Ctx &c, int stage) {
-  const int64_t N = c.N;
-  static const int64_t words[5] = {0, 11, 10, 12, 6};
-  KTimer t(c, "rk_fields", words[stage] * 8 * N);
-  hipLaunchKernelGGL(k_rk_fields, grid1(N), dim3(256), 0, c.s, c.qs, c.qd, c.qsi, c.qsf, c.qdi,
-                     c.qdf, c.sqs, c.sqd, c.emq, stage, c.dsc, N);
+  static const int64_t words[5] = {0, 13, 13, 14, 9};
+  KTimer t(c, "rk_fields", words[stage] * 8 * c.N);
+  const RkArgs a = {c.qs,  c.qd, c.qsi, c.qsf, c.qdi,      c.qdf,    c.emq, c.sqs,
+                    c.sqd, c.epq, c.qq, c.pp,  c.p.rekman, c.c.kdsq, c.dsc};
+  const dim3 g = grid1(c.N);
+  if (stage == 1) hipLaunchKernelGGL(k_rk<1>, g, dim3(256), 0, c.s, a, c.N);
+  else if (stage == 2) hipLaunchKernelGGL(k_rk<2>, g, dim3(256), 0, c.s, a, c.N);
+  else if (stage == 3) hipLaunchKernelGGL(k_rk<3>, g, dim3(256), 0, c.s, a, c.N);
+  else hipLaunchKernelGGL(k_rk<4>, g, dim3(256), 0, c.s, a, c.N);
   HYD_HIP(hipGetLastError());
   return HYD_OK;
 }
 
-// Advance the host mirror of t by dt/2 (t=t+dt2, evolution.f90:237, 295).
+// t = t + dt2 after stages 1 and 3 (evolution.f90:237, 295); nothing reads
+// t in between, so both additions are made at the step's end.
 __global__ void k_tick(Scalars *sc) {
-  if (threadIdx.x == 0) sc->t = sc->t + sc->dt2;
+  if (threadIdx.x == 0) sc->t = (sc->t + sc->dt2) + sc->dt2;
 }
 
 // One RK4 step (evolution.f90:166-326).  Stage k's source and field update
@@ -631,9 +642,9 @@ static int on_s2(Ctx &c, Fn fn) {
 
 // A contour grid whose sweep leaves its clearing to the caller (who runs
 // it on the second stream, off the main stream's path).
-static int contour_grid_deferred(Ctx &c) {
+static int contour_grid_deferred(Ctx &c, bool reset, hipEvent_t wait) {
   c.defer_clear = true;
-  const int rc = contour_grid(c);
+  const int rc = contour_grid(c, reset, wait);
   c.defer_clear = false;
   return rc;
 }
@@ -647,17 +658,9 @@ static int fork_s2(Ctx &c) {
 }
 
 int advance(Ctx &c) {
-  const int64_t N = c.N;
   c.after_sweep = nullptr;
   c.n_advances += 1;
   c.n_node_updates += c.nptq;
-  auto fields = [&](int stage) {
-    return on_s2(c, [&]() {
-      HYD_CHECK(rk_fields(c, stage));
-      HYD_HIP(hipEventRecord(c.ev_join, c.s));
-      return HYD_OK;
-    });
-  };
   // stage k's source and field update, started once the next contour
   // grid's sweep is queued (con2grid runs c.after_sweep)
   auto source_fields_later = [&](int stage) {
@@ -665,7 +668,7 @@ int advance(Ctx &c) {
       HYD_CHECK(fork_s2(c));
       return on_s2(c, [&]() {
         HYD_CHECK(sweep_clear(c));  // the sweep just queued
-        HYD_CHECK(source(c, 1));
+        HYD_CHECK(source(c));
         HYD_CHECK(rk_fields(c, stage));
         HYD_HIP(hipEventRecord(c.ev_join, c.s));
         return HYD_OK;
@@ -673,9 +676,8 @@ int advance(Ctx &c) {
     };
   };
   // stage 1 (its sweep's clearing runs on the second stream after adapt)
-  HYD_CHECK(contour_grid_deferred(c));
+  HYD_CHECK(contour_grid_deferred(c, true, nullptr));
   HYD_CHECK(inversion_fields(c));
-  hipLaunchKernelGGL(k_reset, grid1(N), dim3(256), 0, c.s, c.qs, c.qd, c.qc, c.flo, c.fhi, N);
   // saves that fall at this step's start (set by the previous adapt)
   if (c.saves_on && (c.gsave || c.csave)) HYD_CHECK(save_slots(c, c.gsave != 0, c.csave != 0));
   HYD_CHECK(adapt(c));
@@ -683,38 +685,46 @@ int advance(Ctx &c) {
   HYD_CHECK(on_s2(c, [&]() {
     if (!c.saves_on) HYD_CHECK(adapt_copy(c));  // off the main stream's path
     HYD_CHECK(sweep_clear(c));
-    return source(c, 0);
+    return source(c);
   }));
   HYD_CHECK(rk_nodes(c, 1));
-  // stage 2's contour grid needs only the stage-1 nodes: it is queued
+  // stage 2's contour grid needs only the stage-1 nodes: all of it but its
+  // combination with the fields is queued
   // before the host evaluates the integrating factors, so that the GPU has
   // it to run meanwhile; the factors are uploaded and expanded on the
   // second stream, ahead of the stage-1 field update that needs them
-  // (the tick changes t: the scalars' copy on the second stream has read them)
-  if (!c.saves_on) HYD_HIP(hipStreamWaitEvent(c.s, c.ev_sc, 0));
-  hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, c.s, c.dsc);
-  HYD_CHECK(contour_grid(c));
-  HYD_CHECK(on_s2(c, [&]() { return adapt_finish(c); }));
-  // an overflow of an earlier sweep (the scalars are on the host now):
-  // reported, and the table reset, behind the main stream's queued sweep
-  if (c.hsc->sweep_err != 0.0) return c2g_status(c);
-  HYD_CHECK(fields(1));
+  c.before_combine = [&]() {
+    c.before_combine = nullptr;
+    HYD_CHECK(on_s2(c, [&]() { return adapt_finish(c); }));
+    // an overflow of an earlier sweep (the scalars are on the host now):
+    // reported behind the main stream's queued sweep
+    if (c.hsc->sweep_err != 0.0) return c2g_status(c);
+    return on_s2(c, [&]() {
+      HYD_CHECK(rk_fields(c, 1));
+      HYD_HIP(hipEventRecord(c.ev_join, c.s));
+      return HYD_OK;
+    });
+  };
+  const int rc2 = contour_grid(c, false, c.ev_join);
+  c.before_combine = nullptr;
+  HYD_CHECK(rc2);
   // stages 2-4
   for (int stage = 2; stage <= 4; stage++) {
-    if (stage > 2) {
-      if (stage != 3) hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, c.s, c.dsc);
-      HYD_CHECK(contour_grid_deferred(c));  // clearing in the after-sweep work
-    }
-    HYD_HIP(hipStreamWaitEvent(c.s, c.ev_join, 0));
+    if (stage > 2) HYD_CHECK(contour_grid_deferred(c, false, c.ev_join));
     HYD_CHECK(inversion_fields(c));
     if (stage < 4) {
       source_fields_later(stage);
       HYD_CHECK(rk_nodes(c, stage));
     } else {
       HYD_CHECK(fork_s2(c));
-      HYD_CHECK(on_s2(c, [&]() { return source(c, 2); }));
+      HYD_CHECK(on_s2(c, [&]() {
+        HYD_CHECK(source(c));
+        HYD_CHECK(rk_fields(c, stage));
+        hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, c.s, c.dsc);
+        HYD_HIP(hipEventRecord(c.ev_join, c.s));
+        return HYD_OK;
+      }));
       HYD_CHECK(rk_nodes(c, stage));
-      HYD_CHECK(fields(stage));
     }
   }
   c.after_sweep = nullptr;
@@ -759,17 +769,6 @@ int evolution_init(Ctx &c) {
 // RK accumulation.  No host round trip: the integrating factors use the
 // device exp, the sums are parallel reductions, so the step can be captured
 // in a graph.
-
-// qqx = -uu*qqx - vv*qqy in FP32
-PW_KERNEL(k_advect_prod32, (float *__restrict__ qqx, const float *__restrict__ qqy,
-                            const float *__restrict__ uu, const float *__restrict__ vv,
-                            float beta, int withbeta, int64_t n),
-          {
-            if (withbeta)
-              qqx[k] = -uu[k] * qqx[k] - vv[k] * (qqy[k] + beta);
-            else
-              qqx[k] = -uu[k] * qqx[k] - vv[k] * qqy[k];
-          })
 
 // sum of zz^2 per block (FP64 accumulation) and the maxima of zz^2, uu^2+vv^2
 // (one pair per block in mx[2 b], mx[2 b + 1])
@@ -862,9 +861,7 @@ static int adapt_mixed(Ctx &c) {
   return HYD_OK;
 }
 
-static int source_mixed(Ctx &c, int lev) {
-  const int64_t N = c.N;
-  const int wb = c.c.beffect ? 1 : 0;
+static int source_mixed(Ctx &c) {
   {
     const double *in[4] = {c.qd, c.qd, c.qs, c.qs};
     float *out[4] = {c.fa32, c.fb32, c.fd32, c.fe32};
@@ -872,39 +869,27 @@ static int source_mixed(Ctx &c, int lev) {
     const double sg[4] = {1.0, 1.0, 1.0, 1.0};
     HYD_CHECK(fft_spctop32_n(c, 4, in, out, pre, sg, c.t32));
   }
-  hipLaunchKernelGGL(k_advect_prod32, grid1(N), dim3(256), 0, c.s, c.fa32, c.fb32, c.uu32,
-                     c.vv32, (float)c.p.beta, 0, N);
-  hipLaunchKernelGGL(k_advect_prod32, grid1(N), dim3(256), 0, c.s, c.fd32, c.fe32, c.uu32,
-                     c.vv32, (float)c.p.beta, wb, N);
-  {
-    const float *in[2] = {c.fa32, c.fd32};
-    double *out[2] = {c.sqd, c.sqs};
-    HYD_CHECK(fft_ptospc32_n(c, 2, in, out, c.t32));
-  }
-  hipLaunchKernelGGL(k_source_finish, grid1(N), dim3(256), 0, c.s, c.sqd, c.qq, c.pp, c.epq,
-                     c.p.rekman, c.c.kdsq, lev, N);
+  const ProdArgs a = {{c.fa32, c.fd32}, {c.fb32, c.fe32}, c.uu32, c.vv32, c.p.beta,
+                      c.c.beffect ? 1 : 0};
+  hipLaunchKernelGGL(k_prod<float>, grid1(c.N), dim3(256), 0, c.s, a, c.N);
   HYD_HIP(hipGetLastError());
-  return HYD_OK;
+  const float *in[2] = {c.fa32, c.fd32};
+  double *out[2] = {c.sqd, c.sqs};
+  return fft_ptospc32_n(c, 2, in, out, c.t32);
 }
 
-static int contour_grid_mixed(Ctx &c) {
+static int contour_grid_mixed(Ctx &c, bool reset, hipEvent_t wait) {
   HYD_CHECK(con2grid_mixed(c, nullptr, true));
-  return fft_ptospc32_mean(c, c.fc32, c.part + 1024, c.qc);
+  HYD_CHECK(fft_ptospc32_mean(c, c.fc32, c.part + 1024, c.qc));
+  return combine(c, reset, wait);
 }
 
 static int inversion_fields_mixed(Ctx &c) {
-  const int64_t N = c.N;
-  hipLaunchKernelGGL(k_combine_qq, grid1(N), dim3(256), 0, c.s, c.qq, c.flo, c.qs, c.qc, c.qd, N);
-  hipLaunchKernelGGL(k_green, grid1(N), dim3(256), 0, c.s, c.pp, c.green, c.qq, N);
-  HYD_HIP(hipGetLastError());
-  {
-    const double *in[2] = {c.pp, c.pp};
-    float *out[2] = {c.vv32, c.uu32};
-    const int pre[2] = {PRE_XDERIV, PRE_YDERIV};
-    const double sg[2] = {1.0, -1.0};
-    HYD_CHECK(fft_spctop32_n(c, 2, in, out, pre, sg, c.t32));
-  }
-  return HYD_OK;
+  const double *in[2] = {c.pp, c.pp};
+  float *out[2] = {c.vv32, c.uu32};
+  const int pre[2] = {PRE_XDERIV, PRE_YDERIV};
+  const double sg[2] = {1.0, -1.0};
+  return fft_spctop32_n(c, 2, in, out, pre, sg, c.t32);
 }
 
 // The same stage overlap as the plain step (advance); the fork and join are
@@ -914,10 +899,8 @@ static int inversion_fields_mixed(Ctx &c) {
 // four stages), so that a loop can read the scalars back between the two
 // and decide the next step while the tail runs.
 int advance_mixed_head(Ctx &c) {
-  const int64_t N = c.N;
-  HYD_CHECK(contour_grid_mixed(c));
+  HYD_CHECK(contour_grid_mixed(c, true, nullptr));
   HYD_CHECK(inversion_fields_mixed(c));
-  hipLaunchKernelGGL(k_reset, grid1(N), dim3(256), 0, c.s, c.qs, c.qd, c.qc, c.flo, c.fhi, N);
   return adapt_mixed(c);
 }
 
@@ -927,25 +910,20 @@ int advance_mixed(Ctx &c) {
 }
 
 int advance_mixed_tail(Ctx &c) {
-  auto fields = [&](int stage) {
-    return on_s2(c, [&]() {
-      HYD_CHECK(rk_fields(c, stage));
-      HYD_HIP(hipEventRecord(c.ev_join, c.s));
-      return HYD_OK;
-    });
-  };
   for (int stage = 1; stage <= 4; stage++) {
     if (stage > 1) {
-      if (stage != 3) hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, c.s, c.dsc);
-      HYD_CHECK(contour_grid_mixed(c));
-      HYD_HIP(hipStreamWaitEvent(c.s, c.ev_join, 0));
+      HYD_CHECK(contour_grid_mixed(c, false, c.ev_join));
       HYD_CHECK(inversion_fields_mixed(c));
     }
     HYD_CHECK(fork_s2(c));
-    const int lev = stage == 1 ? 0 : (stage == 4 ? 2 : 1);
-    HYD_CHECK(on_s2(c, [&]() { return source_mixed(c, lev); }));
+    HYD_CHECK(on_s2(c, [&]() {
+      HYD_CHECK(source_mixed(c));
+      HYD_CHECK(rk_fields(c, stage));
+      if (stage == 4) hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, c.s, c.dsc);
+      HYD_HIP(hipEventRecord(c.ev_join, c.s));
+      return HYD_OK;
+    }));
     HYD_CHECK(rk_nodes(c, stage));
-    HYD_CHECK(fields(stage));
   }
   HYD_HIP(hipStreamWaitEvent(c.s, c.ev_join, 0));
   HYD_HIP(hipGetLastError());

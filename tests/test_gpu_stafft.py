@@ -54,3 +54,35 @@ def test_xderiv_yderiv_bitwise(ctx):
         want = np.empty_like(s)
         getattr(olib(), f"hyo_{name}deriv")(64, 64, o.d(k, 64), s, want)
         assert bits_equal(fn(s), want), name
+
+
+# every length: the last block whole, one vector short and one vector full
+@pytest.mark.parametrize("n", [8, 16, 32, 64, 128, 256, 512, 1024, 2048, 4096])
+def test_every_length_bitwise(ctx, n):
+    from hydra_amd import initfft
+    from oracle.hyo import lib as olib
+    f, t = initfft(n)
+    for m in (1, 15, 16, 33):
+        x = np.random.default_rng(100 * n + m).standard_normal(m * n)
+        want = x.copy()
+        olib().hyo_forfft(m, n, want, t, f)
+        assert bits_equal(ctx.forfft(m, n, x, t, f), want), ("forfft", m)
+        back = want.copy()
+        olib().hyo_revfft(m, n, back, t, f)
+        assert bits_equal(ctx.revfft(m, n, want, t, f), back), ("revfft", m)
+
+
+# the grids whose transforms take one, two and three passes over LDS, with
+# and without a factor 2
+@pytest.mark.parametrize("ng", [16, 128, 512, 1024])
+def test_2d_transforms_bitwise(ng):
+    from hydra_amd import Hydra
+    from oracle.hyo import Oracle
+    x = np.random.default_rng(ng).standard_normal((ng, ng))
+    o, h = Oracle(ng), Hydra(ng)
+    try:
+        want = o.ptospc(x)
+        assert bits_equal(h.ptospc(x), want)
+        assert bits_equal(h.spctop(want), o.spctop(want))
+    finally:
+        h.close()
