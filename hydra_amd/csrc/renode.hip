@@ -6,7 +6,7 @@
 // expression order.  The two sequential pieces -- the sum of the fractional
 // node counts (contours.f90:799-802, whose nint decides how many nodes the
 // contour keeps) and the accumulator walk that places the new nodes
-// (813-930) -- run as wavefront-uniform chains: 64 consecutive values are
+// (813-930) -- run as wavefront-uniform chains: consecutive values are
 // staged in LDS and every lane reads each one by broadcast, so the serial
 // chain is the floating-point additions alone.  The walk is written per old
 // node: acc + e(i) is the only rounded operation (acc - 1 is exact for acc
@@ -144,28 +144,41 @@ __device__ __forceinline__ double e_at(const double *se, int64_t o, int n, int i
   return se[o + i];
 }
 
+// The chains of long stretches take kRnBlock nodes at a time through LDS, the
+// next ones in flight meanwhile.
+static constexpr int kRnPer = 4, kRnBlock = 64 * kRnPer;
+__device__ __forceinline__ void load_block(double (&v)[kRnPer], const double *se, int64_t o, int n,
+                                           int ibeg, int q0, int len) {
+  const int l = threadIdx.x & 63;
+#pragma unroll
+  for (int j = 0; j < kRnPer; j++) {
+    const int q = q0 + 64 * j + l;
+    v[j] = q < len ? e_at(se, o, n, ibeg, q % n) : 0.0;
+  }
+}
+
 // Sequential sum of e over len nodes from ibeg (wrapping: next() order),
 // contours.f90:799-802 and 880-884.  Wavefront-uniform (every lane returns
-// the same value); lds holds 64 doubles of the calling wavefront.
+// the same value); lds holds kRnBlock doubles of the calling wavefront.
+// Bound by the serial additions, 4.3 ns each from LDS.
 __device__ double seq_sum_e(const double *se, int64_t o, int n, int ibeg, int len,
                             double *lds) {
   const int l = threadIdx.x & 63;
-  double s = 0.0;
-  double v = l < len ? e_at(se, o, n, ibeg, l) : 0.0;
-  for (int q0 = 0; q0 < len; q0 += 64) {
-    const int qn = q0 + 64 + l;
-    const double vn = qn < len ? e_at(se, o, n, ibeg, qn) : 0.0;  // next block in flight
-    lds[l] = v;
-    wave_sync();
-    const int m = len - q0 < 64 ? len - q0 : 64;
-    if (m == 64) {
+  double s = 0.0, v[kRnPer];
+  load_block(v, se, o, n, ibeg, 0, len);
+  for (int q0 = 0; q0 < len; q0 += kRnBlock) {
 #pragma unroll
-      for (int j = 0; j < 64; j++) s = s + lds[j];
-    } else {
-      for (int j = 0; j < m; j++) s = s + lds[j];
-    }
+    for (int j = 0; j < kRnPer; j++) lds[64 * j + l] = v[j];
+    if (q0 + kRnBlock < len) load_block(v, se, o, n, ibeg, q0 + kRnBlock, len);
     wave_sync();
-    v = vn;
+    const int m = len - q0 < kRnBlock ? len - q0 : kRnBlock;
+    int j = 0;
+    for (; j + 64 <= m; j += 64) {
+#pragma unroll
+      for (int k = 0; k < 64; k++) s = s + lds[j + k];
+    }
+    for (; j < m; j++) s = s + lds[j];
+    wave_sync();
   }
   return s;
 }
@@ -173,55 +186,69 @@ __device__ double seq_sum_e(const double *se, int64_t o, int n, int ibeg, int le
 // The accumulator walk (contours.f90:826-838, 858-868, 907-920) over the
 // nodes ibeg, next(ibeg), ... for `want` new nodes, written to out slots
 // oo+1 .. oo+want (old node index, acc after the subtraction).  acc starts
-// at 0; at most maxlen old nodes are visited.  Wavefront 0 only.
-__device__ void walk_nodes(const RenodeArgs &g, int64_t o, int n, int ibeg, int maxlen,
+// at 0; e sums to the wanted count over len nodes, at most maxlen old nodes
+// are visited.  Wavefront 0 only; lds_e and lds_s hold kRnBlock doubles.
+__device__ void walk_nodes(const RenodeArgs &g, int64_t o, int n, int ibeg, int len, int maxlen,
                            int want, int64_t oo, double *lds_e, double *lds_s) {
   const int l = threadIdx.x & 63;
-  double acc = 0.0;
+  double acc = 0.0, v[kRnPer];
   int done = 0;
-  double v = l < maxlen ? e_at(g.se, o, n, ibeg, l % n) : 0.0;
-  for (int q0 = 0; q0 < maxlen && done < want; q0 += 64) {
-    const int qn = q0 + 64 + l;
-    const double vn = qn < maxlen ? e_at(g.se, o, n, ibeg, qn % n) : 0.0;
-    lds_e[l] = v;
+  load_block(v, g.se, o, n, ibeg, 0, len);
+  int end = len, m;
+  for (int q0 = 0; q0 < maxlen && done < want; q0 += m) {
+#pragma unroll
+    for (int j = 0; j < kRnPer; j++) lds_e[64 * j + l] = v[j];
+    m = end - q0 < kRnBlock ? end - q0 : kRnBlock;
+    if (q0 + m == end) end = maxlen;
+    if (q0 + m < end) load_block(v, g.se, o, n, ibeg, q0 + m, end);
     wave_sync();
-    const int m = maxlen - q0 < 64 ? maxlen - q0 : 64;
-    if (m == 64) {
-#pragma unroll 16
-      for (int j = 0; j < 64; j++) {
-        const double sj = acc + lds_e[j];
-        lds_s[j] = sj;
-        acc = sj - floor(sj);
-      }
-    } else {
-      for (int j = 0; j < m; j++) {
-        const double sj = acc + lds_e[j];
-        lds_s[j] = sj;
-        acc = sj - floor(sj);
+    // s - floor(s) is exact and s >= 0: the hardware's fraction
+    int j = 0;
+    for (; j + 16 <= m; j += 16) {
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        const double sj = acc + lds_e[j + k];
+        lds_s[j + k] = sj;
+        acc = __builtin_amdgcn_fract(sj);
       }
     }
+    for (; j < m; j++) {
+      const double sj = acc + lds_e[j];
+      lds_s[j] = sj;
+      acc = __builtin_amdgcn_fract(sj);
+    }
     wave_sync();
-    // old node q0+l places floor(s) new nodes, capped at the total wanted
-    const double sl = l < m ? lds_s[l] : 0.0;
-    const int k = l < m ? (int)floor(sl) : 0;
-    int incl = k;
+    // old node q0+q places floor(s) new nodes, capped at the total wanted;
+    // a lane takes kRnPer consecutive ones
+    double sl[kRnPer];
+    int k[kRnPer], mine = 0;
+#pragma unroll
+    for (int i = 0; i < kRnPer; i++) {
+      const int q = kRnPer * l + i;
+      sl[i] = q < m ? lds_s[q] : 0.0;
+      k[i] = q < m ? (int)floor(sl[i]) : 0;
+      mine += k[i];
+    }
+    int incl = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const int t = __shfl_up(incl, d, 64);
       if (l >= d) incl += t;
     }
-    const int excl = incl - k;
-    int i = ibeg + ((q0 + l) % n);
-    if (i >= n) i -= n;
-    for (int r = 1; r <= k; r++) {
-      const int slot = done + excl + r;  // 1-based new node after the first
-      if (slot > want) break;
-      g.wi[oo + slot] = i;
-      g.wacc[oo + slot] = sl - (double)r;
+    int slot = done + incl - mine;  // 1-based new node after the first
+    int i0 = ibeg + (q0 + kRnPer * l) % n;
+    if (i0 >= n) i0 -= n;
+#pragma unroll
+    for (int i = 0; i < kRnPer; i++) {
+      for (int r = 1; r <= k[i]; r++) {
+        if (++slot > want) break;
+        g.wi[oo + slot] = i0;
+        g.wacc[oo + slot] = sl[i] - (double)r;
+      }
+      if (++i0 == n) i0 = 0;
     }
     done += __shfl(incl, 63, 64);
     wave_sync();
-    v = vn;
   }
   // (sum(e) = the wanted count, so the walk always ends with done = want;
   // should rounding ever leave slots, they get the last node, never an
@@ -249,8 +276,51 @@ __device__ __forceinline__ void place(const RenodeArgs &g, int64_t o, int i, dou
   yo = g.oms * wrapc(yy, g.elly, g.hlyi);
 }
 
+// Exclusive prefix of v over the workgroup's 256 threads, and the total;
+// lds holds 4 integers.
+__device__ __forceinline__ int block_excl(int v, int *lds, int &total) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int incl = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int t = __shfl_up(incl, d, 64);
+    if (l >= d) incl += t;
+  }
+  __syncthreads();  // the previous call's reads
+  if (l == 63) lds[w] = incl;
+  __syncthreads();
+  const int t0 = lds[0], t1 = lds[1], t2 = lds[2], t3 = lds[3];
+  total = t0 + t1 + t2 + t3;
+  return incl - v + (w > 0 ? t0 : 0) + (w > 1 ? t1 : 0) + (w > 2 ? t2 : 0);
+}
+
+// The stretches between corners (contours.f90:873-929) of a contour, kept
+// from the count pass to the place pass in the scratch of u and v, which the
+// geometry no longer needs (a contour has at most as many corners as nodes):
+// stretch k starts at node beg(k), has len(k) nodes, its e sum to sum(k) and
+// it gets np(k) nodes.
+struct Stretches {
+  int2 *u;      // .x the corner, .y the node count
+  double *sum;
+  int n, ncorn;
+  __device__ Stretches(const RenodeArgs &g, int64_t o, int n_, int nc)
+      : u((int2 *)(g.su + o)), sum(g.sv + o), n(n_), ncorn(nc) {}
+  __device__ int beg(int k) const { return u[k].x; }
+  __device__ int len(int k) const {
+    const int e = u[k + 1 < ncorn ? k + 1 : 0].x, b = u[k].x;
+    return e > b ? e - b : e + n - b;
+  }
+};
+// A stretch of up to kShort nodes is one lane's, longer ones are a wavefront's.
+// A recontoured field's contours have a corner every few nodes, thousands
+// of them on the longest contours: recontouring a developed ng=64 flow took
+// 5.9 + 3.1 ms in the two launches with one wavefront taking a contour's
+// stretches in turn, and takes 0.8 + 1.7 ms; what remains is the longest
+// contour's total, one chain of additions.
+static constexpr int kShort = 64;
+
 // One workgroup of 256 threads per contour: the lane-parallel phases use
-// all of them, the sequential sums and walks run on wavefront 0.
+// all of them, the sequential sums and walks run on a lane or a wavefront.
 // RN_COUNT (PLACE = false): geometry, corners, sums, npr; RN_PLACE: the
 // scaling, the walk and the node positions from the count pass's geometry.
 template <bool PLACE>
@@ -259,45 +329,48 @@ __global__ void __launch_bounds__(256) renode_kernel(RenodeArgs g) {
   if (c >= g.ncont) return;
   const int n = g.npd[c];
   const int64_t o = g.off_in[c];
-  const int t = threadIdx.x, l = t & 63, nt = blockDim.x;
-  const bool w0 = t < 64;
-  __shared__ double lds_e[64], lds_s[64];
-  __shared__ int s_ncorn, s_first, s_tot;
+  const int t = threadIdx.x, l = t & 63, w = t >> 6, nt = blockDim.x;
+  __shared__ double lds_e[4][kRnBlock], lds_s[PLACE ? 4 : 1][PLACE ? kRnBlock : 1];
+  __shared__ int s_scan[4];
   __shared__ double s_sum;
   if (n <= 0) {
     if (!PLACE && t == 0) g.npr[c] = 0;
     return;
   }
+  int ncorn = 0;
   if (!PLACE) {
     renode_geometry(g, o, n);
-    // corners (d holds the flag): count, first; the total of e
-    // (contours.f90:799-809)
-    if (w0) {
-      int ncorn = 0, first = -1;
-      for (int b0 = 0; b0 < n; b0 += 64) {
-        const uint64_t m = __ballot(b0 + l < n && g.sd[o + b0 + l] != 0.0);
-        if (m && first < 0) first = b0 + __ffsll((unsigned long long)m) - 1;
-        ncorn += __popcll(m);
+    // corners (d holds the flag), in order
+    int2 *const corner = (int2 *)(g.su + o);
+    for (int b0 = 0; b0 < n; b0 += 8 * nt) {
+      int f[8], mine = 0, tot;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int i = b0 + 8 * t + j;
+        f[j] = i < n && g.sd[o + i] != 0.0;
+        mine += f[j];
       }
-      const double sum = seq_sum_e(g.se, o, n, 0, n, lds_e);
-      if (l == 0) {
-        s_ncorn = ncorn;
-        s_first = first;
-        s_sum = sum;
-        g.csum[c] = sum;
-        g.cnc[c] = ncorn;
-        g.cfirst[c] = first;
-      }
+      int at = ncorn + block_excl(mine, s_scan, tot);
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (f[j]) corner[at++].x = b0 + 8 * t + j;
+      ncorn += tot;
+    }
+    // the total of e (contours.f90:799-809)
+    if (w == 0) {
+      const double sum = seq_sum_e(g.se, o, n, 0, n, lds_e[0]);
+      if (l == 0) s_sum = sum;
     }
     __syncthreads();
-  } else if (t == 0) {
-    s_sum = g.csum[c];
-    s_ncorn = g.cnc[c];
-    s_first = g.cfirst[c];
+    if (t == 0) {
+      g.csum[c] = s_sum;
+      g.cnc[c] = ncorn;
+      g.cfirst[c] = ncorn ? corner[0].x : -1;
+    }
+  } else {
+    ncorn = g.cnc[c];
   }
-  if (PLACE) __syncthreads();
-  const int ncorn = s_ncorn, first = s_first;
-  const double sum = s_sum;
+  const double sum = PLACE ? g.csum[c] : s_sum;
   const int npr = nint_d(sum) + 1;
   if (npr < 3) {
     if (!PLACE && t == 0) g.npr[c] = 0;
@@ -312,15 +385,15 @@ __global__ void __launch_bounds__(256) renode_kernel(RenodeArgs g) {
     for (int i = t; i < n; i += nt) g.se[o + i] = fac * g.se[o + i];
     __syncthreads();
     const int64_t oo = g.off_out[c];
-    const int start = ncorn == 0 ? 0 : first;
-    if (w0) {
+    const int start = ncorn == 0 ? 0 : g.cfirst[c];
+    if (w == 0) {
       if (l == 0) {
         g.xr[oo] = g.xd[o + start];
         g.yr[oo] = g.yd[o + start];
       }
       // ncorn = 0 walks i = 1, 2, ...; ncorn = 1 starts at the corner and
       // wraps (contours.f90:826-868)
-      walk_nodes(g, o, n, start, n, npr - 1, oo, lds_e, lds_s);
+      walk_nodes(g, o, n, start, n, n, npr - 1, oo, lds_e[0], lds_s[0]);
     }
     __syncthreads();
     for (int im = 1 + t; im < npr; im += nt) {
@@ -332,61 +405,106 @@ __global__ void __launch_bounds__(256) renode_kernel(RenodeArgs g) {
     return;
   }
   // several corners: renode each stretch between consecutive corners
-  // (contours.f90:873-929); wavefront 0 does the sums, scalings and walks.
-  if (w0) {
-    const int64_t oo = PLACE ? g.off_out[c] : 0;
-    int tot = 0;
-    int ibeg = first;
-    for (int kk = 0; kk < ncorn; kk++) {
-      // next corner after ibeg (wrapping to the first one at the end)
-      int iend;
-      if (kk == ncorn - 1) {
-        iend = first;
-      } else {
-        int j = ibeg + 1;
-        for (;;) {
-          const int jb = j & ~63;
-          const uint64_t m = __ballot(jb + l >= j && jb + l < n && g.sd[o + jb + l] != 0.0);
-          if (m) {
-            j = jb + __ffsll((unsigned long long)m) - 1;
-            break;
-          }
-          j = jb + 64;
-        }
-        iend = j;
-      }
-      // sum over the stretch ibeg .. iend (exclusive), with next() wrapping
-      const int len = iend > ibeg ? iend - ibeg : iend + n - ibeg;
-      const double sm = seq_sum_e(g.se, o, n, ibeg, len, lds_e);
-      if (sm > g.small) {
-        const int npseg = nint_d(sm) + 1;
-        if (PLACE) {
-          const double fac = (double)npseg / sm;
-          for (int q0 = l; q0 < len; q0 += 64) {
-            const int q = ibeg + q0 < n ? ibeg + q0 : ibeg + q0 - n;
-            g.se[o + q] = fac * g.se[o + q];
-          }
-          __threadfence();  // the walk reads the scaled values (other lanes' stores)
-          if (l == 0) {
-            g.xr[oo + tot] = g.xd[o + ibeg];
-            g.yr[oo + tot] = g.yd[o + ibeg];
-            g.wi[oo + tot] = -1;
-          }
-          if (npseg > 1) walk_nodes(g, o, n, ibeg, n, npseg - 1, oo + tot, lds_e, lds_s);
-        }
-        tot += npseg;
-      }
-      ibeg = iend;
-    }
-    if (l == 0) s_tot = tot;
-  }
-  __syncthreads();
+  // (contours.f90:873-929)
+  const Stretches st(g, o, n, ncorn);
   if (!PLACE) {
-    if (t == 0) g.npr[c] = s_tot;
+    // sums over the stretches (next() wraps)
+    int mine = 0;
+    auto keep = [&](int k, double sm) {
+      const int np = sm > g.small ? nint_d(sm) + 1 : 0;
+      st.sum[k] = sm;
+      st.u[k].y = np;
+      mine += np;
+    };
+    for (int k = t; k < ncorn; k += nt) {
+      const int len = st.len(k);
+      if (len > kShort) continue;
+      const int ib = st.beg(k);
+      double sm = 0.0;
+      for (int q = 0; q < len; q += 8) {
+        double e[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) e[j] = e_at(g.se, o, n, ib, q + j < len ? q + j : q);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (q + j < len) sm = sm + e[j];
+      }
+      keep(k, sm);
+    }
+    for (int k = w; k < ncorn; k += 4) {
+      const int len = st.len(k);
+      if (len <= kShort) continue;
+      const double sm = seq_sum_e(g.se, o, n, st.beg(k), len, lds_e[w]);
+      if (l == 0) keep(k, sm);
+    }
+    int tot;
+    block_excl(mine, s_scan, tot);
+    if (t == 0) g.npr[c] = tot;
     return;
   }
   const int64_t oo = g.off_out[c];
-  const int tot = s_tot;
+  // each stretch's first slot, in place of its node count
+  int tot = 0;
+  for (int k0 = 0; k0 < ncorn; k0 += nt) {
+    const int k = k0 + t, np = k < ncorn ? st.u[k].y : 0;
+    int add;
+    const int at = tot + block_excl(np, s_scan, add);
+    if (k < ncorn) st.u[k].y = np ? at : -1;
+    tot += add;
+  }
+  __syncthreads();
+  for (int k = t; k < ncorn; k += nt) {
+    const int at = st.u[k].y, ib = st.beg(k), len = st.len(k);
+    if (at < 0) continue;
+    g.xr[oo + at] = g.xd[o + ib];
+    g.yr[oo + at] = g.yd[o + ib];
+    g.wi[oo + at] = -1;
+    if (len > kShort) continue;
+    const double sm = st.sum[k];
+    const int np = nint_d(sm) + 1;
+    const double fac = (double)np / sm;
+    double acc = 0.0;
+    int slot = at;  // the last one written
+    for (int q = 0; q < len; q += 8) {
+      double e[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) e[j] = e_at(g.se, o, n, ib, q + j < len ? q + j : q);
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (q + j < len) {
+          int i = ib + q + j;
+          if (i >= n) i -= n;
+          const double ei = fac * e[j], sj = acc + ei;
+          g.se[o + i] = ei;
+          acc = __builtin_amdgcn_fract(sj);
+          const int kn = (int)floor(sj);
+          for (int r = 1; r <= kn && slot + 1 < at + np; r++) {
+            slot++;
+            g.wi[oo + slot] = i;
+            g.wacc[oo + slot] = sj - (double)r;
+          }
+        }
+    }
+    // (never reached, as in walk_nodes)
+    for (slot++; slot < at + np; slot++) {
+      g.wi[oo + slot] = ib;
+      g.wacc[oo + slot] = 0.0;
+    }
+  }
+  for (int k = w; k < ncorn; k += 4) {
+    const int at = st.u[k].y, ib = st.beg(k), len = st.len(k);
+    if (at < 0 || len <= kShort) continue;
+    const double sm = st.sum[k];
+    const int np = nint_d(sm) + 1;
+    const double fac = (double)np / sm;
+    for (int q0 = l; q0 < len; q0 += 64) {
+      const int q = ib + q0 < n ? ib + q0 : ib + q0 - n;
+      g.se[o + q] = fac * g.se[o + q];
+    }
+    __threadfence_block();  // the walk reads the scaled values (other lanes' stores)
+    if (np > 1) walk_nodes(g, o, n, ib, len, len, np - 1, oo + at, lds_e[w], lds_s[w]);
+  }
+  __syncthreads();
   for (int im = t; im < tot; im += nt) {
     const int i = g.wi[oo + im];
     if (i < 0) continue;  // corner copied above

@@ -246,6 +246,41 @@ def test_renode_bitwise(ng, hyd_cache):
     assert bits_equal(a[0], b[0]) and bits_equal(a[1], b[1])
 
 
+# stretches between corners at the edges of what a lane and a wavefront take
+# (64 nodes) and of a block of the chain (256), corners beyond one pass of
+# their list (2048), no corner and one corner
+@pytest.mark.parametrize("stretches", [[64, 65], [1, 2, 3, 63, 64, 65, 128, 255, 256, 257, 511, 513],
+                                       [1] * 5000, [2, 70] * 30, [3000, 1], [700], []])
+def test_renode_stretches_bitwise(stretches, hyd_cache):
+    from oracle.hyo import Oracle
+    h, o = hyd_cache(64), Oracle(64)
+    nc = len(stretches)
+    if nc > 1:   # a star with alternating radii: every vertex is a corner
+        if nc % 2:
+            stretches, nc = stretches + [5], nc + 1
+        th = 2 * np.pi * np.arange(nc) / nc
+        r = np.where(np.arange(nc) % 2 == 0, 2.5, 0.5)
+        vx, vy = r * np.cos(th), r * np.sin(th)
+        if nc == 2:
+            vy = vy + [0.0, 0.3]
+        x, y = [], []
+        for k, m in enumerate(stretches):
+            f = np.arange(m) / m
+            k1 = (k + 1) % nc
+            bow = 0.02 * np.sin(np.pi * f) * (1 if m > 8 else 0)
+            x.append(vx[k] + f * (vx[k1] - vx[k]) - bow * (vy[k1] - vy[k]))
+            y.append(vy[k] + f * (vy[k1] - vy[k]) + bow * (vx[k1] - vx[k]))
+        x, y = np.concatenate(x), np.concatenate(y)
+    else:        # a circle, or a drop with its tip at the first node
+        n = stretches[0] if nc else 4099
+        th = 2 * np.pi * np.arange(n) / n
+        r = 1.0 - (0.8 * np.exp(-th * 3) + 0.8 * np.exp(-(2 * np.pi - th) * 3) if nc else 0.0)
+        x, y = r * np.cos(th), r * np.sin(th)
+    a, b = h.renode(x, y, cap=1 << 20), o.renode(x, y, cap=1 << 20)
+    assert len(a[0]) == len(b[0])
+    assert bits_equal(a[0], b[0]) and bits_equal(a[1], b[1])
+
+
 @pytest.mark.parametrize("ng", NGS)
 def test_recontour_from_field_bitwise(ng):
     """congen from the initial field: contour count, node count, topology and
