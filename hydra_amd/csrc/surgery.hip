@@ -188,19 +188,84 @@ struct SgState {
   int32_t *nhit;
 };
 
-__device__ void mark_boxes(const SgState &s, int j, int lv, const SgLevels &L) {
-  const int nbx = L.nbx[lv], nby = L.nby[lv];
-  const int32_t *r = s.rng + 4 * (j - 1);
-  for (int mbx = r[0]; mbx <= r[1]; mbx++) {
-    const int mmbx = mbx % nbx;
-    for (int mby = r[2]; mby <= r[3]; mby++) {
-      const int mb = nby * mmbx + mby % nby + 1;
-      s.boxdirty[L.boxbase[lv] + mb - 1] = 1;
-    }
+// The reconnection of contours.f90:569-608 between node i (successor of ib)
+// and the segment listed by slot value isb (its successor is), with what
+// sg_test left; returns the node's new partner.  Everything it reads is
+// loaded at once -- the four nodes' increments one node to a lane -- and the
+// reference's statements follow in registers (any two of the four may be the
+// same node, the later statement then sees the earlier one's value); storing
+// in between makes every load wait for the store before it, which took some
+// thirty trips to memory for a reconnection (a developed ng=256 flow: the
+// replay 2.25 -> 1.21 ms).
+__device__ int sg_reconnect(const SgState &s, int ib, int i, int isb, int is, double delx,
+                            double dely, double aa, int lv, const SgLevels &L, const SgConst &k) {
+  const int l = threadIdx.x & 63;
+  const int nis = s.nextq[is - 1];
+  const double sdx = s.dx[is - 1], sdy = s.dy[is - 1], sds = s.dsq[is - 1];
+  double dxa, dya;
+  if (sds + 2.0 * aa < 0.0) {
+    dxa = 0.5 * (delx + sdx);
+    dya = 0.5 * (dely + sdy);
+    isb = is;
+    is = nis;
+  } else {
+    dxa = 0.5 * delx;
+    dya = 0.5 * dely;
   }
+  const int A = i, B = isb, C = is, D = ib;
+  const int r = l & 3, own = r == 0 ? A : r == 1 ? B : r == 2 ? C : D;
+  const double mdx = s.dx[own - 1], mdy = s.dy[own - 1];
+  const double xi = s.x[A - 1], yi = s.y[A - 1];
+  const int prB = s.prev[B - 1], prD = s.prev[D - 1];
+  const double xn = k.oms * wrp(xi + dxa, k.ellx, k.hlxi);
+  const double yn = k.oms * wrp(yi + dya, k.elly, k.hlyi);
+  double d[2][4];
+  for (int v = 0; v < 2; v++) {
+    const double m = v ? mdy : mdx, da = v ? dya : dxa;
+    const double a0 = __shfl(m, 0), b0 = __shfl(m, 1), c0 = __shfl(m, 2), d0 = __shfl(m, 3);
+    d[v][0] = a0 - da;
+    d[v][1] = (B == A ? d[v][0] : b0) - da;
+    d[v][2] = (C == B ? d[v][1] : C == A ? d[v][0] : c0) + da;
+    d[v][3] = (D == C ? d[v][2] : D == B ? d[v][1] : D == A ? d[v][0] : d0) + da;
+  }
+  // the last statement about a node stands
+  const bool last = r == 0 ? A != B && A != C && A != D : r == 1 ? B != C && B != D : r == 3 || C != D;
+  if (l < 4) {
+    if (last) {
+      const double dx = r == 0 ? d[0][0] : r == 1 ? d[0][1] : r == 2 ? d[0][2] : d[0][3];
+      const double dy = r == 0 ? d[1][0] : r == 1 ? d[1][1] : r == 2 ? d[1][2] : d[1][3];
+      s.dx[own - 1] = dx;
+      s.dy[own - 1] = dy;
+      s.dsq[own - 1] = dx * dx + dy * dy;
+    }
+    if (r == 0 || r == 2) {
+      s.x[own - 1] = xn;
+      s.y[own - 1] = yn;
+      s.posdirty[own - 1] = 1;
+      if (r == 2 || A != C) s.prev[own - 1] = r == 0 ? B : D;
+    } else {
+      if (r == 3 || B != D) s.nextq[own - 1] = r == 1 ? A : C;
+      s.nextdirty[own - 1] = 1;
+    }
+    if (l == 0) atomicAdd(s.nhit, 1);
+  }
+  // the boxes that later tests find the changed segments in: 16 lanes each
+  const int g = l >> 4;
+  const int pB = B == C ? D : B == A ? B : prB, pD = D == C ? D : D == A ? B : prD;
+  const int j = g == 0 ? B : g == 1 ? D : g == 2 ? pB : pD;
+  const int nbx = L.nbx[lv], nby = L.nby[lv];
+  const int32_t *q = s.rng + 4 * (int64_t)(j - 1);
+  const int x1 = q[0], x2 = q[1], y1 = q[2], y2 = q[3], ny = y2 - y1 + 1;
+  const int cnt = x2 >= x1 && ny > 0 ? (x2 - x1 + 1) * ny : 0;
+  for (int t = l & 15; t < cnt; t += 16) {
+    const int mbx = x1 + t / ny, mby = y1 + t % ny;
+    s.boxdirty[L.boxbase[lv] + nby * (mbx % nbx) + mby % nby] = 1;
+  }
+  return C;
 }
 
-// 4. ordered replay, one wavefront per level.
+// 4. ordered replay, one wavefront per level.  Bound by latency: the busiest
+// level's reconnections are one serial chain of trips to memory.
 __global__ void __launch_bounds__(64) sg_replay(SgState s, SgLevels L, SgConst k, int nlev) {
   const int lv = blockIdx.x;
   if (lv >= nlev) return;
@@ -229,69 +294,23 @@ __global__ void __launch_bounds__(64) sg_replay(SgState s, SgLevels L, SgConst k
       int64_t kk = k1;
       while (kk <= k2) {
         const int64_t slot = kk + l;
-        int hl = 0;
+        int hl = 0, isb = 1;
         double delx = 0.0, dely = 0.0, aa = 0.0;
-        if (slot <= k2)
-          hl = sg_test(s.x, s.y, s.nextq, s.dx, s.dy, s.dsq, ibb, i, s.node[slot], k, delx, dely,
-                       aa);
+        if (slot <= k2) {
+          isb = s.node[slot];
+          hl = sg_test(s.x, s.y, s.nextq, s.dx, s.dy, s.dsq, ibb, i, isb, k, delx, dely, aa);
+        }
         const uint64_t hm = __ballot(hl != 0);
         if (hm == 0) {
           kk += 64;
           continue;
         }
         const int h = __ffsll((unsigned long long)hm) - 1;
-        // reconnection (contours.f90:569-608), done by lane h
-        int inew = 0;
-        if (l == h) {
-          int isb = s.node[kk + h];
-          int is = s.nextq[isb - 1];
-          double dxa, dya;
-          if (s.dsq[is - 1] + 2.0 * aa < 0.0) {
-            dxa = 0.5 * (delx + s.dx[is - 1]);
-            dya = 0.5 * (dely + s.dy[is - 1]);
-            isb = is;
-            is = s.nextq[is - 1];
-          } else {
-            dxa = 0.5 * delx;
-            dya = 0.5 * dely;
-          }
-          double xx = s.x[i - 1] + dxa;
-          s.x[i - 1] = k.oms * wrp(xx, k.ellx, k.hlxi);
-          double yy = s.y[i - 1] + dya;
-          s.y[i - 1] = k.oms * wrp(yy, k.elly, k.hlyi);
-          s.dx[i - 1] = s.dx[i - 1] - dxa;
-          s.dy[i - 1] = s.dy[i - 1] - dya;
-          s.dsq[i - 1] = s.dx[i - 1] * s.dx[i - 1] + s.dy[i - 1] * s.dy[i - 1];
-          s.nextq[isb - 1] = i;
-          s.dx[isb - 1] = s.dx[isb - 1] - dxa;
-          s.dy[isb - 1] = s.dy[isb - 1] - dya;
-          s.dsq[isb - 1] = s.dx[isb - 1] * s.dx[isb - 1] + s.dy[isb - 1] * s.dy[isb - 1];
-          s.x[is - 1] = s.x[i - 1];
-          s.y[is - 1] = s.y[i - 1];
-          s.dx[is - 1] = s.dx[is - 1] + dxa;
-          s.dy[is - 1] = s.dy[is - 1] + dya;
-          s.dsq[is - 1] = s.dx[is - 1] * s.dx[is - 1] + s.dy[is - 1] * s.dy[is - 1];
-          s.nextq[ibb - 1] = is;
-          s.dx[ibb - 1] = s.dx[ibb - 1] + dxa;
-          s.dy[ibb - 1] = s.dy[ibb - 1] + dya;
-          s.dsq[ibb - 1] = s.dx[ibb - 1] * s.dx[ibb - 1] + s.dy[ibb - 1] * s.dy[ibb - 1];
-          // what later tests read and this reconnection touched
-          s.nextdirty[isb - 1] = 1;
-          s.nextdirty[ibb - 1] = 1;
-          s.posdirty[i - 1] = 1;
-          s.posdirty[is - 1] = 1;
-          s.prev[i - 1] = isb;
-          s.prev[is - 1] = ibb;
-          mark_boxes(s, isb, lv, L);
-          mark_boxes(s, ibb, lv, L);
-          mark_boxes(s, s.prev[isb - 1], lv, L);
-          mark_boxes(s, s.prev[ibb - 1], lv, L);
-          atomicAdd(s.nhit, 1);
-          inew = is;
-          __threadfence();
-        }
-        i = __shfl(inew, h);
-        __threadfence();
+        isb = __shfl(isb, h);
+        i = sg_reconnect(s, ibb, i, isb, s.nextq[isb - 1], __shfl(delx, h), __shfl(dely, h),
+                         __shfl(aa, h), lv, L, k);
+        // a level's nodes and boxes are its wavefront's alone
+        __threadfence_block();
         if (i == ibb) break;
         kk = kk + h + 1;
       }

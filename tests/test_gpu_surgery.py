@@ -35,6 +35,28 @@ def test_surgery_tangle_bitwise(seed, ncirc, rmin, rmax):
     h.close()
 
 
+# polygons of 4 to 18 nodes crowded so that a reconnection's four nodes
+# coincide in pairs (a segment next to the node, contours of three nodes left)
+@pytest.mark.parametrize("ncirc,rmin,rmax", [(900, 0.3, 0.8), (700, 0.5, 2.0)])
+def test_surgery_of_small_contours_bitwise(ncirc, rmin, rmax):
+    from hydra_amd import Hydra
+    from oracle.hyo import Oracle
+    ng = 32
+    o = Oracle(ng)
+    dm = o.getd("dm")
+    c = tangle_contours(dm, np.random.default_rng(ncirc), ncirc, levels=(1, 2), rmin=rmin * dm,
+                        rmax=rmax * dm)
+    c["x"], c["y"] = 0.25 * c["x"], 0.25 * c["y"]   # a sixteenth of the area
+    o.set_contours(c)
+    h = Hydra(ng)
+    h.set_field(np.zeros((ng, ng)))
+    h.set_contours(c)
+    o.surgery()
+    h.surgery()
+    _same_contours(h.contours(), o.contours())
+    h.close()
+
+
 @pytest.mark.parametrize("ng", [32, 64])
 def test_surgery_after_evolution_bitwise(ng):
     """Surgery on contours advected until twist exceeds 2.5 (the state in
