@@ -1447,10 +1447,10 @@ int hyd_run_batch(hyd_ctx **hs, int32_t n, int32_t nsteps) {
         HYD_HIP(hipMemcpyAsync(c.dsc, c.hsc, sizeof(Scalars), hipMemcpyHostToDevice, c.s));
       }
       tstart[i] = c.hsc->t;
-      if (c.p.precision == 1)
-        HYD_CHECK(advance_mixed_graph(c));
-      else
-        HYD_CHECK(advance(c));
+      c.crowded = n >= 4;
+      const int rc = c.p.precision == 1 ? advance_mixed_graph(c) : advance(c);
+      c.crowded = false;
+      HYD_CHECK(rc);
       HYD_HIP(hipMemcpyAsync(c.hsc, c.dsc, sizeof(Scalars), hipMemcpyDeviceToHost, c.s));
       stepped[i] = 1;
     }

@@ -226,6 +226,7 @@ struct Ctx {
   double *diag_out = nullptr;    // 8 scratch results
   hipStream_t s2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  bool crowded = false;  // a step among several flows' (run_batch)
   // The clearing that ends a sweep (counters zeroed) may be left to the caller (defer_clear), who runs it
   // later on either stream (sweep_clear); the next sweep first waits for it
   // (sweep_clear_join), or runs it itself if nobody has.

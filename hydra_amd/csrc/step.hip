@@ -626,6 +626,16 @@ __global__ void k_tick(Scalars *sc) {
 // needs only the moved nodes); the field part of stage k+1's inversion waits
 // for the update.  Every kernel sees the same inputs as in the reference's
 // serial order.
+// Two cases run it all on the main stream.  Up to ng=64 the kernels are too
+// short to be worth the events between the streams (two streams -> one: ten
+// steps of ng=32 4697 -> 4081 us, four of ng=64 5726 -> 5527; from ng=256 on
+// two are as fast or faster, ng=512 18867 against 18372 us for twenty).  And
+// from four flows at once the flows overlap each other, and a second stream
+// each shares the same four hardware queues (eight flows of ng=128 to 512:
+// 19.2 -> 17.2 ms).
+static constexpr int kOneStreamNg = 64;
+static bool one_stream(const Ctx &c) { return c.c.nx <= kOneStreamNg || c.crowded; }
+
 // Runs fn on the second stream (c.s points at it meanwhile, so that every
 // launch and timer inside goes there).
 template <class Fn>
@@ -634,7 +644,7 @@ static int on_s2(Ctx &c, Fn fn) {
   // with per-launch timing on, everything stays on the main stream, in
   // program order (a valid order of the same work), so that each timed
   // launch runs alone
-  c.s = c.timing ? main : c.s2;
+  c.s = c.timing || one_stream(c) ? main : c.s2;
   const int rc = fn();
   c.s = main;
   return rc;
@@ -652,6 +662,7 @@ static int contour_grid_deferred(Ctx &c, bool reset, hipEvent_t wait) {
 // Fork: the second stream continues after everything enqueued so far on
 // the main stream.
 static int fork_s2(Ctx &c) {
+  if (one_stream(c)) return HYD_OK;
   HYD_HIP(hipEventRecord(c.ev_fork, c.s));
   HYD_HIP(hipStreamWaitEvent(c.s2, c.ev_fork, 0));
   return HYD_OK;

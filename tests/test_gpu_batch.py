@@ -43,6 +43,30 @@ def test_batch_equals_single_runs():
         h.close()
 
 
+# grids that use two streams alone and one among four flows, going from one
+# way to the other and back
+@pytest.mark.parametrize("prec", [0, 1])
+def test_crowded_batch_equals_single_runs(prec):
+    from hydra_amd import Hydra
+    a = [_make(128, 20 + i, prec) for i in range(4)]
+    b = [_make(128, 20 + i, prec) for i in range(4)]
+    for h in a:
+        h.run(9)
+    for h in b:
+        h.run(3)
+    Hydra.run_batch(b, 3)
+    for h in b:
+        h.run(3)
+    for h, g in zip(a, b):
+        (c1, qs1, t1), (c2, qs2, t2) = _state(h), _state(g)
+        for k in ("x", "y", "nextq", "i1q", "i2q", "npq", "indq"):
+            assert np.array_equal(c1[k], c2[k]), k
+        assert np.array_equal(qs1, qs2)
+        assert t1 == t2
+        h.close()
+        g.close()
+
+
 def test_batch_rejects_repeated_context():
     from hydra_amd import Hydra, HydraError
     h = _make(32, 3, 0)
