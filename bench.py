@@ -79,9 +79,9 @@ def pmc_summary(fetch_dir, write_dir, ng, out_json):
     """HBM traffic of the FFT kernels from two rocprofv3 --pmc runs
     (FETCH_SIZE, WRITE_SIZE; KiB per dispatch), each scaled by the same
     counter on the calibration copy, as bytes per algorithmic byte
-    (aggregated over the batch variants VT).  A dispatch's algorithmic bytes
+    (aggregated over the batch variants V).  A dispatch's algorithmic bytes
     are (sizeof in + sizeof out) x n x vectors; the vectors are its blocks
-    (grid size / workgroup size, both in the record) times the VT in the
+    (grid size / workgroup size, both in the record) times the V in the
     kernel's name."""
     import csv
     import glob
@@ -105,12 +105,12 @@ def pmc_summary(fetch_dir, write_dir, ng, out_json):
             if "k_copy_calib" in k:
                 copy.append(v)
                 continue
-            m = re.search(r"fft_kernel<(\d+), (true|false), (\w+), (\w+), (\w+), (\d+)>", k)
+            m = re.search(r"fft_kernel<(\d+), (true|false), (\w+), (\w+), (\w+), (\d+), \w+>", k)
             if not m:
                 continue
             n = int(m.group(1))
             ti, to = size[m.group(3)], size[m.group(5)]
-            # its blocks, VT vectors each (all fields of the launch)
+            # its blocks, V vectors each (all fields of the launch)
             vectors = int(row["Grid_Size"]) // int(row["Workgroup_Size"]) * int(m.group(6))
             alg = (ti + to) * n * vectors
             key = "fft_kernel<%s, %s, %s, %s, %s>" % m.group(1, 2, 3, 4, 5)
