@@ -230,7 +230,6 @@ static int create(const hyd_params *p, hyd_ctx **out) {
   TRY(dalloc(&c->dsum, 8));
   TRY(dalloc(&c->amax, 2048));
   TRY(dalloc(&c->seq_tot, N / 64 + 64));
-  c->seq_cap = (std::max<int64_t>(N, 4 * N) + 255) / 256 + 64;
   {
     void *w = nullptr;
     if (hipMalloc(&w, seqsum_work_bytes(4 * N)) != hipSuccess) {

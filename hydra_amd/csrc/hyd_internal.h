@@ -236,8 +236,8 @@ struct Ctx {
   hipEvent_t ev_cleared = nullptr;
   // work that the plain step starts on its second stream once the contour
   // grid's node and sweep kernels are queued (so that those run alone on
-  // the GPU and the second stream's work overlaps the single-workgroup
-  // sequential mean instead); con2grid runs and clears it
+  // the GPU and the second stream's work overlaps the few-workgroup
+  // exact mean instead); con2grid runs and clears it
   std::function<int()> after_sweep;
   // work that the plain step queues just before a contour grid is combined
   // with the fields

@@ -627,7 +627,7 @@ __global__ void k_tick(Scalars *sc) {
 // for the update.  Every kernel sees the same inputs as in the reference's
 // serial order.
 // Two cases run it all on the main stream.  Up to ng=64 the kernels are too
-// short to be worth the events between the streams (two streams -> one: ten
+// short to be worth the events between the streams (two streams -> one: eight
 // steps of ng=32 4697 -> 4081 us, four of ng=64 5726 -> 5527; from ng=256 on
 // two are as fast or faster, ng=512 18867 against 18372 us for twenty).  And
 // from four flows at once the flows overlap each other, and a second stream
