@@ -656,8 +656,10 @@ __global__ void __launch_bounds__(64) seq_fold(const SeqTab *__restrict__ in, in
   const bool first = blockIdx.x == 0;  // starts at the sum's beginning
   Walk w = class_start(t[0].g);
   if (first) {
+    // entry 0's exact end, unless it did not fold itself (its c[0] is then
+    // whatever an earlier sum left there)
     w.S = t[0].c[0].e;
-    w.ok = true;
+    w.ok = t[0].M < 0;
   }
   const double s0 = w.S;
   for (int k = first ? 1 : 0; k < m; k++) walk_tab(t[k], w);

@@ -192,6 +192,24 @@ def test_sum_sequential_level_edges_bitwise(n, hyd_2048):
         assert (np.isnan(got) and np.isnan(want)) or got == want
 
 
+def test_sum_sequential_unfolded_start_after_another_sum(hyd_2048):
+    """A first group of segments that does not fold (a run up to 1e300 and
+    back in its second segment) under two folded levels, in a work area that
+    another sum of the same length, alike from the third segment on, has
+    filled: nothing of that sum may be taken for this one's start."""
+    import ctypes as C
+    from oracle.hyo import lib
+    ol = lib()
+    ol.hyo_sum_seq.restype = C.c_double
+    ol.hyo_sum_seq.argtypes = [np.ctypeslib.ndpointer(dtype=np.float64), C.c_int64]
+    n = (1 << 22) + 8 * 4096
+    a = np.full(n, 0.75)
+    b = a.copy()
+    b[5000:5003] = [1e300, -1e300, 2.25]
+    for x in (a, b, a):
+        assert hyd_2048.sum_sequential(x) == ol.hyo_sum_seq(x, n)
+
+
 @pytest.mark.parametrize("ng", [32, 64])
 def test_advance_bitwise(ng):
     """Several RK4 steps of the device-resident state, every field and node
