@@ -115,6 +115,7 @@ def lib():
         L.hyd_save_counters.argtypes = [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
         L.hyd_run_batch.argtypes = [C.POINTER(C.c_void_p), C.c_int32, C.c_int32]
         L.hyd_get_tuning.argtypes = [C.c_void_p, _I]
+        L.hyd_step_graphs.argtypes = [C.c_void_p, _I]
         L.hyd_copy_calibration.argtypes = [C.c_void_p, C.c_int64]
         L.hyd_event_overhead.argtypes = [C.c_void_p, C.c_int32, C.POINTER(C.c_double)]
         L.hyd_set_timing.argtypes = [C.c_void_p, C.c_int32]
@@ -495,6 +496,13 @@ class Hydra:
         """FFT batch per layout class picked by the autotuner at init."""
         v = np.zeros(4, dtype=np.int32)
         _check(self.L.hyd_get_tuning(self.h, v))
+        return v.tolist()
+
+    def step_graphs(self):
+        """Node counts of the mixed step's captured graphs (on two streams,
+        on one); -1: none."""
+        v = np.zeros(2, dtype=np.int32)
+        _check(self.L.hyd_step_graphs(self.h, v))
         return v.tolist()
 
     def copy_calibration(self, nbytes):

@@ -118,8 +118,10 @@ static void free_ctx(Ctx *c) {
     hipEventDestroy(r.a);
     hipEventDestroy(r.b);
   }
-  if (c->step_graph) hipGraphExecDestroy(c->step_graph);
-  if (c->step_graph_tail) hipGraphExecDestroy(c->step_graph_tail);
+  for (const Ctx::StepGraph &g : c->graphs) {
+    if (g.head) hipGraphExecDestroy(g.head);
+    if (g.tail) hipGraphExecDestroy(g.tail);
+  }
   if (c->s2) hipStreamDestroy(c->s2);
   if (c->s) hipStreamDestroy(c->s);
   delete c;
@@ -515,7 +517,7 @@ int hyd_set_correction(hyd_ctx *h, hyd_cnn *net, double su, double sq, double sd
   c.net_su = su;
   c.net_sq = sq;
   c.net_sd = sd;
-  c.graph_nptq = -1;  // the captured step changes
+  c.drop_graphs();  // the captured step changes
   return HYD_OK;
 }
 
@@ -985,7 +987,7 @@ int hyd_sum_sequential(hyd_ctx *h, const double *a, int64_t n, double *sum) {
 
 int hyd_set_field(hyd_ctx *h, const double *qq, double t0) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   if (c.c.beffect) {
     set_error("beta != 0 is not supported by the device step");
     return HYD_EARG;
@@ -1015,7 +1017,7 @@ int hyd_set_contours(hyd_ctx *h, int32_t nptq, int32_t nq, const double *xq, con
                      const int32_t *nextq, const int32_t *i1q, const int32_t *i2q,
                      const int32_t *npq, const int32_t *indq, double qjump) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   if (nptq < 0 || nptq > c.cap || nq < 0) {
     set_error("set_contours: counts outside capacity");
     return HYD_ECAPACITY;
@@ -1093,7 +1095,7 @@ int hyd_get_field(hyd_ctx *h, int32_t id, double *out) {
 
 int hyd_put_field(hyd_ctx *h, int32_t id, const double *in) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   double *f = field_ptr(c, id);
   if (!f) {
     set_error("unknown field id");
@@ -1124,7 +1126,7 @@ int hyd_get_scalar(hyd_ctx *h, int32_t id, double *out) {
 
 int hyd_set_scalar(hyd_ctx *h, int32_t id, double val) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // the captured step holds scalars (qjump) as launch arguments
+  c.drop_graphs();  // the captured step holds scalars (qjump) as launch arguments
   HYD_HIP(hipMemcpyAsync(c.hsc, c.dsc, sizeof(Scalars), hipMemcpyDeviceToHost, c.s));
   HYD_HIP(hipStreamSynchronize(c.s));
   double *v = scalar_slot(*c.hsc, id);
@@ -1161,7 +1163,7 @@ static int advect_start(Ctx &c) {
 
 int hyd_evolution_init(hyd_ctx *h) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   if (!c.have_field) {
     set_error("evolution_init before set_field");
     return HYD_ESTATE;
@@ -1172,7 +1174,7 @@ int hyd_evolution_init(hyd_ctx *h) {
 
 int hyd_prepare(hyd_ctx *h) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   HYD_CHECK(prepare(c));
   c.phase = 0;
   return c2g_status(c);
@@ -1180,7 +1182,7 @@ int hyd_prepare(hyd_ctx *h) {
 
 int hyd_recontour(hyd_ctx *h) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   if (!c.have_field) {
     set_error("recontour before set_field");
     return HYD_ESTATE;
@@ -1248,27 +1250,29 @@ static int capture_graph(Ctx &c, int (*part)(Ctx &), hipGraphExec_t *out) {
 // The mixed-precision step has no host round trip: after one eager call it
 // is captured as two graphs (head and tail) and replayed; the capture is
 // redone whenever the node count changed (surgery, recontouring) and
-// skipped while timing.  With copy_scalars the step's scalars are copied to
+// skipped while timing.  A step alone and one among several flows' run on
+// different streams (one_stream): each way has its own capture.  With copy_scalars the step's scalars are copied to
 // the host mirror between head and tail (ev_sc; sc_pending set).
 static int advance_mixed_graph(Ctx &c, bool copy_scalars = false) {
   c.sweep_clean = false;  // its sweeps leave their counts behind
   c.n_advances += 1;
   c.n_node_updates += c.nptq;
   const bool eager = c.timing || c.mixed_calls++ == 0;
-  if (!eager && (!c.step_graph || !c.step_graph_tail || c.graph_nptq != c.nptq)) {
-    HYD_CHECK(capture_graph(c, advance_mixed_head, &c.step_graph));
-    HYD_CHECK(capture_graph(c, advance_mixed_tail, &c.step_graph_tail));
-    c.graph_nptq = c.nptq;
+  Ctx::StepGraph &g = c.graphs[one_stream(c) ? 1 : 0];
+  if (!eager && (!g.head || !g.tail || g.nptq != c.nptq)) {
+    HYD_CHECK(capture_graph(c, advance_mixed_head, &g.head));
+    HYD_CHECK(capture_graph(c, advance_mixed_tail, &g.tail));
+    g.nptq = c.nptq;
   }
   if (eager) HYD_CHECK(advance_mixed_head(c));
-  else HYD_HIP(hipGraphLaunch(c.step_graph, c.s));
+  else HYD_HIP(hipGraphLaunch(g.head, c.s));
   if (copy_scalars) {
     HYD_HIP(hipMemcpyAsync(c.hsc, c.dsc, sizeof(Scalars), hipMemcpyDeviceToHost, c.s));
     HYD_HIP(hipEventRecord(c.ev_sc, c.s));
     c.sc_pending = true;
   }
   if (eager) return advance_mixed_tail(c);
-  HYD_HIP(hipGraphLaunch(c.step_graph_tail, c.s));
+  HYD_HIP(hipGraphLaunch(g.tail, c.s));
   return HYD_OK;
 }
 
@@ -1312,7 +1316,7 @@ int hyd_advance(hyd_ctx *h) {
 
 int hyd_surgery(hyd_ctx *h) {
   Ctx &c = *C(h);
-  c.graph_nptq = -1;  // state changed outside the captured step
+  c.drop_graphs();  // state changed outside the captured step
   HYD_CHECK(timed_surgery(c));
   HYD_HIP(hipStreamSynchronize(c.s));
   return HYD_OK;
@@ -1531,6 +1535,12 @@ int hyd_copy_calibration(hyd_ctx *h, int64_t nbytes) {
 int hyd_get_tuning(hyd_ctx *h, int32_t *v) {
   Ctx &c = *C(h);
   for (int k = 0; k < 4; k++) v[k] = c.fft_v[k];
+  return HYD_OK;
+}
+
+int hyd_step_graphs(hyd_ctx *h, int32_t *nptq) {
+  Ctx &c = *C(h);
+  for (int k = 0; k < 2; k++) nptq[k] = c.graphs[k].nptq;
   return HYD_OK;
 }
 

@@ -247,11 +247,15 @@ struct Ctx {
   int64_t seq_cap = 0;      // chunks it holds
   // work buffers of recontour / renode, allocated on first use
   std::map<std::string, DBuf> cg_bufs;
-  // captured mixed-precision step, head and tail (replayed while the node
-  // count is unchanged)
-  hipGraphExec_t step_graph = nullptr, step_graph_tail = nullptr;
+  // captured mixed-precision step, head and tail, on two streams ([0]) and on
+  // one ([1]); each replayed while the node count is the captured one
+  struct StepGraph {
+    hipGraphExec_t head = nullptr, tail = nullptr;
+    int nptq = -1;
+  };
+  StepGraph graphs[2];
+  void drop_graphs() { graphs[0].nptq = graphs[1].nptq = -1; }
   bool sc_pending = false;  // a mixed step's scalars are on their way to the host (ev_sc)
-  int graph_nptq = -1;
   int mixed_calls = 0;
   // timing
   int timing = 0;  // 0 off, 1 single-kernel ("k:") records only, 2 all records
@@ -281,6 +285,7 @@ int fft_spctop32(Ctx &c, const double *svar, float *rvar, int pre, double post_s
 int con2grid_mixed(Ctx &c, float *qc, bool defer_mean = false);
 int fft_ptospc32_mean(Ctx &c, const float *rvar, const double *mean, double *svar);
 int advance_mixed(Ctx &c);
+bool one_stream(const Ctx &c);  // which of the two ways the next step runs
 int advance_mixed_head(Ctx &c);
 int advance_mixed_tail(Ctx &c);
 int fft_autotune(Ctx &c);

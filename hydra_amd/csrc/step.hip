@@ -634,7 +634,7 @@ __global__ void k_tick(Scalars *sc) {
 // each shares the same four hardware queues (eight flows of ng=128 to 512:
 // 19.2 -> 17.2 ms).
 static constexpr int kOneStreamNg = 64;
-static bool one_stream(const Ctx &c) { return c.c.nx <= kOneStreamNg || c.crowded; }
+bool one_stream(const Ctx &c) { return c.c.nx <= kOneStreamNg || c.crowded; }
 
 // Runs fn on the second stream (c.s points at it meanwhile, so that every
 // launch and timer inside goes there).

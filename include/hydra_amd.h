@@ -302,6 +302,9 @@ int hyd_sync(hyd_ctx *ctx);
    strided->rows, forward strided->strided, reverse strided->strided and
    reverse rows->strided (v[0..3]). */
 int hyd_get_tuning(hyd_ctx *ctx, int32_t *v);
+/* No reference counterpart: the node counts that the mixed step's captured
+   graphs hold, on two streams (nptq[0]) and on one (nptq[1]); -1: none. */
+int hyd_step_graphs(hyd_ctx *ctx, int32_t *nptq);
 /* No reference counterpart (measurement aid): one plain streaming copy
    kernel of nbytes (<= 128 ng^2) read and nbytes written, the reference
    point that scales hardware traffic counters. */

@@ -67,6 +67,22 @@ def test_crowded_batch_equals_single_runs(prec):
         g.close()
 
 
+def test_crowded_batch_has_its_own_graphs():
+    """A mixed flow's captured step runs on two streams alone and on one
+    among four flows: each way replays its own capture."""
+    from hydra_amd import Hydra
+    hs = [_make(128, 20 + i, 1) for i in range(4)]
+    for h in hs:
+        h.run(2)  # one eager step, one captured
+    n = [h.counts()[0] for h in hs]
+    assert [h.step_graphs() for h in hs] == [[k, -1] for k in n]
+    Hydra.run_batch(hs, 1)
+    assert [h.counts()[0] for h in hs] == n
+    assert [h.step_graphs() for h in hs] == [[k, k] for k in n]
+    for h in hs:
+        h.close()
+
+
 def test_batch_rejects_repeated_context():
     from hydra_amd import Hydra, HydraError
     h = _make(32, 3, 0)
