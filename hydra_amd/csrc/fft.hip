@@ -83,39 +83,52 @@ static int fft_launch_t(Ctx &c, int F, const TI *const *in, TO *const *out, int 
 }
 
 // Holds the stream for some 40 us, so that the launches timed after it are
-// all queued before the first one starts: at 3-10 us a pass, launches issued
-// to an idle stream would time the host instead.
+// queued ahead of the GPU: at 3-10 us a pass, launches issued to an idle
+// stream would time the host instead.
 __global__ void fft_tune_hold() {
   for (int i = 0; i < 12; i++) __builtin_amdgcn_s_sleep(127);
 }
 
+// A pair of events for each batch that a class can try.
+static constexpr int kTuneV = 5;  // 1, 2, 4, 8, 16
+static_assert(1 << (kTuneV - 1) == kMaxV, "batches");
+struct TuneEvents {
+  hipEvent_t a[kTuneV] = {}, b[kTuneV] = {};
+};
+
 // The best batch of one layout class: each candidate timed over three
 // rounds that visit the candidates in turn (so that a slow spell of the
-// device does not favour one), keeping its best round.  Every V gives
+// device does not favour one), keeping its best round.  A round is queued
+// whole behind one hold and waited for once (a hold and a wait for each
+// candidate: hyd_init took 12.0 ms instead of 8.3 at ng=128, 21.7 instead of
+// 16.1 at ng=256).  Every V gives
 // bit-identical results (each vector's arithmetic is the same).
 template <class RUN>
-static int fft_tune_class(Ctx &c, int n, int tsize, int &tab, hipEvent_t e0, hipEvent_t e1,
-                          RUN run) {
-  float best[kMaxV + 1];
-  for (int V = 0; V <= kMaxV; V++) best[V] = 1e30f;
-  for (int round = 0; round < 3; round++)
-    for (int V = 1; V <= kMaxV; V *= 2) {
-      if (!fft_v_fits(n, V, tsize) || (V > n && V > 16)) continue;
-      tab = V;
+static int fft_tune_class(Ctx &c, int n, int tsize, int &tab, const TuneEvents &ev, RUN run) {
+  float best[kTuneV];
+  for (float &b : best) b = 1e30f;
+  for (int round = 0; round < 3; round++) {
+    hipLaunchKernelGGL(fft_tune_hold, dim3(1), dim3(64), 0, c.s);
+    for (int k = 0; k < kTuneV; k++) {
+      if (!fft_v_fits(n, 1 << k, tsize)) continue;
+      tab = 1 << k;
       HYD_CHECK(run());
-      hipLaunchKernelGGL(fft_tune_hold, dim3(1), dim3(64), 0, c.s);
-      HYD_HIP(hipEventRecord(e0, c.s));
+      HYD_HIP(hipEventRecord(ev.a[k], c.s));
       for (int r = 0; r < 8; r++) HYD_CHECK(run());
-      HYD_HIP(hipEventRecord(e1, c.s));
-      HYD_HIP(hipEventSynchronize(e1));
-      float ms = 0.0f;
-      HYD_HIP(hipEventElapsedTime(&ms, e0, e1));
-      best[V] = std::min(best[V], ms);
+      HYD_HIP(hipEventRecord(ev.b[k], c.s));
     }
-  int bestV = 1;
-  for (int V = 2; V <= kMaxV; V *= 2)
-    if (best[V] < best[bestV]) bestV = V;
-  tab = bestV;
+    HYD_HIP(hipStreamSynchronize(c.s));
+    for (int k = 0; k < kTuneV; k++) {
+      if (!fft_v_fits(n, 1 << k, tsize)) continue;
+      float ms = 0.0f;
+      HYD_HIP(hipEventElapsedTime(&ms, ev.a[k], ev.b[k]));
+      best[k] = std::min(best[k], ms);
+    }
+  }
+  int bk = 0;
+  for (int k = 1; k < kTuneV; k++)
+    if (best[k] < best[bk]) bk = k;
+  tab = 1 << bk;
   return HYD_OK;
 }
 
@@ -125,7 +138,7 @@ static int fft_tune_class(Ctx &c, int n, int tsize, int &tab, hipEvent_t e0, hip
 // half the grid, so a smaller batch may fill the device better) and
 // four-field ones (fft_v4; outputs in the fine-grid scratch), and for the
 // mixed step's FP32 passes (fft_v32).
-static int fft_tune_all(Ctx &c, hipEvent_t e0, hipEvent_t e1) {
+static int fft_tune_all(Ctx &c, const TuneEvents &ev) {
   const int n = c.c.nx;
   const double post[4] = {1.0, 1.0, 1.0, 1.0};
   for (int F : {2, 1, 4}) {
@@ -133,19 +146,19 @@ static int fft_tune_all(Ctx &c, hipEvent_t e0, hipEvent_t e1) {
     const double *in[4] = {c.wa, c.wc, c.wb, c.wd};
     double *out[4] = {F == 4 ? c.fq : c.wb, F == 4 ? c.fq + c.N : c.wd, c.fq + 2 * c.N,
                       c.fq + 3 * c.N};
-    HYD_CHECK(fft_tune_class(c, n, 8, tab[0], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 8, tab[0], ev, [&]() {
       return fft_launch_t<true, double, double, double, true>(c, F, in, out, n, n, nullptr, nullptr,
                                                               post, c.xtrig);
     }));
-    HYD_CHECK(fft_tune_class(c, n, 8, tab[1], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 8, tab[1], ev, [&]() {
       return fft_launch_t<true, double, double, double, false>(c, F, in, out, n, n, nullptr,
                                                                nullptr, post, c.xtrig);
     }));
-    HYD_CHECK(fft_tune_class(c, n, 8, tab[2], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 8, tab[2], ev, [&]() {
       return fft_launch_t<false, double, double, double, false>(c, F, in, out, n, n, nullptr,
                                                                 nullptr, post, c.ytrig);
     }));
-    HYD_CHECK(fft_tune_class(c, n, 8, tab[3], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 8, tab[3], ev, [&]() {
       return fft_launch_t<false, double, double, double, true>(c, F, in, out, n, n, nullptr,
                                                                nullptr, post, c.ytrig);
     }));
@@ -156,19 +169,19 @@ static int fft_tune_all(Ctx &c, hipEvent_t e0, hipEvent_t e1) {
     const double *ind[2] = {c.wa, c.wc};
     double *outd[2] = {c.wb, c.wd};
     int *tab = c.fft_v32;
-    HYD_CHECK(fft_tune_class(c, n, 4, tab[0], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 4, tab[0], ev, [&]() {
       return fft_launch_t<true, float, float, float, true>(c, 2, in, out, n, n, nullptr, nullptr,
                                                            post, c.xtrig32);
     }));
-    HYD_CHECK(fft_tune_class(c, n, 4, tab[1], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 4, tab[1], ev, [&]() {
       return fft_launch_t<true, float, float, double, false>(c, 2, in, outd, n, n, nullptr, nullptr,
                                                              post, c.xtrig32);
     }));
-    HYD_CHECK(fft_tune_class(c, n, 4, tab[2], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 4, tab[2], ev, [&]() {
       return fft_launch_t<false, double, float, float, false>(c, 2, ind, out, n, n, nullptr,
                                                               nullptr, post, c.ytrig32);
     }));
-    HYD_CHECK(fft_tune_class(c, n, 4, tab[3], e0, e1, [&]() {
+    HYD_CHECK(fft_tune_class(c, n, 4, tab[3], ev, [&]() {
       return fft_launch_t<false, float, float, float, true>(c, 2, in, out, n, n, nullptr, nullptr,
                                                             post, c.ytrig32);
     }));
@@ -177,12 +190,16 @@ static int fft_tune_all(Ctx &c, hipEvent_t e0, hipEvent_t e1) {
 }
 
 int fft_autotune(Ctx &c) {
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  int rc = HYD_EHIP;
-  if (hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess)
-    rc = fft_tune_all(c, e0, e1);
-  if (e0) hipEventDestroy(e0);
-  if (e1) hipEventDestroy(e1);
+  TuneEvents ev;
+  int rc = HYD_OK;
+  for (int k = 0; k < kTuneV; k++)
+    if (hipEventCreate(&ev.a[k]) != hipSuccess || hipEventCreate(&ev.b[k]) != hipSuccess)
+      rc = HYD_EHIP;
+  if (rc == HYD_OK) rc = fft_tune_all(c, ev);
+  for (int k = 0; k < kTuneV; k++) {
+    if (ev.a[k]) hipEventDestroy(ev.a[k]);
+    if (ev.b[k]) hipEventDestroy(ev.b[k]);
+  }
   if (rc != HYD_OK) set_error("fft autotuning failed");
   return rc;
 }
