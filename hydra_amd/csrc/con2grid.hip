@@ -371,10 +371,12 @@ __device__ __forceinline__ void c2g_wave_sync() {
 // each bucket in memory, 431 us with those lanes spread over the GPU, 34 us
 // so; ng=256, 300 steps in: 1754, 346 and 65 us.
 static constexpr int kWaveSort = 512;
-__device__ double bucket_sums(const Buckets &b, int nb, double qjump, int32_t *lds) {
+__device__ double bucket_sums(const Buckets &b, int nb, double qjump, int32_t *lds,
+                              int32_t *flags) {
   const int l = threadIdx.x & 63;
   const int sz = nb >= 0 ? b.list[4 * nb + 1] : 0;
   const int first = nb >= 0 ? b.list[4 * nb] : 0;
+  if (nb >= 0 && b.list[4 * nb + 2] != sz) atomicOr(&flags[8], 2);  // not filled exactly
   int32_t *e = b.slots + first;
   uint64_t big = __ballot(sz > 32 && sz <= kWaveSort);
   while (big) {
@@ -482,11 +484,8 @@ __global__ void __launch_bounds__(1024) c2g_qbot(int32_t *qjx, double *qbot, int
     for (int b0 = (wv * (gridDim.x - 1) + blockIdx.x - 1) * 64; b0 < nb_used; b0 += stride) {
       const int nb = b0 + l;
       const bool mine = nb < nb_used && bk.cell[nb] < nkey;
-      const double s = bucket_sums(bk, mine ? nb : -1, qjump, lds);
-      if (mine) {
-        bk.vals[nb] = s;
-        if (bk.list[4 * nb + 2] != bk.list[4 * nb + 1]) atomicOr(&flags[8], 2);
-      }
+      const double s = bucket_sums(bk, mine ? nb : -1, qjump, lds, flags);
+      if (mine) bk.vals[nb] = s;
     }
     return;
   }
@@ -507,7 +506,7 @@ __global__ void __launch_bounds__(1024) c2g_qbot(int32_t *qjx, double *qbot, int
       const int32_t nb = fl ? bucket_of(w[u]) : -1;
       cv[u] = w[u] && !fl ? cell_value(w[u], qjump, bk) : 0.0;
       if (__ballot(fl)) {
-        const double s = bucket_sums(bk, nb < bk.bcap ? nb : -1, qjump, lds);
+        const double s = bucket_sums(bk, nb < bk.bcap ? nb : -1, qjump, lds, flags);
         if (fl) cv[u] = nb < bk.bcap ? s : 0.0 / 0.0;
       }
       cnt += w[u] != 0;
