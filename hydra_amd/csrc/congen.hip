@@ -326,7 +326,10 @@ __global__ void cg_successor(const int64_t *kib, const int32_t *lev_of_gid, int6
     if (k == -1) break;
     p = (p + 1) & (uint64_t)(h.cap - 1);
   }
-  succ[gid] = -1;
+  // no exit (a field with NaN has boxes that a contour enters and does not
+  // leave): counted, and a loop of its own for the chains' tables
+  succ[gid] = gid;
+  sad2[gid] = -1;
   atomicAdd(err, 1);
 }
 
@@ -480,15 +483,21 @@ struct WalkGraph {
   int8_t *state;      // per chain (work space): visits left of its saddle, used
 };
 
+// Crossings without a successor (errs: the host's four error counts): the
+// chains' tables hold no walk, and the kernels below leave them alone.
+__device__ __forceinline__ bool tables_broken(const int32_t *errs) {
+  return errs[0] != 0 || errs[1] != 0;
+}
+
 __global__ void cw_saddle_flag(const int64_t *sad2, int64_t n, int32_t *flag) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c < n) flag[c] = sad2[c] >= 0 ? 1 : 0;
 }
 __global__ void cw_graph(const int64_t *succ, const int64_t *sad2, const int32_t *lev_of_gid,
                          const int64_t *lev_base, const int64_t *lev_n, int64_t n, ChainTab t,
-                         WalkGraph g) {
+                         WalkGraph g, const int32_t *errs) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n || sad2[c] < 0) return;
+  if (c >= n || sad2[c] < 0 || tables_broken(errs)) return;
   const int lv = lev_of_gid[c];
   const int64_t lb = lev_base[lv], le = lb + lev_n[lv];
   const int32_t r0 = g.rank[lb], j = g.rank[c];
@@ -582,7 +591,9 @@ __global__ void __launch_bounds__(64) cw_walk(const int32_t *starts, const int64
                                               const int64_t *lev_n, ChainTab t, WalkGraph g,
                                               int64_t ntot, int32_t nchain, int64_t *cyc_start,
                                               int32_t *cyc_len, int32_t *cyc_count,
-                                              int32_t *err) {
+                                              int32_t *errs) {
+  if (tables_broken(errs)) return;
+  int32_t *err = errs + 2;
   extern __shared__ __align__(16) unsigned char walk_raw[];
   WalkLds &L = *(WalkLds *)walk_raw;
   const int lv = blockIdx.x, l = threadIdx.x;
@@ -675,9 +686,9 @@ __global__ void __launch_bounds__(64) cw_walk(const int32_t *starts, const int64
     cyc_count[lv] = nc;
   }
 }
-__global__ void cw_expand(ChainTab t, int64_t n, const int32_t *err, int64_t *order) {
+__global__ void cw_expand(ChainTab t, int64_t n, const int32_t *errs, int64_t *order) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n || *err) return;  // a failed walk leaves offsets unset
+  if (c >= n || tables_broken(errs) || errs[2]) return;  // a failed walk leaves offsets unset
   const int32_t k = t.key[c], p = t.pos[c];
   const int64_t o = p >= t.afrom[k] ? t.aoff[k] + (p - t.afrom[k]) : t.boff[k] + p;
   if (o >= 0 && o < n) order[o] = c;
@@ -1100,7 +1111,7 @@ int recontour(Ctx &c, const double *qq) {
       HYD_HIP(hipStreamSynchronize(c.s));
       nchain = last[0] + last[1];
       hipLaunchKernelGGL(cw_graph, gb, dim3(256), 0, c.s, succ, sad2, lev_of_gid, d_lev_base,
-                         d_lev_n, ntot, tb, wg);
+                         d_lev_n, ntot, tb, wg, errs);
       HYD_HIP(hipGetLastError());
     }
     std::vector<int32_t> hlc(nlev);
@@ -1117,8 +1128,8 @@ int recontour(Ctx &c, const double *qq) {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     hipLaunchKernelGGL(cw_walk, dim3(nlev), dim3(64), sizeof(WalkLds), c.s, starts, d_soff, levcnt,
                        d_lev_base, d_lev_n, tb, wg, ntot, nchain, cyc_start, cyc_len, cyc_count,
-                       errs + 2);
-    if (ntot > 0) hipLaunchKernelGGL(cw_expand, gb, dim3(256), 0, c.s, tb, ntot, errs + 2, order);
+                       errs);
+    if (ntot > 0) hipLaunchKernelGGL(cw_expand, gb, dim3(256), 0, c.s, tb, ntot, errs, order);
     HYD_HIP(hipGetLastError());
   }
   std::vector<int32_t> hcc(nlev), herr(4);

@@ -508,6 +508,30 @@ def test_con2grid_crowded_cells_bitwise(kind, least, hyd_cache):
         assert bits_equal(h.con2grid(c["x"], c["y"], c["nextq"], c["qjump"]), qc_o)
 
 
+def test_recontour_of_nan_is_refused():
+    """A field with one NaN gives boxes that a contour enters and does not
+    leave: an error, after which the context contours a sound field."""
+    from hydra_amd import Hydra, HydraError
+    from hydra_amd.ic import random_pv
+    ng = 32
+    q = random_pv(ng, seed=5)
+    h = Hydra(ng)
+    h.set_field(q)
+    h.recontour()
+    want = h.contours()
+    bad = q.copy()
+    bad[11, 17] = np.nan
+    h.set_field(bad)
+    with pytest.raises(HydraError, match="inconsistent crossing tables"):
+        h.recontour()
+    h.set_field(q)
+    h.recontour()
+    got = h.contours()
+    for k in ("x", "y", "nextq", "i1q", "i2q", "npq", "indq"):
+        assert np.array_equal(got[k], want[k]), k
+    h.close()
+
+
 @pytest.mark.parametrize("ng", [64, 256])
 def test_recontour_of_noise_bitwise(ng):
     """White noise has a saddle in every few grid boxes: the ordered walk
