@@ -37,8 +37,9 @@ namespace hyd {
 // exactly p+q entries and replaces the cell's counter by the bucket number
 // (mark_bucket), so that whoever meets the cell later needs no search; a
 // fill pass over the nodes drops each crossing's (node, sign) into its
-// cell's bucket, and one thread per bucket, over the whole GPU, orders the
-// entries by node and adds them as the reference does.
+// cell's bucket, and the buckets' sums, one to a lane over the whole GPU
+// (with the wavefront's help from 33 entries on), order the entries by node
+// and add them as the reference does.
 // A developed flow has 10^4 to 10^5 such cells.  300 steps into an ng=256
 // flow (4e5 nodes) the sweep's claim takes 5 us (205 us when it revisited
 // the nodes, with a hash table and two same-address atomics per cell) and
@@ -79,8 +80,11 @@ __device__ __forceinline__ bool is_flagged(int32_t w) {
 }
 
 // The counter of a claimed cell holds its bucket: 15 bits in each half, the
-// top bit of both set, which makes it a flagged word; every flagged cell is
-// claimed before the marks are read, so no count is mistaken for one.
+// top bit of both set, which makes it a flagged word.  While the list holds
+// every flagged cell all of them are claimed before the marks are read, and
+// no count is mistaken for one.  A cell beyond the list keeps its counts,
+// which then read as some bucket's mark (its entries stay inside that
+// bucket); the sticky error, set with it, has the sweep refused.
 static constexpr int32_t kNoBucket = 0x3fffffff;  // the bucket list was full
 __device__ __forceinline__ int32_t mark_bucket(int32_t b) {
   return (int32_t)(0x80008000u | ((uint32_t)(b >> 15) << 16) | (uint32_t)(b & 0x7fff));
@@ -464,8 +468,8 @@ __device__ __forceinline__ double cell_value_fast(int32_t w, double qjump, const
 // after it; every counter then reads the value after the last non-empty one
 // at or before it.  The additions are the reference's, in its order.
 // Any nxf (passes of kQbotPart).  Block 0 runs the chain; the others make
-// the bucket sums of the order-dependent cells meanwhile, one thread per
-// bucket (block 0 those of its own counters).  Being the last reader of the
+// the bucket sums of the order-dependent cells meanwhile, one to a lane
+// (block 0 those of its own counters).  Being the last reader of the
 // bottom-row counters, block 0 leaves them zero for the next sweep.
 static constexpr int kQbotPart = 4096;  // counters per pass, four per thread
 static constexpr int kQbotPer = kQbotPart / 1024;

@@ -532,6 +532,26 @@ def test_recontour_of_nan_is_refused():
     h.close()
 
 
+# more entries of order-dependent cells than the buckets hold (2^22), and
+# more such cells (2^20; each has at least four entries) besides
+@pytest.mark.parametrize("ng,nodes", [(32, 150000), (512, 90000)])
+def test_con2grid_overflow_is_reported_once(ng, nodes, hyd_cache):
+    """A sweep whose order-dependent cells exceed the buckets is refused; the
+    next one is right again."""
+    from hydra_amd import HydraError
+    from oracle.hyo import Oracle
+    h = hyd_cache(ng)
+    rng = np.random.default_rng(nodes)
+    x, y = rng.uniform(-np.pi, np.pi, (2, nodes))
+    nxt = np.r_[np.arange(2, nodes + 1), 1].astype(np.int32)
+    with pytest.raises(HydraError, match="error -3"):
+        h.con2grid(x, y, nxt, 0.37)
+    c = _hairpins(ng)
+    o = Oracle(ng)
+    o.set_contours(c)
+    assert bits_equal(h.con2grid(c["x"], c["y"], c["nextq"], c["qjump"]), o.con2grid())
+
+
 @pytest.mark.parametrize("ng", [64, 256])
 def test_recontour_of_noise_bitwise(ng):
     """White noise has a saddle in every few grid boxes: the ordered walk
