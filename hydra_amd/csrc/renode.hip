@@ -186,21 +186,22 @@ __device__ double seq_sum_e(const double *se, int64_t o, int n, int ibeg, int le
 // The accumulator walk (contours.f90:826-838, 858-868, 907-920) over the
 // nodes ibeg, next(ibeg), ... for `want` new nodes, written to out slots
 // oo+1 .. oo+want (old node index, acc after the subtraction).  acc starts
-// at 0; e sums to the wanted count over len nodes, at most maxlen old nodes
-// are visited.  Wavefront 0 only; lds_e and lds_s hold kRnBlock doubles.
-__device__ void walk_nodes(const RenodeArgs &g, int64_t o, int n, int ibeg, int len, int maxlen,
-                           int want, int64_t oo, double *lds_e, double *lds_s) {
+// at 0.  The scaled e of the len nodes sum to want + 1, so the walk ends
+// among them: the roundings of its additions (len (want + 1) 2^-53 at most)
+// do not make up for that one.  Wavefront-uniform; lds_e and lds_s hold
+// kRnBlock doubles of the calling wavefront.
+__device__ void walk_nodes(const RenodeArgs &g, int64_t o, int n, int ibeg, int len, int want,
+                           int64_t oo, double *lds_e, double *lds_s) {
   const int l = threadIdx.x & 63;
   double acc = 0.0, v[kRnPer];
   int done = 0;
   load_block(v, g.se, o, n, ibeg, 0, len);
-  int end = len, m;
-  for (int q0 = 0; q0 < maxlen && done < want; q0 += m) {
+  int m;
+  for (int q0 = 0; q0 < len && done < want; q0 += m) {
 #pragma unroll
     for (int j = 0; j < kRnPer; j++) lds_e[64 * j + l] = v[j];
-    m = end - q0 < kRnBlock ? end - q0 : kRnBlock;
-    if (q0 + m == end) end = maxlen;
-    if (q0 + m < end) load_block(v, g.se, o, n, ibeg, q0 + m, end);
+    m = len - q0 < kRnBlock ? len - q0 : kRnBlock;
+    if (q0 + m < len) load_block(v, g.se, o, n, ibeg, q0 + m, len);
     wave_sync();
     // s - floor(s) is exact and s >= 0: the hardware's fraction
     int j = 0;
@@ -250,11 +251,10 @@ __device__ void walk_nodes(const RenodeArgs &g, int64_t o, int n, int ibeg, int 
     done += __shfl(incl, 63, 64);
     wave_sync();
   }
-  // (sum(e) = the wanted count, so the walk always ends with done = want;
-  // should rounding ever leave slots, they get the last node, never an
-  // index outside the contour)
+  // (should slots ever be left, they get the last node, never an index
+  // outside the contour)
   for (int slot = done + 1 + l; slot <= want; slot += 64) {
-    int i = ibeg + (maxlen - 1) % n;
+    int i = ibeg + len - 1;
     if (i >= n) i -= n;
     g.wi[oo + slot] = i;
     g.wacc[oo + slot] = 0.0;
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(256) renode_kernel(RenodeArgs g) {
       }
       // ncorn = 0 walks i = 1, 2, ...; ncorn = 1 starts at the corner and
       // wraps (contours.f90:826-868)
-      walk_nodes(g, o, n, start, n, n, npr - 1, oo, lds_e[0], lds_s[0]);
+      walk_nodes(g, o, n, start, n, npr - 1, oo, lds_e[0], lds_s[0]);
     }
     __syncthreads();
     for (int im = 1 + t; im < npr; im += nt) {
@@ -502,7 +502,7 @@ __global__ void __launch_bounds__(256) renode_kernel(RenodeArgs g) {
       g.se[o + q] = fac * g.se[o + q];
     }
     __threadfence_block();  // the walk reads the scaled values (other lanes' stores)
-    if (np > 1) walk_nodes(g, o, n, ib, len, len, np - 1, oo + at, lds_e[w], lds_s[w]);
+    if (np > 1) walk_nodes(g, o, n, ib, len, np - 1, oo + at, lds_e[w], lds_s[w]);
   }
   __syncthreads();
   for (int im = t; im < tot; im += nt) {
