@@ -72,9 +72,10 @@ def test_every_length_bitwise(ctx, n):
         assert bits_equal(ctx.revfft(m, n, want, t, f), back), ("revfft", m)
 
 
-# the grids whose transforms take one, two and three passes over LDS, with
-# and without a factor 2
-@pytest.mark.parametrize("ng", [16, 128, 512, 1024])
+# every shape of the 2D passes: none (8, 16), one (32, 64), two (128, 256;
+# 1024 and 2048, two stages a pass) and three (512) exchanges through LDS,
+# with a leading factor 2 (8, 32, 128, 512, 2048) and without
+@pytest.mark.parametrize("ng", [8, 16, 32, 64, 128, 256, 512, 1024, 2048])
 def test_2d_transforms_bitwise(ng):
     from hydra_amd import Hydra
     from oracle.hyo import Oracle
