@@ -554,12 +554,51 @@ def test_con2grid_overflow_is_reported_once(ng, nodes, hyd_cache):
 
 @pytest.mark.parametrize("ng", [64, 256])
 def test_recontour_of_noise_bitwise(ng):
-    """White noise has a saddle in every few grid boxes: the ordered walk
-    through them, with a level's chains in LDS (ng=64) and, beyond its
-    capacity of 12000 chains a level, in global memory (ng=256)."""
+    """White noise: tens of thousands of short contours (a level hardly ever
+    passes through a saddle: chains that close on themselves)."""
     from hydra_amd import Hydra
     from oracle.hyo import Oracle
     q = np.random.default_rng(ng).standard_normal((ng, ng))
+    o = Oracle(ng, ncontq=3)
+    o.init_from_field(q)
+    o.recontour(o.d("qr").copy())
+    h = Hydra(ng, ncontq=3)
+    h.set_field(q)
+    h.recontour()
+    c, g = o.contours(), h.contours()
+    for k in ("nextq", "i1q", "i2q", "npq", "indq"):
+        assert np.array_equal(g[k], c[k]), k
+    assert bits_equal(g["x"], c["x"]) and bits_equal(g["y"], c["y"])
+    h.close()
+
+
+def _saddle_boxes(q, level):
+    """Boxes of the 16 times finer bilinear field whose corners alternate
+    about a level."""
+    i = np.arange(16 * len(q))
+    i, p = i // 16, i % 16 / 16.0
+    j = (i + 1) % len(q)
+    a = q[i] * (1 - p)[:, None] + q[j] * p[:, None]
+    s = a[:, i] * (1 - p) + a[:, j] * p >= level
+    r, t = np.roll(s, -1, 0), np.roll(s, -1, 1)
+    return int(np.sum((s == np.roll(r, -1, 1)) & (r == t) & (s != r)))
+
+
+@pytest.mark.parametrize("ng,in_lds", [(64, True), (128, False)])
+def test_recontour_through_saddles_bitwise(ng, in_lds):
+    """A product of two alternating sequences has a saddle at the same value
+    in every grid box, off the fine grid's vertices; shifted so that a level
+    has that value, each is a box that two chains enter: the ordered walk
+    through them, with the level's chains in LDS and beyond its capacity of
+    12000 in global memory."""
+    from hydra_amd import Hydra
+    from oracle.hyo import Oracle
+    rng = np.random.default_rng(ng)
+    sign = (-1.0) ** np.arange(ng)
+    q = np.outer(sign * rng.uniform(0.6, 1.4, ng), sign * rng.uniform(0.6, 1.4, ng))
+    q += (q.max() - q.min()) / 6  # half of the level spacing
+    chains = 2 * _saddle_boxes(q, (q.max() - q.min()) / 6)
+    assert 0 < chains <= 12000 if in_lds else chains > 12000
     o = Oracle(ng, ncontq=3)
     o.init_from_field(q)
     o.recontour(o.d("qr").copy())
