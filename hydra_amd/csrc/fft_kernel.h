@@ -14,8 +14,8 @@
 // results are stafft's bit for bit whatever the blocking.
 //
 // What bounds it: memory at large grids (a pass of four 1024^2 FP64 fields
-// moves 67 MB in 18-20 us, 3.5 TB/s; a stage at a time through LDS it took
-// 23-25), latency at small ones.  All of a thread's (up to 32) global loads
+// moves 67 MB in 18-20 us, 3.5 TB/s, and in 21 beside the other stream's
+// kernels; a stage at a time through LDS it took 23-25), latency at small ones.  All of a thread's (up to 32) global loads
 // are issued before the first use.  FP32 gains most: its passes at 2048^2
 // were bound by the LDS exchanges.
 #pragma once

@@ -627,12 +627,19 @@ __global__ void k_tick(Scalars *sc) {
 // for the update.  Every kernel sees the same inputs as in the reference's
 // serial order.
 // Two cases run it all on the main stream.  Up to ng=64 the kernels are too
-// short to be worth the events between the streams (two streams -> one: eight
-// steps of ng=32 4697 -> 4081 us, four of ng=64 5726 -> 5527; from ng=256 on
-// two are as fast or faster, ng=512 18867 against 18372 us for twenty).  And
-// from four flows at once the flows overlap each other, and a second stream
-// each shares the same four hardware queues (eight flows of ng=128 to 512:
-// 19.2 -> 17.2 ms).
+// short to be worth the events between the streams.  And from four flows at
+// once the flows overlap each other, and a second stream each shares the same
+// four hardware queues.  us, two streams -> one:
+//   eight steps of ng=32 4697 -> 4081, four of ng=64 5726 -> 5527, twenty of
+//   ng=512 18372 -> 18867
+//   a step of four flows: ng=128 2560 -> 1955, mixed 1600 -> 1040; ng=512
+//   3080 -> 2730, mixed 1730 -> 1505
+//   a step of eight: ng=512 5520 -> 5130, mixed 3270 -> 3035; mixed ng=128 to
+//   512 3070 -> 2285
+// The lines lie where the gain was sure; one stream is also the faster way
+// for a step of ng=128 alone (676 -> 660, mixed 430 -> 367) and of two flows
+// (ng=128 1290 -> 1075, mixed 785 -> 530; ng=512 1620 -> 1500, mixed 960 ->
+// 735), where both still run on two.
 static constexpr int kOneStreamNg = 64;
 bool one_stream(const Ctx &c) { return c.c.nx <= kOneStreamNg || c.crowded; }
 
