@@ -358,6 +358,33 @@ def test_recontour_cycle_bitwise():
     h.close()
 
 
+def test_recontour_with_contours_ng256_bitwise():
+    """Two recontourings with contours at ng=256, whose ultra-fine mean is a
+    sum with two folded levels, in one work area."""
+    from hydra_amd import Hydra
+    from hydra_amd.ic import random_pv
+    from oracle.hyo import Oracle
+    ng = 256
+    o, h = Oracle(ng, ncontq=15), Hydra(ng, ncontq=15)
+    q = random_pv(ng, seed=7)
+    o.init_from_field(q)
+    h.set_field(q)
+    o.recontour(o.d("qr").copy())
+    h.recontour()
+    for _ in range(2):
+        for m in (o, h):
+            m.evolution_init()
+            m.advance()
+            m.prepare()
+        o.recontour(o.d("qr").copy())
+        h.recontour()
+        c, g = o.contours(), h.contours()
+        for k in ("nextq", "i1q", "i2q", "npq", "indq"):
+            assert np.array_equal(g[k], c[k]), k
+        assert bits_equal(g["x"], c["x"]) and bits_equal(g["y"], c["y"])
+    h.close()
+
+
 def _hairpins(ng, nest=4):
     """Closed thin loops whose crossings of one fine x-gridline fall in one
     fine cell with both signs, `nest` of each: order-dependent cells
